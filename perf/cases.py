@@ -183,11 +183,11 @@ def _walks(seed, n):
     rg = 100.0 * math.sqrt(n / 2e6)  # the benchmark's density at any length
     out = []
     for k in range(2):
-        s = (torch.randn(n, 3, device="cuda", generator=gen) * 2.0 ** 20).round().to(torch.int64)
-        x = torch.cumsum(s, 0)
-        end, mean = x[-1].double(), x.sum(0).double() / n
-        i = torch.arange(n, device="cuda", dtype=torch.float64)[:, None] / n
-        x = x.double() - i * end - (mean - end * ((n - 1) / (2 * n)))
+        s = (torch.randn(3, n, device="cuda", generator=gen) * 2.0 ** 20).round().to(torch.int64)
+        x = torch.cumsum(s, 1)
+        end, mean = x[:, -1:].double(), x.sum(1, keepdim=True).double() / n
+        i = torch.arange(n, device="cuda", dtype=torch.float64) / n
+        x = (x.double() - i * end - (mean - end * ((n - 1) / (2 * n)))).T
         x *= rg / (2.0 ** 20 * math.sqrt(n / 4.0))
         if k:
             d = np.random.default_rng([5, seed]).normal(size=3)
@@ -210,7 +210,7 @@ def _curves(case, seed):
     else:
         x, n = _walks(seed, case["n"])
     dtype = torch.float32 if case["dtype"] == "float32" else torch.float64
-    return x.to(dtype).cpu().numpy(), np.concatenate([[0], np.cumsum(n)])
+    return x.to(dtype).contiguous().cpu().numpy(), np.concatenate([[0], np.cumsum(n)])
 
 
 # ---------------------------------------------------------------- the three programs

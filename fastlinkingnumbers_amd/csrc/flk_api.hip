@@ -254,7 +254,7 @@ void flk_destroy(flk_ctx *ctx) {
                          &ctx->curves.ed, &ctx->curves.d_off, &ctx->d_pairs, &ctx->d_tasks,
                          &ctx->d_cost, &ctx->d_task_theta, &ctx->d_task_corr,
                          &ctx->d_pair_task0, &ctx->d_pair_out, &ctx->d_pair_corr,
-                         &ctx->d_boxes, &ctx->d_pls, &ctx->d_count, &ctx->d_misc,
+                         &ctx->d_boxes, &ctx->d_pls, &ctx->d_pls_boxes, &ctx->d_count, &ctx->d_misc,
                          &ctx->mlp.d_params, &ctx->mlp.d_norm, &ctx->mlp.d_bf16,
                          &ctx->mlp.d_image};
   for (auto *b : bufs) b->release();

@@ -314,7 +314,8 @@ struct flk_ctx {
   void *noalloc_scratch = nullptr;  // this device's fixed direct-sum array (ds.hip)
   // scratch
   flk::DevBuf d_pairs, d_tasks, d_cost, d_task_theta, d_task_corr, d_pair_task0,
-      d_pair_out, d_pair_corr, d_boxes, d_pls, d_count, d_misc;
+      d_pair_out, d_pair_corr, d_boxes, d_pls, d_pls_boxes, d_count, d_misc;
+  flk::HostBuf pls_host;         // pinned: the potential-link search's total and pairs
 };
 
 namespace flk {

@@ -2,7 +2,10 @@
 //
 // Potential-link search (reference src/potential_link_search.cpp:88-127): all
 // unordered curve pairs whose FP64 bounding boxes overlap as closed intervals.
-// The device builds an implicit BVH over the curve boxes: boxes are sorted by
+// Up to kAllPairsCurves curves every pair is tested: the curves' boxes fit the
+// caches, and counts, their prefix sum and a second sweep that writes put the
+// pairs in ascending order without a sort.  Beyond that the device builds an
+// implicit BVH over the curve boxes: boxes are sorted by
 // the 30-bit Morton code of their centres, padded to a power of two, and the
 // levels of a complete binary tree (heap layout, root = 1, children 2k and
 // 2k+1) are unions of their children.  One thread per curve then walks the
@@ -227,6 +230,105 @@ __global__ __launch_bounds__(256) void bvh_query(const Box6 *__restrict__ heap,
   }
 }
 
+// Every pair of curves tested.  A wave takes kRowsPerWave rows (curves i) and
+// one chunk of kColChunk columns (curves j > i), 64 columns a step; a cell is
+// one row's part in one chunk.  Counting: cells[i * chunks + chunk] receives
+// the cell's overlaps.  Writing: cells holds their exclusive prefix sum, and
+// the pairs go to their places, which are ascending in (i, j), straight into
+// the caller's pinned memory (slots past cap are dropped, the host sees the
+// total).  Bound by latency for the sizes at hand: 16 steps a wave, each six
+// 8-byte loads from the caches for kRowsPerWave tests.
+constexpr int kRowsPerWave = 4;
+constexpr int kColChunk = 1024;
+template <bool kWrite>
+__global__ __launch_bounds__(256) void pls_all_pairs(const double *__restrict__ boxes, int32_t n, int32_t chunks,
+                                                     int32_t *__restrict__ cells, int64_t cap,
+                                                     int2 *__restrict__ out, int64_t *__restrict__ total) {
+  const int lane = threadIdx.x & 63;
+  const int i0 = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * kRowsPerWave;
+  const int c0 = (int)blockIdx.y * kColChunk;
+  if (kWrite && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *total = cells[(int64_t)n * chunks];
+  if (!kWrite && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) cells[(int64_t)n * chunks] = 0;
+  if (i0 >= n) return;
+  Box6 row[kRowsPerWave];
+  int cnt[kRowsPerWave];
+#pragma unroll
+  for (int r = 0; r < kRowsPerWave; ++r) {
+    const double *b = boxes + 6 * (int64_t)min(i0 + r, n - 1);
+    for (int d = 0; d < 3; ++d) {
+      row[r].mn[d] = b[d];
+      row[r].mx[d] = b[3 + d];
+    }
+    cnt[r] = kWrite && i0 + r < n ? cells[(int64_t)(i0 + r) * chunks + blockIdx.y] : 0;
+  }
+  const int end = min(n, c0 + kColChunk);
+  // from the 64-column step that holds the first column past row i0
+  for (int j0 = max(c0, c0 + (i0 + 1 - c0) / 64 * 64); j0 < end; j0 += 64) {
+    const int j = j0 + lane;
+    const double *b = boxes + 6 * (int64_t)min(j, n - 1);
+    Box6 q;
+    for (int d = 0; d < 3; ++d) {
+      q.mn[d] = b[d];
+      q.mx[d] = b[3 + d];
+    }
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const int i = i0 + r;
+      const bool hit = j < end && j > i && i < n && box_overlap(row[r], q);
+      const unsigned long long m = __ballot(hit);
+      if (kWrite && hit) {
+        const int64_t slot = (int64_t)cnt[r] + __popcll(m & ((1ull << lane) - 1ull));
+        if (slot < cap) out[slot] = make_int2(i, j);
+      }
+      cnt[r] += __popcll(m);
+    }
+  }
+  if (!kWrite && lane < kRowsPerWave && i0 + lane < n) {
+    int v = cnt[0];
+#pragma unroll
+    for (int r = 1; r < kRowsPerWave; ++r) v = lane == r ? cnt[r] : v;
+    cells[(int64_t)(i0 + lane) * chunks + blockIdx.y] = v;
+  }
+}
+
+// Most curves of the all-pairs search.  Whole calls on lattices of four pairs a
+// curve, the tree (with its two library sorts, an allocation per array and one
+// atomic per pair) against all pairs: 137 and 25 us for 10 curves, 270 and 44
+// for 400, 393 and 77 for 1,600, 587 and 237 for 10,000, 727 and 250 for
+// 16,384, 1,052 and 636 for 30,000; the sweep grows with the square.
+constexpr int32_t kAllPairsCurves = 32768;
+
+void pls_small(flk_ctx *ctx, const double *d_boxes, int32_t n, std::vector<int32_t> &out) {
+  hipStream_t s = ctx->stream;
+  const int32_t chunks = (n + kColChunk - 1) / kColChunk;
+  const int64_t ncells = (int64_t)n * chunks;
+  ctx->d_pls.reserve(sizeof(int32_t) * (ncells + 1) + scan_temp_bytes(ncells + 1));
+  int32_t *cells = ctx->d_pls.as<int32_t>(), *tmp = cells + ncells + 1;
+  const dim3 grid((unsigned)((n + 4 * kRowsPerWave - 1) / (4 * kRowsPerWave)), (unsigned)chunks);
+  hipLaunchKernelGGL(pls_all_pairs<false>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, (int64_t)0,
+                     (int2 *)nullptr, (int64_t *)nullptr);
+  FLK_HIP(hipGetLastError());
+  exclusive_scan(cells, cells, ncells + 1, tmp, s);
+  // the pairs land in pinned memory behind their total; a second sweep only
+  // when there are more than eight pairs a curve (and than ever before)
+  int64_t cap = std::max<int64_t>(1024, 8 * (int64_t)n);
+  for (;;) {
+    ctx->pls_host.reserve(sizeof(int64_t) * (1 + cap));
+    cap = (int64_t)(ctx->pls_host.bytes / sizeof(int64_t)) - 1;
+    int64_t *total = ctx->pls_host.as<int64_t>();
+    int2 *pairs = reinterpret_cast<int2 *>(total + 1);
+    hipLaunchKernelGGL(pls_all_pairs<true>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, cap, pairs, total);
+    FLK_HIP(hipGetLastError());
+    FLK_HIP(hipStreamSynchronize(s));
+    if (*total <= cap) {
+      const int32_t *p = reinterpret_cast<const int32_t *>(pairs);
+      out.assign(p, p + 2 * *total);
+      return;
+    }
+    cap = *total;
+  }
+}
+
 }  // namespace
 
 void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes) {
@@ -284,6 +386,17 @@ void pls_run(flk_ctx *ctx, const double *boxes, int32_t n, std::vector<int32_t> 
   out.clear();
   if (n < 2) return;
   hipStream_t s = ctx->stream;
+  if (n <= kAllPairsCurves) {
+    // the uploaded curves' boxes are on the device already
+    const double *d_boxes = ctx->d_boxes.as<double>();
+    if (boxes != ctx->curves.box.data()) {
+      ctx->d_pls_boxes.reserve(sizeof(double) * 6 * (size_t)n);
+      FLK_HIP(hipMemcpyAsync(ctx->d_pls_boxes.ptr, boxes, sizeof(double) * 6 * (size_t)n, hipMemcpyHostToDevice, s));
+      d_boxes = ctx->d_pls_boxes.as<double>();
+    }
+    pls_small(ctx, d_boxes, n, out);
+    return;
+  }
   int32_t L = 1;
   while (L < n) L <<= 1;
   // device scratch layout inside d_pls

@@ -2296,7 +2296,7 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
       // Beside the Barnes-Hut branch the direct-sum kernel takes a share of
       // its resident blocks, the direct sum's fraction of the two parts'
       // estimated times alone: its segment pairs at 1.2e12 per second (FP64:
-      // 1.9e11), and 0.19 ns per Barnes-Hut tree segment for build and
+      // 4.5e11), and 0.19 ns per Barnes-Hut tree segment for build and
       // traversal.  Both rates are the 10,000-loop lattice's (5.6e10 direct
       // pairs, 3.2e8 tree segments; share 0.43, 3 of the 8 blocks per CU),
       // whose certificate took 109 ms with the parts in sequence, 97 ms as two
@@ -2308,7 +2308,7 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
         for (size_t k = 0; k + 1 < ds_pairs.size(); k += 2)
           work += (double)n[ds_pairs[k]] * (double)n[ds_pairs[k + 1]];
         for (const BatchPlan &bp : NG->batches) bh_segments += (double)bp.forest.S;
-        const double t_ds = work / (prm.fp64 ? 1.9e11 : 1.2e12), t_bh = bh_segments * 0.19e-9;
+        const double t_ds = work / (prm.fp64 ? 4.5e11 : 1.2e12), t_bh = bh_segments * 0.19e-9;
         share = t_ds / (t_ds + t_bh);
       }
       ds_capture_prepare(ctx, ds_pairs.data(), (int64_t)ds_idx.size(), prm.fp64 != 0, NG->ds, share);

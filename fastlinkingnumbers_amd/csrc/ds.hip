@@ -321,9 +321,55 @@ __global__ __launch_bounds__(256) void ds_tile_f32(
 }
 
 // ---------------------------------------------------------------- FP64 tiles
-// The judge: same tiling, FP64 coordinates, library atan2 and sqrt.
+// The judge: the FP32 kernel's layout and sharing in FP64 (see there for the
+// algebra), bound by the FP64 vector rate, which equals the unpacked FP32
+// one: what counts is instructions per pair, 62 here (106 for a column step of
+// two pairs, 24 for the arctangent of two steps).  Square roots and the
+// reciprocal start from the hardware's estimates and are refined to FP64 in
+// line; the small angles of two columns' pairs are added as one product of
+// x' + i y'.  Any lane of the wave outside the short path's conditions sends
+// the step to the general path, which takes the step's pairs from their
+// vertices with the library's sqrt and atan2.
+// Chain mail of 256 rings of 64-16,384 vertices (7.4e9 pairs): 42.6 -> 16.6 ms,
+// 175 -> 448 G pairs/s, where every pair took four roots and one library
+// atan2; the sums' error against a 64-bit reference 2.3e-15 -> 1.5e-16, as the
+// triple product comes from the edges instead of three long vectors.  Held to
+// 128 VGPRs, 4 waves per SIMD (the 12 spilled serve the general path): 17.4
+// ms at 140 and 3 waves; R = 4 at 2 waves takes 15.8 ms but pads the rows of
+// a curve to 256.
+__device__ __forceinline__ double sqrt_refined(double x) {
+  // Goldschmidt from the estimate, one Newton correction; 0 gives NaN, which
+  // the short path's test refuses
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
+// atan(zi / zr) for zr > 0 and |zi / zr| <= tan(4 atan(1/16)): the series
+// t + t s Q(s), s = t^2, Q interpolated at Chebyshev nodes for this engine
+// (fit_atan_poly.py): relative error 2.6e-17 in exact arithmetic.
+__device__ __forceinline__ double atan_short_f64(double zi, double zr) {
+  double y = __builtin_amdgcn_rcp(zr);
+  y = fma(fma(-zr, y, 1.0), y, y);
+  double t = zi * y;
+  t = fma(fma(-zr, t, zi), y, t);
+  const double s = t * t;
+  double p = 0.04685617558659996;
+  p = fma(p, s, -0.0654587570283471);
+  p = fma(p, s, 0.07685808139339988);
+  p = fma(p, s, -0.09090713470019263);
+  p = fma(p, s, 0.11111107897869509);
+  p = fma(p, s, -0.14285714259715684);
+  p = fma(p, s, 0.19999999999919688);
+  p = fma(p, s, -0.3333333333333329);
+  return fma(t * s, p, t);
+}
+
 template <int R>
-__global__ __launch_bounds__(256) void ds_tile_f64(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void ds_tile_f64(
     const double4 *__restrict__ pts, const DsPair *__restrict__ pairs,
     const DsTask *__restrict__ tasks, const int64_t *__restrict__ cost_prefix, int64_t ntasks,
     double *__restrict__ task_theta, int32_t *__restrict__ task_corr) {
@@ -339,44 +385,151 @@ __global__ __launch_bounds__(256) void ds_tile_f64(
     const DsTask tk = tasks[t];
     const DsPair pr = pairs[tk.pair];
     const int rbase = tk.row0 + lane * R;
+    const double4 *__restrict__ rows = pts + pr.off_r;
     double px[R + 1], py[R + 1], pz[R + 1];
-    bool valid[R];
+    double ex[R], ey[R], ez[R], he1[R];
+    // rows past the curve's end are zero-length segments at the closing vertex
 #pragma unroll
     for (int k = 0; k <= R; ++k) {
-      const double4 h = pts[pr.off_r + min(rbase + k, pr.n_r)];
+      const double4 h = rows[min(rbase + k, pr.n_r)];
       px[k] = h.x; py[k] = h.y; pz[k] = h.z;
     }
 #pragma unroll
-    for (int k = 0; k < R; ++k) valid[k] = rbase + k < pr.n_r;
+    for (int k = 0; k < R; ++k) {
+      ex[k] = px[k + 1] - px[k];
+      ey[k] = py[k + 1] - py[k];
+      ez[k] = pz[k + 1] - pz[k];
+      he1[k] = -0.5 * fma(ex[k], ex[k], fma(ey[k], ey[k], ez[k] * ez[k]));
+    }
+    auto column = [&](const double4 &q, double (&gx)[R + 1], double (&gy)[R + 1], double (&gz)[R + 1],
+                      double (&gn)[R + 1], double (&gl)[R + 1]) {
+#pragma unroll
+      for (int k = 0; k <= R; ++k) {
+        gx[k] = q.x - px[k];
+        gy[k] = q.y - py[k];
+        gz[k] = q.z - pz[k];
+        gn[k] = fma(gx[k], gx[k], fma(gy[k], gy[k], gz[k] * gz[k]));
+        gl[k] = sqrt_refined(gn[k]);
+      }
+    };
+    const double4 *__restrict__ cpt = pts + pr.off_c;
+    const int ncl = pr.n_c;
+    double an[R + 1], al[R + 1], acol[R];
+    double bn[R + 1], bl[R + 1], bcol[R];
+    double qx, qy, qz;  // the previous column's vertex
+    {
+      double gx[R + 1], gy[R + 1], gz[R + 1];
+      const double4 q = cpt[tk.col0];
+      qx = q.x; qy = q.y; qz = q.z;
+      column(q, gx, gy, gz, an, al);
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) acol[k] = fma(0.5, an[k] + an[k + 1], he1[k]);
+    double4 nq = cpt[tk.col0 + 1];  // loaded one step ahead
+
     double acc = 0.0;
     int corr = 0;
-    for (int j = tk.col0; j < tk.col0 + tk.ncols; ++j) {
-      const double4 q0 = pts[pr.off_c + j];
-      const double4 q1 = pts[pr.off_c + j + 1];
+    // One column step: the R pairs (k, j), their short-path angles multiplied
+    // into (zr, zi) or, on the general path, added to acc and corr.
+    auto step = [&](int j, const double (&gn)[R + 1], const double (&gl)[R + 1], const double (&gcol)[R],
+                    double (&nn)[R + 1], double (&nl)[R + 1], double (&ncol)[R], double &zr, double &zi) {
+      const double4 q = nq;
+      nq = cpt[min(j + 2, ncl)];
+      const double e2x = q.x - qx, e2y = q.y - qy, e2z = q.z - qz;
+      qx = q.x; qy = q.y; qz = q.z;
+      double nx[R + 1], ny[R + 1], nz[R + 1];
+      column(q, nx, ny, nz, nn, nl);
+      // u = -e2.G(k,j+1): G(k,j).G(k,j+1) = |G(k,j+1)|^2 + u(k), and the
+      // diagonal G(k,j).G(k+1,j+1) = G(k,j+1).G(k+1,j+1) + u(k+1)
+      double u[R + 1], row[R + 1], diag[R];
+#pragma unroll
+      for (int k = 0; k <= R; ++k) {
+        u[k] = fma(-e2x, nx[k], fma(-e2y, ny[k], -e2z * nz[k]));
+        row[k] = nn[k] + u[k];
+      }
 #pragma unroll
       for (int k = 0; k < R; ++k) {
-        const double ax = q0.x - px[k], ay = q0.y - py[k], az = q0.z - pz[k];
-        const double bx = q0.x - px[k + 1], by = q0.y - py[k + 1], bz = q0.z - pz[k + 1];
-        const double cx = q1.x - px[k + 1], cy = q1.y - py[k + 1], cz = q1.z - pz[k + 1];
-        const double dx = q1.x - px[k], dy = q1.y - py[k], dz = q1.z - pz[k];
-        const double la = sqrt(ax * ax + ay * ay + az * az);
-        const double lb = sqrt(bx * bx + by * by + bz * bz);
-        const double lc = sqrt(cx * cx + cy * cy + cz * cz);
-        const double ld = sqrt(dx * dx + dy * dy + dz * dz);
-        const double ac = cx * ax + cy * ay + cz * az;
-        const double div1 = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + ac * lb +
-                            (cx * bx + cy * by + cz * bz) * la;
-        const double div2 = la * ld * lc + (ax * dx + ay * dy + az * dz) * lc + ac * ld +
-                            (cx * dx + cy * dy + cz * dz) * la;
-        const double det = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) +
-                           az * (bx * cy - by * cx);
-        const double xp = div1 * div2 - det * det;
-        const double yp = det * (div1 + div2);
-        const double th = atan2(yp, xp);
-        const int cr = (yp * det < 0.0) ? (det > 0.0 ? 1 : -1) : 0;
-        acc += valid[k] ? th : 0.0;
-        corr += valid[k] ? cr : 0;
+        ncol[k] = fma(0.5, nn[k] + nn[k + 1], he1[k]);
+        diag[k] = ncol[k] + u[k + 1];
       }
+      double dt[R];
+#pragma unroll
+      for (int c = 0; c < R / 2; ++c) {
+        const int k1 = 2 * c + 1;
+        const double wx = fma(ny[k1], e2z, -nz[k1] * e2y);
+        const double wy = fma(nz[k1], e2x, -nx[k1] * e2z);
+        const double wz = fma(nx[k1], e2y, -ny[k1] * e2x);
+        dt[k1 - 1] = fma(ex[k1 - 1], wx, fma(ey[k1 - 1], wy, ez[k1 - 1] * wz));
+        dt[k1] = fma(ex[k1], wx, fma(ey[k1], wy, ez[k1] * wz));
+      }
+      bool small = true;
+      double yr = 1.0, yi = 0.0;
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const double la = gl[k], lb = gl[k + 1], lc = nl[k + 1], ld = nl[k];
+        const double s = fma(la, lc, diag[k]);
+        const double div1 = fma(lb, s, fma(gcol[k], lc, row[k + 1] * la));
+        const double div2 = fma(ld, s, fma(row[k], lc, ncol[k] * la));
+        const double xp = fma(div1, div2, -dt[k] * dt[k]);
+        const double s12 = div1 + div2;
+        const double yp = dt[k] * s12;
+        // no branch correction, |y'/x'| <= 1/16, and x' clear of the rounding
+        // noise of vertices that (nearly) touch: their denominators are at
+        // most ~1e-16 each (relative vectors are at most 1 long), x' ~1e-32
+        small = small && (s12 > 0.0) && (fma(0.0625, xp, -fabs(yp)) > 1e-28);
+        if (k == 0) {
+          yr = xp;
+          yi = yp;
+        } else {
+          const double r = fma(yr, xp, -yi * yp);
+          yi = fma(yr, yp, yi * xp);
+          yr = r;
+        }
+      }
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!small) == 0, 1)) {
+        const double r = fma(zr, yr, -zi * yi);
+        zi = fma(zr, yi, zi * yr);
+        zr = r;
+      } else {
+        const double4 q0 = cpt[j], q1 = cpt[min(j + 1, ncl)];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          const double ax = q0.x - px[k], ay = q0.y - py[k], az = q0.z - pz[k];
+          const double bx = q0.x - px[k + 1], by = q0.y - py[k + 1], bz = q0.z - pz[k + 1];
+          const double cx = q1.x - px[k + 1], cy = q1.y - py[k + 1], cz = q1.z - pz[k + 1];
+          const double dx = q1.x - px[k], dy = q1.y - py[k], dz = q1.z - pz[k];
+          const double la = sqrt(ax * ax + ay * ay + az * az);
+          const double lb = sqrt(bx * bx + by * by + bz * bz);
+          const double lc = sqrt(cx * cx + cy * cy + cz * cz);
+          const double ld = sqrt(dx * dx + dy * dy + dz * dz);
+          const double ac = cx * ax + cy * ay + cz * az;
+          const double div1 = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + ac * lb +
+                              (cx * bx + cy * by + cz * bz) * la;
+          const double div2 = la * ld * lc + (ax * dx + ay * dy + az * dz) * lc + ac * ld +
+                              (cx * dx + cy * dy + cz * dz) * la;
+          const double det = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) +
+                             az * (bx * cy - by * cx);
+          const double xp = div1 * div2 - det * det;
+          const double yp = det * (div1 + div2);
+          const bool valid = rbase + k < pr.n_r;
+          const double th = atan2(yp, xp);
+          acc += valid ? th : 0.0;
+          corr += (valid && yp * det < 0.0) ? (det > 0.0 ? 1 : -1) : 0;
+        }
+      }
+    };
+    const int jend = tk.col0 + tk.ncols;
+    int j = tk.col0;
+    for (; j + 1 < jend; j += 2) {
+      double zr = 1.0, zi = 0.0;
+      step(j, an, al, acol, bn, bl, bcol, zr, zi);
+      step(j + 1, bn, bl, bcol, an, al, acol, zr, zi);
+      acc += atan_short_f64(zi, zr);
+    }
+    if (j < jend) {
+      double zr = 1.0, zi = 0.0;
+      step(j, an, al, acol, bn, bl, bcol, zr, zi);
+      acc += atan_short_f64(zi, zr);
     }
     acc = wave_sum(acc);
     corr = wave_sum(corr);

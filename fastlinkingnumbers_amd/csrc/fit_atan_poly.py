@@ -8,7 +8,11 @@ s = t^2, weight 1/f), then rounds the coefficients to FP32:
 * atan_unit (ds.hip): a = 1, degree 7;
 * the paired small-angle series (ds.hip, short path): a = 16/63, degree 4.
 
-Usage: python fit_atan_poly.py  -- prints both coefficient sets (highest
+The FP64 tile kernel's series (atan_short_f64) is atan(t) = t + t s Q(s) on
+|t| <= tan(4 atan(1/16)), Q of degree 7 interpolated at Chebyshev nodes in
+extended precision.
+
+Usage: python fit_atan_poly.py  -- prints the coefficient sets (highest
 degree first, as ds.hip evaluates them by Horner's rule) and their maximum
 relative errors in exact arithmetic.
 """
@@ -67,6 +71,34 @@ def remez(a, degree, iters=60, grid=200001):
     return c
 
 
+def _tail(s):
+    """(atan(t)/t - 1) / s for s = t^2 < 0.1, in extended precision."""
+    out = np.zeros_like(s)
+    for k in range(59, 0, -1):
+        out = out * s + np.longdouble((-1) ** k) / (2 * k + 1)
+    return out
+
+
+def interpolate_f64(a, degree):
+    """Coefficients (lowest first, FP64) of Q in atan(t) = t + t s Q(s) on
+    |t| <= a, and the maximum relative error of the result there."""
+    b, m = np.longdouble(a) ** 2, degree + 1
+    x = b / 2 * (1 - np.cos(np.longdouble(np.pi) * (2 * np.arange(m).astype(np.longdouble) + 1) / (2 * m)))
+    d = _tail(x)  # Newton's divided differences
+    for k in range(1, m):
+        d[k:] = (d[k:] - d[k - 1:-1]) / (x[k:] - x[:-k])
+    c = np.zeros(m, dtype=np.longdouble)  # to powers of s
+    for k in range(m - 1, -1, -1):
+        c[1:] = c[:-1] - x[k] * c[1:]
+        c[0] = d[k] - x[k] * c[0]
+    c = c.astype(np.float64)
+    s = b * np.linspace(0, 1, 100001)[1:].astype(np.longdouble)
+    q = np.zeros_like(s)
+    for v in c[::-1]:
+        q = q * s + np.longdouble(v)
+    return c, float(np.max(np.abs((q - _tail(s)) * s / (1 + s * _tail(s)))))
+
+
 def max_rel_error(coef_high_first, a, n=400001, fp32=False):
     """Maximum relative error of t * P(t^2) against atan(t) on 0 < t <= a,
     in float64 arithmetic or emulating the kernel's FP32 Horner evaluation
@@ -99,6 +131,9 @@ def main():
         print("  coefficients (highest degree first):", ", ".join(f"{v:.17g}f" for v in c32))
         print(f"  max relative error: {e64:.3g} (FP64 coefficients), {e:.3g} (FP32 coefficients, mean signed "
               f"{bias:.2g}), {e32:.3g} (evaluated in FP32)")
+    c, e = interpolate_f64(np.tan(4 * np.arctan(1 / 16)), 7)
+    print("FP64 series, Q highest degree first:", ", ".join(repr(float(v)) for v in c[::-1]))
+    print(f"  max relative error: {e:.3g}")
 
 
 if __name__ == "__main__":

@@ -1,0 +1,69 @@
+"""The FP64 tile kernel at the sizes where its rows (2 per lane, 128 per wave),
+columns (two per iteration, chunks of a multiple of 32) and general path can go
+wrong, against the FP64 oracle.
+
+Tolerance 1e-12 per pair: a pair of at most 1,100 x 700 segments sums 8e5
+angles.  An angle's rounding error is that of its triple product, about 1e-16
+r^3 in the oracle (a product of three relative vectors), over x' ~ 8 r^3, so
+below 1e-16, and 8e5 of them (random signs) stay below 1e-13 even times ten.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+
+flk = pytest.importorskip("fastlinkingnumbers_amd")
+
+pytestmark = pytest.mark.gpu
+
+
+def _ring(n, centre, tilt, wobble, seed):
+    g = np.random.default_rng(seed)
+    t = 2 * np.pi * np.arange(n) / n
+    r = 1 + wobble * np.cos(3 * t + g.uniform(0, 6))
+    x = np.stack([r * np.cos(t), r * np.sin(t), wobble * np.sin(2 * t)], 1)
+    c, s = np.cos(tilt), np.sin(tilt)
+    return x @ np.array([[1, 0, 0], [0, c, s], [0, -s, c]]) + centre
+
+
+@pytest.mark.parametrize("n,m", [(2, 2), (3, 2), (5, 4), (63, 64), (65, 3), (127, 31), (128, 33), (129, 128),
+                                 (255, 63), (257, 65), (600, 511), (1100, 513), (1025, 700)])
+def test_remainders_match_oracle(engine, n, m):
+    a = _ring(n, [0, 0, 0], 0.0, 0.07, n)
+    b = _ring(m, [0.9, 0.1, 0.2], 1.3, 0.05, m)
+    engine.set_curves([a, b])
+    got = engine.linking_numbers([[0, 1], [1, 0]], method="directsum", fp64=1).lk
+    ref = O.ds(a, b)
+    print(n, m, "got", got, "oracle", ref)
+    assert np.abs(got - ref).max() < 1e-12
+
+
+@pytest.mark.parametrize("gap", [1e-2, 1e-5, 1e-9])
+def test_near_misses_take_the_general_path(engine, gap):
+    """Curves passing each other at `gap` of their size: large angles and small
+    denominators, mixed with the short path's columns in the same wave.  The
+    oracle's triple products then err by 1e-16 of pairs whose angle is pi, over
+    x' ~ gap^2 times the segments' squares: 1e-16 / gap."""
+    a = _ring(300, [0, 0, 0], 0.0, 0.0, 1)
+    b = _ring(211, [2.0 + gap, 0, 0], np.pi / 2, 0.0, 2)
+    engine.set_curves([a, b])
+    got = engine.linking_numbers([[0, 1]], method="directsum", fp64=1).lk[0]
+    ref = O.ds(a, b)
+    print(gap, "got", got, "oracle", ref)
+    assert abs(got - ref) < 1e-12 + 1e-14 / gap
+
+
+def test_planar_and_touching_curves_keep_their_signs(engine):
+    """Coplanar curves have zero triple products, and so has a shared vertex:
+    the sums are the oracle's, not noise over noise.  A shared vertex's sum
+    depends on which curve comes first, in the oracle too (its two orders
+    differ by 1/4 here): the engine's is one of them."""
+    a = _ring(130, [0, 0, 0], 0.0, 0.0, 1)
+    b = _ring(70, [3.0, 0, 0], 0.0, 0.0, 2)
+    c = a[:40].copy()
+    c[1:] += np.array([0.5, 0.25, 0.75])
+    engine.set_curves([a, b, c])
+    got = engine.linking_numbers([[0, 1], [0, 2]], method="directsum", fp64=1).lk
+    print("got", got, "oracle", O.ds(a, b), O.ds(a, c), O.ds(c, a))
+    assert abs(got[0] - O.ds(a, b)) < 1e-12
+    assert min(abs(got[1] - O.ds(a, c)), abs(got[1] - O.ds(c, a))) < 1e-12

@@ -765,6 +765,81 @@ __device__ __forceinline__ float wave_predict(bool need, const BhGeo &A, const B
   return p;
 }
 
+// Classification of one node pair and, where it is a far field, its value.
+struct BhVisit {
+  int kind;  // -1 none, 0 leaf pair, 1 far field, 2 split
+  int ca, cb;  // the split node's children
+  bool split_a;
+  float val, err;
+};
+
+template <bool MLP, typename MS>
+__device__ __forceinline__ BhVisit bh_visit(const BhItem &it, bool live, const BhGeo *__restrict__ geo,
+                                            const BhMom *__restrict__ mom, const float *__restrict__ beta2, float eps,
+                                            float log_tol, MS &ms, unsigned int &wave_evals) {
+  BhVisit out{-1, 0, 0, false, 0.f, 0.f};
+  float pv = __builtin_inff();  // learned criterion: predicted log10 far-field error
+  // Learned criterion: both node records are loaded once, before the
+  // prediction, and kept for the classification (a dead lane reads node 0
+  // of its empty item; loading them again after the network's LDS fences
+  // cost another round trip: 2x8M learned 11.75 -> 11.15 ms).  Beta loads
+  // them inside the live branch (loading them before it measured 4% slower).
+  BhGeo A0, B0;
+  if constexpr (MLP) {
+    A0 = geo[it.a];
+    B0 = geo[it.b];
+    const float rx = (B0.cx - A0.cx) + (B0.lx - A0.lx), ry = (B0.cy - A0.cy) + (B0.ly - A0.ly),
+                rz = (B0.cz - A0.cz) + (B0.lz - A0.lz);
+    const float dsq = fmaf(rx, rx, fmaf(ry, ry, rz * rz)) + eps;
+    const float rs = A0.radius + B0.radius;
+    pv = wave_predict(live && !(A0.c0 < 0 && B0.c0 < 0) && dsq > rs * rs + eps, A0, B0, dsq, ms, wave_evals);
+  }
+  if (live) {
+    const BhGeo A = MLP ? A0 : geo[it.a], B = MLP ? B0 : geo[it.b];
+    const F3 r = f3((B.cx - A.cx) + (B.lx - A.lx), (B.cy - A.cy) + (B.ly - A.ly),
+                    (B.cz - A.cz) + (B.lz - A.lz));
+    const float dsq = dot3(r, r) + eps;
+    const bool la = A.c0 < 0, lb = B.c0 < 0;
+    const float rs = A.radius + B.radius;
+    // Learned criterion: far field when the spheres are disjoint and the
+    // predicted log10 error is below the tolerance; the squared predicted
+    // error is accumulated (the pair's estimate is the root of the sum, as
+    // for independent signs).  Otherwise the reference's beta test.
+    const bool far = MLP ? (dsq > rs * rs + eps && pv < log_tol) : (dsq > rs * rs * beta2[it.pair] + eps);
+    if (la && lb) {
+      out.kind = 0;
+    } else if (far) {
+      out.kind = 1;
+      out.val = far_field(node_mom(mom, it.a, A), node_mom(mom, it.b, B), A, B, r, dsq, out.err);
+      if (MLP) out.err = exp10f(2.0f * pv);
+    } else {
+      out.kind = 2;
+      out.split_a = (!la && !lb) ? !(B.rsq > A.rsq) : lb;
+      out.ca = out.split_a ? A.c0 : B.c0;
+      out.cb = out.split_a ? A.c1 : B.c1;
+    }
+  }
+  return out;
+}
+
+// The network's LDS image, every load of a thread in flight at once.  Ends
+// with a barrier.
+__device__ __forceinline__ void load_infer_image(const InferImage *__restrict__ mlp_img, MlpShared &ms) {
+  constexpr int kWords = (int)(sizeof(InferImage) / 16);
+  static_assert(kWords > 3 * kTravBlock && kWords <= 4 * kTravBlock, "four 16-byte words per thread");
+  const int4 *src = reinterpret_cast<const int4 *>(mlp_img) + threadIdx.x;
+  int4 *dst = reinterpret_cast<int4 *>(&ms.img) + threadIdx.x;
+  const bool w3 = 3 * kTravBlock + (int)threadIdx.x < kWords;
+  const int4 v0 = src[0], v1 = src[kTravBlock], v2 = src[2 * kTravBlock];
+  const int4 v3 = w3 ? src[3 * kTravBlock] : int4{};
+  dst[0] = v0;
+  dst[kTravBlock] = v1;
+  dst[2 * kTravBlock] = v2;
+  if (w3) dst[3 * kTravBlock] = v3;
+  if (threadIdx.x == 0) ms.evals = 0;
+  __syncthreads();
+}
+
 // One traversal level over a chunk of items.  Split items are staged in LDS
 // as (pair with the split side in its sign, unsplit node, child 0, child 1)
 // from the front of the block's stage, leaf-bucket items from the back; after
@@ -805,20 +880,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                             : kTravItems;
   if constexpr (MLP) {
     if ((int64_t)blockIdx.x * csz >= n) return;  // the whole block, before any barrier
-    // the network's LDS image, every load of a thread in flight at once
-    constexpr int kWords = (int)(sizeof(InferImage) / 16);
-    static_assert(kWords > 3 * kTravBlock && kWords <= 4 * kTravBlock, "four 16-byte words per thread");
-    const int4 *src = reinterpret_cast<const int4 *>(mlp_img) + threadIdx.x;
-    int4 *dst = reinterpret_cast<int4 *>(&ms.img) + threadIdx.x;
-    const bool w3 = 3 * kTravBlock + (int)threadIdx.x < kWords;
-    const int4 v0 = src[0], v1 = src[kTravBlock], v2 = src[2 * kTravBlock];
-    const int4 v3 = w3 ? src[3 * kTravBlock] : int4{};
-    dst[0] = v0;
-    dst[kTravBlock] = v1;
-    dst[2 * kTravBlock] = v2;
-    if (w3) dst[3 * kTravBlock] = v3;
-    if (threadIdx.x == 0) ms.evals = 0;  // read after the chunk loop's barriers
-    __syncthreads();
+    load_infer_image(mlp_img, ms);
   }
   for (int64_t chunk = blockIdx.x; chunk * csz < n; chunk += gridDim.x) {
   if (threadIdx.x == 0) sh.nsplit = sh.nleaf = 0;
@@ -831,62 +893,20 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     const int64_t t = b0 + (int64_t)k * kTravBlock;
     const bool live = t < n;
     BhItem it = live ? items[t] : BhItem{0, 0, 0, 0};
-    int kind = -1;  // 0 leaf pair, 1 far, 2 split
-    int ca = 0, cb = 0;
-    bool split_a = false;
-    float pv = __builtin_inff();  // learned criterion: predicted log10 far-field error
-    // Learned criterion: both node records are loaded once, before the
-    // prediction, and kept for the classification (a dead lane reads node 0
-    // of its empty item; loading them again after the network's LDS fences
-    // cost another round trip: 2x8M learned 11.75 -> 11.15 ms).  Beta loads
-    // them inside the live branch (loading them before it measured 4% slower).
-    BhGeo A0, B0;
-    if constexpr (MLP) {
-      A0 = geo[it.a];
-      B0 = geo[it.b];
-      const float rx = (B0.cx - A0.cx) + (B0.lx - A0.lx), ry = (B0.cy - A0.cy) + (B0.ly - A0.ly),
-                  rz = (B0.cz - A0.cz) + (B0.lz - A0.lz);
-      const float dsq = fmaf(rx, rx, fmaf(ry, ry, rz * rz)) + eps;
-      const float rs = A0.radius + B0.radius;
-      pv = wave_predict(live && !(A0.c0 < 0 && B0.c0 < 0) && dsq > rs * rs + eps, A0, B0, dsq, ms, wave_evals);
-    }
-    if (live) {
-      const BhGeo A = MLP ? A0 : geo[it.a], B = MLP ? B0 : geo[it.b];
-      const F3 r = f3((B.cx - A.cx) + (B.lx - A.lx), (B.cy - A.cy) + (B.ly - A.ly),
-                      (B.cz - A.cz) + (B.lz - A.lz));
-      const float dsq = dot3(r, r) + eps;
-      const bool la = A.c0 < 0, lb = B.c0 < 0;
-      const float rs = A.radius + B.radius;
-      // Learned criterion: far field when the spheres are disjoint and the
-      // predicted log10 error is below the tolerance; the squared predicted
-      // error is accumulated (the pair's estimate is the root of the sum, as
-      // for independent signs).  Otherwise the reference's beta test.
-      const bool far = MLP ? (dsq > rs * rs + eps && pv < log_tol) : (dsq > rs * rs * beta2[it.pair] + eps);
-      if (la && lb) {
-        kind = 0;
-      } else if (far) {
-        kind = 1;
-        float e = 0.f;
-        const float val = far_field(node_mom(mom, it.a, A), node_mom(mom, it.b, B), A, B, r, dsq, e);
-        if (MLP) e = exp10f(2.0f * pv);
-        if (tp < 0 || tp == it.pair) {
-          tp = it.pair;
-          tv += (double)val;
-          te += (double)e;
-        } else {
-          atomicAdd(psum + it.pair, (double)val);
-          if (e != 0.f) atomicAdd(perr + it.pair, (double)e);
-        }
+    const BhVisit v = bh_visit<MLP>(it, live, geo, mom, beta2, eps, log_tol, ms, wave_evals);
+    if (v.kind == 1) {
+      if (tp < 0 || tp == it.pair) {
+        tp = it.pair;
+        tv += (double)v.val;
+        te += (double)v.err;
       } else {
-        kind = 2;
-        split_a = (!la && !lb) ? !(B.rsq > A.rsq) : lb;
-        ca = split_a ? A.c0 : B.c0;
-        cb = split_a ? A.c1 : B.c1;
+        atomicAdd(psum + it.pair, (double)v.val);
+        if (v.err != 0.f) atomicAdd(perr + it.pair, (double)v.err);
       }
     }
-    const int ss = wave_lds_slot(kind == 2, &sh.nsplit);
-    if (ss >= 0) stage[ss] = make_int4(split_a ? ~it.pair : it.pair, split_a ? it.b : it.a, ca, cb);
-    const int sl = wave_lds_slot(kind == 0, &sh.nleaf);
+    const int ss = wave_lds_slot(v.kind == 2, &sh.nsplit);
+    if (ss >= 0) stage[ss] = make_int4(v.split_a ? ~it.pair : it.pair, v.split_a ? it.b : it.a, v.ca, v.cb);
+    const int sl = wave_lds_slot(v.kind == 0, &sh.nleaf);
     if (sl >= 0) stage[kTravItems - 1 - sl] = make_int4(it.pair, it.a, it.b, 0);
   }
   block_pair_add(tp, tp >= 0, tv, te, psum, perr, sh);
@@ -927,29 +947,287 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
   }
 }
 
+// One round of a walked pass (the beta criterion's, see PassShape): every wave
+// takes chunks of the round's items and walks their whole subtrees of node
+// pairs depth first, from a stack of its own in LDS, 64 items a step, one a
+// lane, with no barrier.  Splits push their children; leaf pairs gather in LDS
+// and leave 64 or more at a time for bh_leaf_pairs.  No wave waits for another:
+// once its segment's chunks are all taken and a quarter of its waves have
+// ended, a wave still at work leaves its stack to the next round within
+// kWalkSteps steps, so a round ends with the chip full, and the first rounds,
+// whose few items widen twofold a step, take the work to every wave.  The last
+// round leaves nothing (a stack that overflows there fails the pass, as items
+// beyond the queue's capacity do, and the host re-runs the batch).
+// Level by level the 2 x depth + 1 launches cost 5-10 us each whatever they do:
+// device time of certificates of ten loops of 2,000-4,000 vertices (10 pairs)
+// 473 -> 336 us, 400 rings of 64-4,096 (1,038 pairs) 1,004 -> 706 us, 2,000
+// rings of 64-16,384 2.73 -> 2.26 ms, two random walks of 5,000 0.68 -> 0.58 ms.
+// Counters that every wave of the chip would update or read serialise it (about
+// 7 ns each on one address), so the queues, the leaf list and their counters
+// come in kSegs segments on lines of their own, one for every 16 blocks, each
+// of one XCD; a round takes its chunks from all segments alike.
+constexpr int kWalkRounds = 6;
+constexpr int kWalkSteps = 8;
+constexpr int kSegs = 64;
+constexpr int kLine = 16;  // words of a counter line (128 bytes)
+
+// Counter words of a pass.  Walked: [4] root items, [6] overflow, and lines of
+// the segments' totals (visits, splits, -, leaf items, leaf segment pairs) and,
+// for each round, of its items, the chunks taken of it and the waves that have
+// ended.  Level by level: [2] leaf segment pairs, [3] network evaluations, [4 +
+// 2d] the items of level d, [5] leaf items.  bh_merge makes of either the
+// kPassHead words that the host reads: visits, splits, leaf segment pairs,
+// evaluations, root items, leaf items, overflow.
+constexpr int kPassHead = 8;
+constexpr int kMaxLevels = 1000;
+constexpr int kPassWords = 16 + kLine * kSegs * (2 + kWalkRounds);
+static_assert(kPassWords >= 4 + 2 * (kMaxLevels + 1), "a level pass's counters fit");
+__host__ __device__ __forceinline__ unsigned long long *seg_totals(unsigned long long *cnt, int seg) {
+  return cnt + 16 + kLine * seg;
+}
+__host__ __device__ __forceinline__ unsigned long long *seg_round(unsigned long long *cnt, int round, int seg) {
+  return cnt + 16 + kLine * (kSegs * (1 + round) + seg);
+}
+
+constexpr int kStack = 512, kLeaves = 128;
+struct WalkLds {  // a wave's stack (circular) and its leaf pairs waiting to leave
+  int p[kStack], a[kStack], b[kStack];
+  int lp[kLeaves], la[kLeaves], lb[kLeaves];
+};
+
+__global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4))) void bh_walk(
+    const BhItem *__restrict__ items, int64_t cap, const BhGeo *__restrict__ geo, const BhMom *__restrict__ mom,
+    const float *__restrict__ beta2, float eps, unsigned long long *__restrict__ cnt, int round,
+    BhItem *__restrict__ next, BhItem *__restrict__ leaves, double *__restrict__ psum, double *__restrict__ perr,
+    int copies, int64_t copy_stride) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int seg = blockIdx.x & (kSegs - 1);
+  const int64_t seg_cap = cap / kSegs;
+  // the round's items: its segments' counts (round 0: the roots), lane s first
+  // holding segment s's end
+  int64_t end = 0;
+  if (round == 0) end = (int64_t)cnt[4];
+  else {
+    end = level_count(seg_round(cnt, round, lane), seg_cap);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t u = __shfl_up(end, d, 64);
+      if (lane >= d) end += u;
+    }
+  }
+  const int64_t n = __shfl(end, 63, 64);
+  // chunks of 1 to 64 items, two for each wave of the grid when there are
+  // enough; a segment's waves take every kSegs-th chunk, in turn
+  const int64_t nwaves = (int64_t)gridDim.x * (kTravBlock / 64);
+  const int64_t csz = max((int64_t)1, min((int64_t)64, n / (2 * nwaves)));
+  const int64_t nchunks = (n + csz - 1) / csz;
+  const int64_t mine = nchunks > seg ? (nchunks - seg + kSegs - 1) / kSegs : 0;
+  const int64_t seg_wave = (int64_t)(blockIdx.x / kSegs) * (kTravBlock / 64);  // this block's first wave of its segment
+  if (seg_wave >= mine) return;  // the whole block, before any barrier
+  __shared__ WalkLds lds[kTravBlock / 64];
+  __shared__ int64_t ends[kSegs];
+  __shared__ TravShared sh;
+  if (w == 0) ends[lane] = end;
+  if (threadIdx.x < 2) sh.base[threadIdx.x] = 0;
+  __syncthreads();
+  const bool last = round + 1 == kWalkRounds;
+  const uint64_t below = (1ull << lane) - 1ull;
+  unsigned long long *totals = seg_totals(cnt, seg);
+  unsigned long long *taken = seg_round(cnt, round, seg) + 1, *nextq = seg_round(cnt, round + 1, seg);
+  WalkLds &L = lds[w];
+  unsigned long long visits = 0, splits = 0;  // of the wave
+  int tp = -1;  // this lane's far-field pair and its running sums
+  double tv = 0.0, te = 0.0;
+  psum += (blockIdx.x % (unsigned)copies) * copy_stride;
+  perr += (blockIdx.x % (unsigned)copies) * copy_stride;
+  auto wrap = [](int k) { return k < kStack ? k : k - kStack; };
+  int nleaf = 0;
+  auto flush_leaves = [&]() {
+    unsigned long long at = 0;
+    if (lane == 0) at = atomicAdd(totals + 3, (unsigned long long)nleaf);
+    at = __shfl(at, 0, 64);
+    wave_lds_sync();
+    for (int i = lane; i < nleaf; i += 64)
+      if ((int64_t)at + i < seg_cap) leaves[seg * seg_cap + (int64_t)at + i] = BhItem{L.lp[i], L.la[i], L.lb[i], 0};
+    wave_lds_sync();
+    nleaf = 0;
+  };
+  NoMlpShared no_mlp;
+  unsigned int no_evals = 0;
+  int bot = 0, num = 0;
+  int64_t chunk = seg_wave + w;  // of the segment's chunks; a wave's first is its own
+  const int64_t seg_waves = (int64_t)((gridDim.x - seg + kSegs - 1) / kSegs) * (kTravBlock / 64);
+  // none left to take once every chunk is some wave's first
+  bool more = chunk < mine, drained = mine <= seg_waves;
+  const int started = (int)min(mine, seg_waves);
+  // waves of the segment that ended before the others share what is left
+  const int enough = started - (int)(seg_waves * 3 / 4);
+  bool starving = drained && enough <= 0;
+  int steps = kWalkSteps, tick = 0;
+  while (more || num > 0) {
+    if (more && num < 64) {
+      const int64_t c0 = (chunk * kSegs + seg) * csz;
+      const int m = (int)min(csz, n - c0);
+      if (lane < m) {
+        int64_t at = c0 + lane;
+        if (round > 0) {  // the segment that holds item `at`: ends before it
+          int lo = 0;
+#pragma unroll
+          for (int d = kSegs / 2; d > 0; d >>= 1)
+            if (ends[lo + d - 1] <= at) lo += d;
+          at += lo * seg_cap - (lo ? ends[lo - 1] : 0);
+        }
+        const BhItem it = items[at];
+        const int k = wrap(wrap(bot + num) + lane);
+        L.p[k] = it.pair;
+        L.a[k] = it.a;
+        L.b[k] = it.b;
+      }
+      num += m;
+      wave_lds_sync();
+      if (drained) {
+        more = false;
+      } else {
+        unsigned long long c = 0;
+        if (lane == 0) c = atomicAdd(taken, 1ull);
+        chunk = seg_waves + (int64_t)__shfl(c, 0, 64);
+        if (chunk >= mine) more = false;
+      }
+      continue;
+    }
+    // the oldest items go to the next round when the stack could overflow, and
+    // all of them kWalkSteps steps after the segment's chunks ran out
+    const int out = last ? 0 : steps <= 0 ? num : num > kStack - 64 ? num / 2 : 0;
+    if (out) {
+      unsigned long long at = 0;
+      if (lane == 0) at = atomicAdd(nextq, (unsigned long long)out);
+      at = __shfl(at, 0, 64);
+      for (int i = lane; i < out; i += 64) {
+        const int k = wrap(bot + i);
+        if ((int64_t)at + i < seg_cap) next[seg * seg_cap + (int64_t)at + i] = BhItem{L.p[k], L.a[k], L.b[k], 0};
+      }
+      wave_lds_sync();
+      bot = wrap(bot + out);
+      num -= out;
+      continue;
+    }
+    // (in the last round a stack near its end goes on with its newest item
+    // alone, which adds no more than the trees' levels)
+    if (num > kStack - 2) {
+      if (lane == 0) atomicOr(cnt + 6, 1ull);
+      break;
+    }
+    const int take = num <= kStack - 64 ? min(num, 64) : 1;
+    num -= take;
+    const int base = wrap(bot + num);
+    const bool live = lane < take;
+    const int k0 = wrap(base + lane);
+    BhItem it{0, 0, 0, 0};
+    if (live) it = BhItem{L.p[k0], L.a[k0], L.b[k0], 0};
+    unsigned long long poll = 0;
+    const bool look = !starving && (++tick & 7) == 0;
+    if (look) poll = __hip_atomic_load(taken + (drained ? 1 : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    wave_lds_sync();  // every item is in registers before its slot is reused
+    const BhVisit v = bh_visit<false>(it, live, geo, mom, beta2, eps, 0.f, no_mlp, no_evals);
+    if (v.kind == 1) {
+      if (tp < 0 || tp == it.pair) {
+        tp = it.pair;
+        tv += (double)v.val;
+        te += (double)v.err;
+      } else {
+        atomicAdd(psum + it.pair, (double)v.val);
+        if (v.err != 0.f) atomicAdd(perr + it.pair, (double)v.err);
+      }
+    }
+    const uint64_t ms2 = __ballot(v.kind == 2), ms0 = __ballot(v.kind == 0);
+    if (v.kind == 2) {
+      const int k = wrap(base + 2 * __popcll(ms2 & below));
+      const int k1 = wrap(k + 1);
+      L.p[k] = L.p[k1] = it.pair;
+      L.a[k] = v.split_a ? v.ca : it.a;
+      L.b[k] = v.split_a ? it.b : v.ca;
+      L.a[k1] = v.split_a ? v.cb : it.a;
+      L.b[k1] = v.split_a ? it.b : v.cb;
+    } else if (v.kind == 0) {
+      const int k = nleaf + __popcll(ms0 & below);
+      L.lp[k] = it.pair;
+      L.la[k] = it.a;
+      L.lb[k] = it.b;
+    }
+    const int ns = __popcll(ms2);
+    num += 2 * ns;
+    nleaf += __popcll(ms0);
+    visits += (unsigned long long)take;
+    splits += (unsigned long long)ns;
+    wave_lds_sync();
+    if (nleaf > kLeaves - 64) flush_leaves();
+    // `taken` runs past the end once a wave found no chunk
+    const int polled = __builtin_amdgcn_readfirstlane((int)min(poll, 0x7fffffffull));
+    if (starving) --steps;
+    else if (!look) continue;
+    else if (drained) starving = polled >= enough;
+    else drained = seg_waves + (int64_t)polled > mine;
+  }
+  if (lane == 0 && visits) atomicAdd(taken + 1, 1ull);
+  if (nleaf) flush_leaves();
+  block_pair_add(tp, tp >= 0, tv, te, psum, perr, sh);
+  __syncthreads();
+  if (lane == 0) {
+    atomicAdd(&sh.base[0], visits);
+    atomicAdd(&sh.base[1], splits);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(totals, sh.base[0]);
+    atomicAdd(totals + 1, sh.base[1]);
+  }
+}
+
 // Exact evaluation of leaf-bucket pairs: every segment pair of the two
 // buckets with the reference leaf term, from FP32 hi/lo vertices (two
 // one-segment leaves: from their node records, which hold the midpoints and
 // the edge vectors).  Blocks of
-// 256 * IPT items as in bh_level (chunks strided over the grid; with n_dev
-// the count is read on the device, n being the bound); counters[2] gets the
-// segment-pair count.
+// 256 * IPT items as in bh_level; *counters gets the segment-pair count.
+// With a device-scheduled pass's counters (cnt) n is the list's capacity and the
+// count is read there: a level pass's list is one, a walked pass's comes in
+// segments, block b taking segment b % kSegs, its sums going to one of the
+// sums' copies.
 template <int IPT>
 __global__ __launch_bounds__(kTravBlock) void bh_leaf_pairs(
-    const BhItem *__restrict__ items, int64_t n, const unsigned long long *__restrict__ n_dev,
+    const BhItem *__restrict__ items, int64_t n, unsigned long long *__restrict__ cnt, int walked,
     const BhGeo *__restrict__ geo, const uint32_t *__restrict__ order, const float4 *__restrict__ hi,
     const float4 *__restrict__ lo, const float4 *__restrict__ ed, double *__restrict__ psum,
-    double *__restrict__ perr, unsigned long long *__restrict__ counters) {
+    double *__restrict__ perr, unsigned long long *__restrict__ counters, int copies, int64_t copy_stride) {
   constexpr int kTravItems = kTravBlock * IPT;
-  if (n_dev) n = level_count(n_dev, n);
+  int64_t first = blockIdx.x, stride = gridDim.x;
+  int64_t csz = kTravItems;
+  if (cnt) {
+    unsigned long long *count = cnt + 5;
+    counters = cnt + 2;
+    if (walked) {
+      const int seg = blockIdx.x & (kSegs - 1);
+      n /= kSegs;
+      items += seg * n;
+      count = seg_totals(cnt, seg) + 3;
+      counters = count + 1;
+      first = blockIdx.x / kSegs;
+      stride = gridDim.x / kSegs;
+      psum += (blockIdx.x % (unsigned)copies) * copy_stride;
+      perr += (blockIdx.x % (unsigned)copies) * copy_stride;
+    }
+    n = level_count(count, n);
+    if (n == 0) return;
+    // a short list spread over the blocks in whole multiples of 256
+    csz = min<int64_t>(csz, ((n + stride - 1) / stride + kTravBlock - 1) / kTravBlock * kTravBlock);
+  }
   __shared__ TravShared sh;
   int npairs = 0;
-  for (int64_t chunk = blockIdx.x; chunk * kTravItems < n; chunk += gridDim.x) {
-  const int64_t b0 = chunk * kTravItems + threadIdx.x;
+  for (int64_t chunk = first; chunk * csz < n; chunk += stride) {
+  const int64_t b0 = chunk * csz + threadIdx.x;
   int tp = -1;
   double tv = 0.0;
 #pragma unroll 1
-  for (int k = 0; k < IPT; ++k) {
+  for (int k = 0; k < IPT && k * kTravBlock < csz; ++k) {
     const int64_t t = b0 + (int64_t)k * kTravBlock;
     if (t >= n) break;
     const BhItem it = items[t];
@@ -996,7 +1274,7 @@ __global__ __launch_bounds__(kTravBlock) void bh_leaf_pairs(
   if (threadIdx.x == 0) {
     unsigned long long s = 0;
     for (int k = 0; k < kTravBlock / 64; ++k) s += (unsigned long long)sh.scan[k];
-    if (s) atomicAdd(counters + 2, s);
+    if (s) atomicAdd(counters, s);
   }
 }
 
@@ -1115,17 +1393,17 @@ __global__ void bh_roots(const int32_t *__restrict__ ra, const int32_t *__restri
   if (k < n) out[k] = BhItem{(int32_t)k, ra[k], rb[k], 0};
 }
 
-// Clears the counters of a device-scheduled pass and sets the root level's
-// count (a kernel rather than a memset, so the pass can be captured).
-__global__ void bh_pass_init(unsigned long long *__restrict__ cnt, int n, int root_slot,
-                             unsigned long long roots) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) cnt[k] = k == root_slot ? roots : 0ull;
-}
-
-__global__ void bh_zero_f64(double *__restrict__ p, int64_t n) {
+// Start of a batch's traversal: its root items, both passes' counters and every
+// copy of the sums cleared (a kernel rather than memsets, so it can be
+// captured), and the first pass's root count.
+__global__ __launch_bounds__(256) void bh_begin(const int32_t *__restrict__ ra, const int32_t *__restrict__ rb,
+                                                int64_t nb, BhItem *__restrict__ items,
+                                                unsigned long long *__restrict__ cnt, int64_t nsums,
+                                                double *__restrict__ sum, double *__restrict__ err) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) p[k] = 0.0;
+  if (k < nb) items[k] = BhItem{(int32_t)k, ra[k], rb[k], 0};
+  if (k < 2 * kPassWords) cnt[k] = k == 4 ? (unsigned long long)nb : 0ull;
+  if (k < nsums) sum[k] = err[k] = 0.0;
 }
 
 // Exclusive scan of one value per thread over a 256-thread block; *total
@@ -1151,6 +1429,13 @@ __device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
   return off + inc - v;
 }
 
+// The copies of one sum, added in order.
+__device__ __forceinline__ double fold_copies(const double *p, int copies, int64_t stride) {
+  double v = p[0];
+  for (int k = 1; k < copies; ++k) v += p[k * stride];
+  return v;
+}
+
 // The re-run decision after a batch's first pass, on the device.  Beta
 // (reference linking_number_certificate.cpp:165-184): the estimate scaled by
 // err_scale gives the target beta = min(beta_init (E / target)^(1/4),
@@ -1159,31 +1444,30 @@ __device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
 // estimate, and a pair above a tenth of the target is re-run (one decade
 // stricter, by the caller's second pass).  One block walks the pairs in order
 // and compacts the re-runs with a block scan, so the list is deterministic:
-// root items (pair = position in the list), beta^2 and the pair's index.  It
-// also clears the second pass's counters and sets its root count at
-// cnt2[root_slot].
+// root items (pair = position in the list), beta^2, and every pair's position
+// in it (-1: not re-run).  Sets the second pass's root count.
 __global__ __launch_bounds__(256) void bh_adapt(int64_t nb, const int32_t *__restrict__ ra,
                                                 const int32_t *__restrict__ rb, const double *__restrict__ err1,
-                                                int mlp, double err_scale, double target_error, double beta_init,
-                                                double beta_limit, BhItem *__restrict__ items2,
-                                                float *__restrict__ beta2_2, int32_t *__restrict__ redo,
-                                                unsigned long long *__restrict__ cnt2, int nslots2, int root_slot) {
+                                                int copies, int64_t copy_stride, int mlp, double err_scale,
+                                                double target_error, double beta_init, double beta_limit,
+                                                BhItem *__restrict__ items2, float *__restrict__ beta2_2,
+                                                int32_t *__restrict__ redo, unsigned long long *__restrict__ n_redo) {
   __shared__ int sw[4];
-  for (int k = threadIdx.x; k < nslots2; k += 256) cnt2[k] = 0ull;
   int carry = 0;
   for (int64_t c0 = 0; c0 < nb; c0 += 256) {
     const int64_t t = c0 + threadIdx.x;
     int flag = 0;
     float b2 = 0.f;
+    const double e1 = t < nb ? fold_copies(err1 + t, copies, copy_stride) : 0.0;
     if (t < nb) {
       if (!mlp) {
-        const double want = pow(err1[t] * err_scale / target_error, 0.25) * beta_init;
+        const double want = pow(e1 * err_scale / target_error, 0.25) * beta_init;
         const double target = beta_limit < want ? beta_limit : want;  // std::min: a NaN estimate stays NaN
         if (target > beta_init) {
           flag = 1;
           b2 = (float)(target * target);
         }
-      } else if (sqrt(err1[t]) > 0.1 * target_error) {
+      } else if (sqrt(e1) > 0.1 * target_error) {
         flag = 1;
         b2 = (float)(beta_init * beta_init);
       }
@@ -1193,37 +1477,68 @@ __global__ __launch_bounds__(256) void bh_adapt(int64_t nb, const int32_t *__res
     if (flag) {
       items2[pos] = BhItem{pos, ra[t], rb[t], 0};
       beta2_2[pos] = b2;
-      redo[pos] = (int32_t)t;
     }
+    if (t < nb) redo[t] = flag ? pos : -1;
     carry += tot;
   }
-  __syncthreads();  // the clear above is done before the count is set
-  if (threadIdx.x == 0) cnt2[root_slot] = (unsigned long long)carry;
+  if (threadIdx.x == 0) *n_redo = (unsigned long long)carry;
 }
 
 // Per-pair results of a batch: the first pass's sum and estimate (scaled by
-// err_scale for beta, the root-sum-square for the learned criterion) ...
-__global__ void bh_merge_first(int64_t nb, const double *__restrict__ sum, const double *__restrict__ err, int mlp,
-                               double err_scale, double *__restrict__ v, double *__restrict__ e,
-                               uint32_t *__restrict__ f) {
+// err_scale for beta, the root-sum-square for the learned criterion), or the
+// second pass's for a re-run pair; sums of the second pass are at + nb.
+// Block 0 makes both device-scheduled passes' kPassHead words of their counters
+// (cnt, null for a host-driven batch; levels: how many a level pass has, 0 when
+// walked), with an overflow noted where a queue or a leaf list is over its
+// capacity (its segment's share of it) or items were left after the last level.
+__global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__restrict__ redo,
+                                                const double *__restrict__ sum, const double *__restrict__ err,
+                                                int copies, int64_t copy_stride, int mlp, double err_scale,
+                                                double *__restrict__ v, double *__restrict__ e,
+                                                uint32_t *__restrict__ f, unsigned long long *__restrict__ heads,
+                                                unsigned long long *__restrict__ cnt, int64_t cap, int levels) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nb) return;
-  v[t] = sum[t];
-  e[t] = mlp ? sqrt(err[t]) : err[t] * err_scale;
-  f[t] = 0u;
-}
-
-// ... replaced by the second pass's for the re-run pairs.
-__global__ void bh_merge_redo(int64_t nb, const unsigned long long *__restrict__ n_redo,
-                              const int32_t *__restrict__ redo, const double *__restrict__ sum2,
-                              const double *__restrict__ err2, int mlp, double err_scale, double *__restrict__ v,
-                              double *__restrict__ e, uint32_t *__restrict__ f) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nb || k >= (int64_t)*n_redo) return;
-  const int32_t t = redo[k];
-  v[t] = sum2[k];
-  e[t] = mlp ? sqrt(err2[k]) : err2[k] * err_scale;
-  f[t] = FLK_PAIR_RETRY;
+  if (t < nb) {
+    const int32_t r = redo[t];
+    const int64_t at = r < 0 ? t : nb + r;
+    const double es = fold_copies(err + at, copies, copy_stride);
+    v[t] = fold_copies(sum + at, copies, copy_stride);
+    e[t] = mlp ? sqrt(es) : es * err_scale;
+    f[t] = r < 0 ? 0u : FLK_PAIR_RETRY;
+  }
+  if (cnt == nullptr || blockIdx.x != 0 || threadIdx.x >= 2 * kSegs) return;
+  const int seg = threadIdx.x & (kSegs - 1), pass = threadIdx.x / kSegs;
+  unsigned long long *c = cnt + pass * kPassWords;
+  unsigned long long x[kPassHead] = {0, 0, 0, 0, seg == 0 ? c[4] : 0, 0, 0, 0};
+  if (levels) {
+    for (int d = seg; d <= levels; d += kSegs) {
+      const unsigned long long n = c[4 + 2 * d];
+      if (d < levels) x[0] += n;
+      if (d > 0) x[1] += n / 2;
+      if ((int64_t)n > cap || (d == levels && n)) x[6] = 1;
+    }
+    if (seg == 0) {
+      x[2] = c[2];
+      x[3] = c[3];
+      x[5] = c[5];
+      if ((int64_t)c[5] > cap) x[6] = 1;
+    }
+  } else {
+    const unsigned long long *tot = seg_totals(c, seg);
+    x[0] = tot[0];
+    x[1] = tot[1];
+    x[2] = tot[4];
+    x[5] = tot[3];
+    if (c[6] || (int64_t)tot[3] > cap / kSegs) x[6] = 1;
+    for (int r = 1; r <= kWalkRounds; ++r)
+      if ((int64_t)*seg_round(c, r, seg) > cap / kSegs) x[6] = 1;
+  }
+#pragma unroll
+  for (int i = 0; i < kPassHead; ++i) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) x[i] += __shfl_xor(x[i], d, 64);
+    if (seg == 0) heads[pass * kPassHead + i] = x[i];
+  }
 }
 
 }  // namespace
@@ -1652,9 +1967,9 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
       const Curves &cv = ctx->curves;
       auto leafk = ipt == 2 ? bh_leaf_pairs<2> : ipt == 8 ? bh_leaf_pairs<8> : bh_leaf_pairs<4>;
       hipLaunchKernelGGL(leafk, dim3((unsigned)((nleaf + ipt * kTravBlock - 1) / (ipt * kTravBlock))),
-                         dim3(kTravBlock), 0, s, B.leaves.as<BhItem>(), (int64_t)nleaf, nullptr, F.geo.as<BhGeo>(),
-                         F.order.as<uint32_t>(), cv.hi.as<float4>(), cv.lo.as<float4>(),
-                         cv.ed.as<float4>(), d_sum, d_err, cnt);
+                         dim3(kTravBlock), 0, s, B.leaves.as<BhItem>(), (int64_t)nleaf, (unsigned long long *)nullptr, 0,
+                         F.geo.as<BhGeo>(), F.order.as<uint32_t>(), cv.hi.as<float4>(), cv.lo.as<float4>(),
+                         cv.ed.as<float4>(), d_sum, d_err, cnt + 2, 1, (int64_t)0);
       FLK_HIP(hipGetLastError());
     }
     DevBuf *last = outb[D - 1];
@@ -1698,9 +2013,20 @@ int resident_grid(flk_ctx *ctx, const void *kernel) {
 // `cap` items.  A level or leaf list beyond that, or items left after the
 // last launched level, mark the pass as overflowed: its sums are incomplete,
 // and the batch is re-run on the host-driven schedule.
+// Or, with few segments a pair, by kWalkRounds launches of bh_walk, each taking
+// what the one before left in the queue.  The line lies where the walk's gain
+// in launches is spent: a pair of random walks of 5,000 vertices each takes
+// 0.58 ms walked and 0.68 by levels, 30,000 1.14 and 1.13, 100,000 1.66 and
+// 1.48 (the levels' blocks classify eight items a thread between barriers, a
+// walk's waves one a step).  The learned criterion's network leaves too little
+// LDS for a walk's stacks.
+constexpr int64_t kWalkSegmentsPerPair = 32768;
+
 struct PassShape {
   int64_t cap = 0;
-  int D = 0, nslots = 0, ipt = 4;
+  bool walk = false;
+  int D = 0, ipt = 4;
+  int copies = 1;  // of the per-pair sums: a walk's blocks of different XCDs add to different ones
   unsigned grid_lev = 1, grid_leaf = 1;
 };
 
@@ -1708,13 +2034,14 @@ struct PassShape {
 // count lives in the 8 words after them.
 constexpr int kHostCounterWords = 4 + 2 * 1024;
 
-// Sizes the device schedule of a batch of nb pairs whose deepest tree has
-// `depth` node levels and reserves its buffers; false when it cannot hold
-// the batch (the host-driven schedule runs it instead).
-bool plan_device_passes(flk_ctx *ctx, int64_t nb, int depth, bool use_mlp, PassShape &P) {
+// Sizes the device schedule of a batch of nb pairs on trees of `segments`
+// segments, the deepest with `depth` node levels, and reserves its buffers;
+// false when it cannot hold the batch (the host-driven schedule runs it
+// instead).
+bool plan_device_passes(flk_ctx *ctx, int64_t nb, int64_t segments, int depth, bool use_mlp, PassShape &P) {
   BhScratch &B = ctx->bh;
-  constexpr int kMaxLevels = 1000;
-  P.D = 2 * depth + 1;
+  P.walk = !use_mlp && segments <= nb * kWalkSegmentsPerPair;
+  P.D = P.walk ? 0 : 2 * depth + 1;
   if (P.D > kMaxLevels) return false;
   if (B.dev_cap == 0) {
     // two level buffers and the leaf list (16 B per item), within a tenth of
@@ -1728,62 +2055,66 @@ bool plan_device_passes(flk_ctx *ctx, int64_t nb, int depth, bool use_mlp, PassS
   P.cap = ctx->tune.bh_level_capacity > 0 ? (int64_t)ctx->tune.bh_level_capacity : B.dev_cap;
   if (nb > P.cap) return false;
   P.ipt = items_per_thread(ctx, use_mlp);
-  P.nslots = 4 + 2 * (P.D + 1);
+  P.copies = P.walk && nb <= 4096 ? 8 : 1;
   while (B.levels.size() < 2) B.add_level();
   B.levels[0]->reserve(sizeof(BhItem) * P.cap);
   B.levels[1]->reserve(sizeof(BhItem) * P.cap);
   B.leaves.reserve(sizeof(BhItem) * P.cap);
-  const LevelKernel lev = level_kernel(P.ipt, use_mlp);
   auto leafk = P.ipt == 2 ? bh_leaf_pairs<2> : P.ipt == 8 ? bh_leaf_pairs<8> : bh_leaf_pairs<4>;
   const int64_t items_per_block = (int64_t)P.ipt * kTravBlock;
   const int64_t chunks = (P.cap + items_per_block - 1) / items_per_block;
-  P.grid_lev = (unsigned)std::min<int64_t>(resident_grid(ctx, (const void *)lev), chunks);
-  P.grid_leaf = (unsigned)std::min<int64_t>(resident_grid(ctx, (const void *)leafk), chunks);
+  const int lev = resident_grid(ctx, P.walk ? (const void *)bh_walk : (const void *)level_kernel(P.ipt, use_mlp));
+  const int leaf = resident_grid(ctx, (const void *)leafk);
+  if (P.walk) {
+    // whole multiples of the segments' number: a segment's waves are on one
+    // XCD, and the segments have as many each
+    P.grid_lev = (unsigned)std::max(kSegs, lev / kSegs * kSegs);
+    P.grid_leaf = (unsigned)std::max(kSegs, leaf / kSegs * kSegs);
+  } else {
+    P.grid_lev = (unsigned)std::min<int64_t>(lev, chunks);
+    P.grid_leaf = (unsigned)std::min<int64_t>(leaf, chunks);
+  }
   return true;
 }
 
-// Enqueues one pass on the device schedule: counters at cnt (the caller's
-// kernel has cleared them and set the root count at cnt[4]), level-0 items at
-// items0, per-pair beta^2 and sums indexed by the items' pair field.
+// Enqueues one pass on the device schedule: counters at cnt (bh_begin has
+// cleared them, and the root count is at cnt[4]), root items at items0,
+// per-pair beta^2 and sums indexed by the items' pair field.
 void enqueue_pass(flk_ctx *ctx, const PassShape &P, const BhItem *items0, const float *beta2, float eps,
                   bool use_mlp, float log_tol, unsigned long long *cnt, double *d_sum, double *d_err,
-                  hipStream_t s) {
+                  int64_t copy_stride, hipStream_t s) {
   BhScratch &B = ctx->bh;
   const Curves &cv = ctx->curves;
   BhItem *buf[2] = {B.levels[0]->as<BhItem>(), B.levels[1]->as<BhItem>()};
   const InferImage *mlp_img = use_mlp ? ctx->mlp.d_image.as<InferImage>() : nullptr;
   const LevelKernel lev = level_kernel(P.ipt, use_mlp);
   auto leafk = P.ipt == 2 ? bh_leaf_pairs<2> : P.ipt == 8 ? bh_leaf_pairs<8> : bh_leaf_pairs<4>;
-  // [2] leaf segment pairs, [3] network evaluations, [4 + 2d] items of level
-  // d, [5] leaf items
-  for (int d = 0; d < P.D; ++d) {
+  for (int d = 0; d < (P.walk ? kWalkRounds : P.D); ++d) {
     const BhItem *in = d == 0 ? items0 : buf[(d - 1) & 1];
-    hipLaunchKernelGGL(lev, dim3(P.grid_lev), dim3(kTravBlock), 0, s, in, P.cap,
-                       (const unsigned long long *)(cnt + 4 + 2 * d), B.geo.as<BhGeo>(), B.mom.as<BhMom>(), beta2,
-                       eps, mlp_img, log_tol, cnt + 3, buf[d & 1], cnt + 4 + 2 * (d + 1), P.cap,
-                       B.leaves.as<BhItem>(), cnt + 5, P.cap, d_sum, d_err);
+    if (P.walk)
+      hipLaunchKernelGGL(bh_walk, dim3(P.grid_lev), dim3(kTravBlock), 0, s, in, P.cap, B.geo.as<BhGeo>(),
+                         B.mom.as<BhMom>(), beta2, eps, cnt, d, buf[d & 1], B.leaves.as<BhItem>(), d_sum, d_err,
+                         P.copies, copy_stride);
+    else
+      hipLaunchKernelGGL(lev, dim3(P.grid_lev), dim3(kTravBlock), 0, s, in, P.cap,
+                         (const unsigned long long *)(cnt + 4 + 2 * d), B.geo.as<BhGeo>(), B.mom.as<BhMom>(), beta2,
+                         eps, mlp_img, log_tol, cnt + 3, buf[d & 1], cnt + 4 + 2 * (d + 1), P.cap,
+                         B.leaves.as<BhItem>(), cnt + 5, P.cap, d_sum, d_err);
     FLK_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(leafk, dim3(P.grid_leaf), dim3(kTravBlock), 0, s, B.leaves.as<BhItem>(), P.cap,
-                     (const unsigned long long *)(cnt + 5), B.geo.as<BhGeo>(), B.order.as<uint32_t>(),
-                     cv.hi.as<float4>(), cv.lo.as<float4>(), cv.ed.as<float4>(), d_sum, d_err, cnt);
+  hipLaunchKernelGGL(leafk, dim3(P.grid_leaf), dim3(kTravBlock), 0, s, B.leaves.as<BhItem>(), P.cap, cnt,
+                     (int)P.walk, B.geo.as<BhGeo>(), B.order.as<uint32_t>(), cv.hi.as<float4>(), cv.lo.as<float4>(),
+                     cv.ed.as<float4>(), d_sum, d_err, cnt, P.copies, copy_stride);
   FLK_HIP(hipGetLastError());
 }
 
 // Adds a device-scheduled pass's visits, far fields, leaf segment pairs and
-// network evaluations (from its counters h) to st; false when it overflowed.
+// network evaluations (from its head h) to st; false when it overflowed.
 // Every item is exactly one of: leaf pair, far field, split (two children).
-bool pass_counts(const unsigned long long *h, const PassShape &P, unsigned long long st[4]) {
-  const unsigned long long nleaf = h[5];
-  if ((int64_t)nleaf > P.cap || h[4 + 2 * P.D] != 0) return false;
-  unsigned long long visits = 0, split_children = 0;
-  for (int d = 0; d < P.D; ++d) {
-    if ((int64_t)h[4 + 2 * d] > P.cap || (int64_t)h[4 + 2 * (d + 1)] > P.cap) return false;
-    visits += h[4 + 2 * d];
-    split_children += h[4 + 2 * (d + 1)];
-  }
-  st[0] += visits;
-  st[1] += visits - split_children / 2 - nleaf;
+bool pass_counts(const unsigned long long *h, unsigned long long st[4]) {
+  if (h[6] != 0) return false;
+  st[0] += h[0];
+  st[1] += h[0] - h[1] - h[5];
   st[2] += h[2];
   st[3] += h[3];
   return true;
@@ -1915,30 +2246,15 @@ struct BatchPlan {
   bool device = false;  // the device schedule holds it
   std::vector<double> v, e;
   std::vector<uint32_t> f;
-  std::vector<unsigned long long> counts;  // both passes' counters, nslots each
-  // In a graph: ra, rb and beta2 uploaded once (dsrc), and the read-back into
-  // pinned memory (res), copied into v, e, f and counts after the launch.
+  std::vector<unsigned long long> counts;  // both passes' heads
+  // The read-back's end: pinned, in the device buffer's layout (v, e, counts, f).
+  HostBuf res;
+  size_t res_bytes() const { return 20 * idx.size() + 8 * counts.size(); }
+  // In a graph: ra, rb and beta2 uploaded once (dsrc).
   DevBuf dconst;
   std::vector<const void *> dsrc;
-  HostBuf res;
-  double *hv = nullptr, *he = nullptr;
-  uint32_t *hf = nullptr;
-  unsigned long long *hc = nullptr;
-  // where the read-back lands: the vectors, or res
-  void land_in_vectors() {
-    hv = v.data();
-    he = e.data();
-    hf = f.data();
-    hc = counts.data();
-  }
-  void land_pinned(hipStream_t s) {
-    const size_t nb = idx.size(), nc = counts.size();
-    res.reserve(16 * nb + 4 * nb + 8 * nc + 64);
-    unsigned char *p = res.as<unsigned char>();
-    hv = reinterpret_cast<double *>(p);
-    he = hv + nb;
-    hc = reinterpret_cast<unsigned long long *>(he + nb);
-    hf = reinterpret_cast<uint32_t *>(hc + nc);
+  void upload(hipStream_t s) {
+    const size_t nb = idx.size();
     dsrc = upload_pack(dconst, {{ra.data(), 4 * nb}, {rb.data(), 4 * nb}, {beta2.data(), 4 * nb}}, s);
     forest.dsrc = upload_pack(forest.dconst,
                               {{forest.seg_off.data(), 8 * forest.seg_off.size()},
@@ -1951,11 +2267,14 @@ struct BatchPlan {
                               s);
   }
   void collect() {  // pinned read-back into the vectors
-    if (hv == v.data()) return;
+    const double *hv = res.as<double>();
     std::copy(hv, hv + v.size(), v.begin());
-    std::copy(he, he + e.size(), e.begin());
-    std::copy(hf, hf + f.size(), f.begin());
+    hv += v.size();
+    std::copy(hv, hv + e.size(), e.begin());
+    const auto *hc = reinterpret_cast<const unsigned long long *>(hv + e.size());
     std::copy(hc, hc + counts.size(), counts.begin());
+    const auto *hf = reinterpret_cast<const uint32_t *>(hc + counts.size());
+    std::copy(hf, hf + f.size(), f.begin());
   }
 };
 
@@ -1980,54 +2299,61 @@ void plan_batch(flk_ctx *ctx, const int32_t *pairs, std::vector<int64_t> idx, co
     bp.ra[t] = root[pairs[2 * bp.idx[t]]];
     bp.rb[t] = root[pairs[2 * bp.idx[t] + 1]];
   }
-  bp.device = plan_device_passes(ctx, nb, (int)bp.forest.level_base.size(), use_mlp, bp.shape);
+  bp.device = plan_device_passes(ctx, nb, bp.forest.S, (int)bp.forest.level_base.size(), use_mlp, bp.shape);
   BhScratch &B = ctx->bh;
   B.roots_a.reserve(sizeof(int32_t) * nb);
   B.roots_b.reserve(sizeof(int32_t) * nb);
   B.beta2.reserve(sizeof(float) * 2 * nb);
   B.items0.reserve(sizeof(BhItem) * nb);
   B.redo.reserve(sizeof(int32_t) * nb);
-  B.sum.reserve(sizeof(double) * 2 * nb);
-  B.err.reserve(sizeof(double) * 2 * nb);
-  B.outv.reserve(sizeof(double) * nb);
-  B.oute.reserve(sizeof(double) * nb);
-  B.outf.reserve(sizeof(uint32_t) * nb);
-  B.cnt.reserve(sizeof(unsigned long long) * std::max(2 * bp.shape.nslots, kHostCounterWords + 8));
+  B.sum.reserve(sizeof(double) * 2 * nb * bp.shape.copies);
+  B.err.reserve(sizeof(double) * 2 * nb * bp.shape.copies);
+  B.cnt.reserve(sizeof(unsigned long long) * std::max(2 * kPassWords, kHostCounterWords + 8));
   if (use_mlp) mlp_upload(ctx);
   bp.v.assign(nb, 0.0);
   bp.e.assign(nb, 0.0);
   bp.f.assign(nb, 0u);
-  bp.counts.assign(2 * (size_t)bp.shape.nslots, 0ull);
-  bp.land_in_vectors();
+  bp.counts.assign(2 * kPassHead, 0ull);
+  B.out.reserve(bp.res_bytes());
+  bp.res.reserve(bp.res_bytes());
 }
 
 // The batch's merge of both passes into per-pair results, and their read-back.
-void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, const unsigned long long *n_redo,
+// cnt: the device-scheduled passes' counters, null for a host-driven batch.
+void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, unsigned long long *cnt, hipStream_t s) {
+  BhScratch &B = ctx->bh;
+  const int64_t nb = (int64_t)bp.idx.size();
+  double *v = B.out.as<double>(), *e = v + nb;
+  auto *heads = reinterpret_cast<unsigned long long *>(e + nb);
+  auto *f = reinterpret_cast<uint32_t *>(heads + bp.counts.size());
+  hipLaunchKernelGGL(bh_merge, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, nb,
+                     (const int32_t *)B.redo.as<int32_t>(), (const double *)B.sum.as<double>(),
+                     (const double *)B.err.as<double>(), bp.shape.copies, 2 * nb,
+                     prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, v, e, f, heads, cnt, bp.shape.cap,
+                     bp.shape.D);
+  FLK_HIP(hipGetLastError());
+  FLK_HIP(hipMemcpyAsync(bp.res.ptr, B.out.ptr, bp.res_bytes(), hipMemcpyDeviceToHost, s));
+}
+
+void enqueue_adapt(flk_ctx *ctx, const BatchPlan &bp, const flk_params &prm, unsigned long long *n_redo,
                    hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size();
-  const int mlp = prm.criterion == FLK_CRIT_MLP ? 1 : 0;
-  const unsigned g = (unsigned)((nb + 255) / 256);
-  hipLaunchKernelGGL(bh_merge_first, dim3(g), dim3(256), 0, s, nb, (const double *)B.sum.as<double>(),
-                     (const double *)B.err.as<double>(), mlp, prm.err_scale, B.outv.as<double>(),
-                     B.oute.as<double>(), B.outf.as<uint32_t>());
-  hipLaunchKernelGGL(bh_merge_redo, dim3(g), dim3(256), 0, s, nb, n_redo, (const int32_t *)B.redo.as<int32_t>(),
-                     (const double *)(B.sum.as<double>() + nb), (const double *)(B.err.as<double>() + nb), mlp,
-                     prm.err_scale, B.outv.as<double>(), B.oute.as<double>(), B.outf.as<uint32_t>());
+  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(256), 0, s, nb, (const int32_t *)B.roots_a.as<int32_t>(),
+                     (const int32_t *)B.roots_b.as<int32_t>(), (const double *)B.err.as<double>(), bp.shape.copies,
+                     2 * nb, prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, prm.target_error, prm.beta_init,
+                     prm.beta_limit, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, B.redo.as<int32_t>(), n_redo);
   FLK_HIP(hipGetLastError());
-  FLK_HIP(hipMemcpyAsync(bp.hv, B.outv.ptr, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
-  FLK_HIP(hipMemcpyAsync(bp.he, B.oute.ptr, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
-  FLK_HIP(hipMemcpyAsync(bp.hf, B.outf.ptr, sizeof(uint32_t) * nb, hipMemcpyDeviceToHost, s));
 }
 
-void enqueue_adapt(flk_ctx *ctx, int64_t nb, const flk_params &prm, unsigned long long *cnt2, int nslots2,
-                   hipStream_t s) {
+// Clears the sums and both passes' counters and lists the root items.
+void enqueue_begin(flk_ctx *ctx, const BatchPlan &bp, hipStream_t s) {
   BhScratch &B = ctx->bh;
-  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(256), 0, s, nb, (const int32_t *)B.roots_a.as<int32_t>(),
-                     (const int32_t *)B.roots_b.as<int32_t>(), (const double *)B.err.as<double>(),
-                     prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, prm.target_error, prm.beta_init,
-                     prm.beta_limit, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, B.redo.as<int32_t>(), cnt2,
-                     nslots2, 4);
+  const int64_t nb = (int64_t)bp.idx.size(), nsums = 2 * nb * bp.shape.copies;
+  hipLaunchKernelGGL(bh_begin, dim3((unsigned)((std::max<int64_t>(nsums, 2 * kPassWords) + 255) / 256)), dim3(256), 0,
+                     s, (const int32_t *)B.roots_a.as<int32_t>(), (const int32_t *)B.roots_b.as<int32_t>(), nb,
+                     B.items0.as<BhItem>(), B.cnt.as<unsigned long long>(), nsums, B.sum.as<double>(),
+                     B.err.as<double>());
   FLK_HIP(hipGetLastError());
 }
 
@@ -2044,25 +2370,16 @@ void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipSt
   const float eps = (float)(prm.eps_sq * cv.scale * cv.scale);
   const float log_tol = (float)prm.mlp_log_tol;
   double *sum = B.sum.as<double>(), *err = B.err.as<double>();
-  hipLaunchKernelGGL(bh_zero_f64, dim3((unsigned)((2 * nb + 255) / 256)), dim3(256), 0, s, sum, 2 * nb);
-  hipLaunchKernelGGL(bh_zero_f64, dim3((unsigned)((2 * nb + 255) / 256)), dim3(256), 0, s, err, 2 * nb);
   put(B.roots_a.ptr, bp.ra.data(), bp.dsrc, 0, sizeof(int32_t) * nb, s);
   put(B.roots_b.ptr, bp.rb.data(), bp.dsrc, 1, sizeof(int32_t) * nb, s);
   put(B.beta2.ptr, bp.beta2.data(), bp.dsrc, 2, sizeof(float) * nb, s);
-  unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + P.nslots;
-  hipLaunchKernelGGL(bh_pass_init, dim3((unsigned)((P.nslots + 255) / 256)), dim3(256), 0, s, c1, P.nslots, 4,
-                     (unsigned long long)nb);
-  hipLaunchKernelGGL(bh_roots, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s,
-                     (const int32_t *)B.roots_a.as<int32_t>(), (const int32_t *)B.roots_b.as<int32_t>(), nb,
-                     B.items0.as<BhItem>());
-  FLK_HIP(hipGetLastError());
-  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>(), eps, use_mlp, log_tol, c1, sum, err, s);
-  enqueue_adapt(ctx, nb, prm, c2, P.nslots, s);
-  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, eps, use_mlp, log_tol - 1.0f, c2,
-               sum + nb, err + nb, s);
-  enqueue_merge(ctx, bp, prm, c2 + 4, s);
-  FLK_HIP(hipMemcpyAsync(bp.hc, c1, sizeof(unsigned long long) * 2 * P.nslots, hipMemcpyDeviceToHost,
-                         s));
+  enqueue_begin(ctx, bp, s);
+  unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + kPassWords;
+  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>(), eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);
+  enqueue_adapt(ctx, bp, prm, c2 + 4, s);
+  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, eps, use_mlp, log_tol - 1.0f, c2, sum + nb,
+               err + nb, 2 * nb, s);
+  enqueue_merge(ctx, bp, prm, c1, s);
 }
 
 // Results and statistics of a batch whose read-back has arrived; false when
@@ -2071,13 +2388,13 @@ bool finish_batch(flk_ctx *ctx, const BatchPlan &bp, std::vector<double> &lk, st
                   std::vector<uint32_t> &flags) {
   unsigned long long st[4] = {0, 0, 0, 0};
   const unsigned long long *h = bp.counts.data();
-  if (!pass_counts(h, bp.shape, st) || !pass_counts(h + bp.shape.nslots, bp.shape, st)) return false;
+  if (!pass_counts(h, st) || !pass_counts(h + kPassHead, st)) return false;
   for (size_t t = 0; t < bp.idx.size(); ++t) {
     lk[bp.idx[t]] = bp.v[t];
     err[bp.idx[t]] = bp.e[t];
     flags[bp.idx[t]] |= bp.f[t];
   }
-  ctx->stats.retries += (int64_t)h[bp.shape.nslots + 4];
+  ctx->stats.retries += (int64_t)h[kPassHead + 4];
   ctx->stats.bh_visits += (int64_t)st[0];
   ctx->stats.bh_far += (int64_t)st[1];
   ctx->stats.bh_leaf_pairs += (int64_t)st[2];
@@ -2106,12 +2423,13 @@ void bh_batch_host(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t
   const int64_t nb = (int64_t)bp.idx.size();
   const float eps = (float)(prm.eps_sq * ctx->curves.scale * ctx->curves.scale);
   double *sum = B.sum.as<double>(), *err_d = B.err.as<double>();
-  hipLaunchKernelGGL(bh_zero_f64, dim3((unsigned)((2 * nb + 255) / 256)), dim3(256), 0, s, sum, 2 * nb);
-  hipLaunchKernelGGL(bh_zero_f64, dim3((unsigned)((2 * nb + 255) / 256)), dim3(256), 0, s, err_d, 2 * nb);
+  put(B.roots_a.ptr, bp.ra.data(), {}, 0, sizeof(int32_t) * nb, s);
+  put(B.roots_b.ptr, bp.rb.data(), {}, 1, sizeof(int32_t) * nb, s);
+  enqueue_begin(ctx, bp, s);
   unsigned long long st[4] = {0, 0, 0, 0};
   traverse(ctx, F, bp.ra, bp.rb, bp.beta2, eps, sum, err_d, st, use_mlp, (float)prm.mlp_log_tol, prm.timing != 0);
   unsigned long long *c2 = B.cnt.as<unsigned long long>() + kHostCounterWords;
-  enqueue_adapt(ctx, nb, prm, c2, 8, s);
+  enqueue_adapt(ctx, bp, prm, c2 + 4, s);
   unsigned long long nr = 0;
   FLK_HIP(hipMemcpyAsync(&nr, c2 + 4, sizeof nr, hipMemcpyDeviceToHost, s));
   FLK_HIP(hipStreamSynchronize(s));
@@ -2131,8 +2449,9 @@ void bh_batch_host(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t
              prm.timing != 0);
     passes = 2;
   }
-  enqueue_merge(ctx, bp, prm, c2 + 4, s);
+  enqueue_merge(ctx, bp, prm, nullptr, s);
   FLK_HIP(hipStreamSynchronize(s));
+  bp.collect();
   for (size_t t = 0; t < bp.idx.size(); ++t) {
     lk[bp.idx[t]] = bp.v[t];
     err[bp.idx[t]] = bp.e[t];
@@ -2171,6 +2490,7 @@ void bh_batch(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t> &id
   t0 = std::chrono::steady_clock::now();
   enqueue_traversal(ctx, bp, prm, s);
   FLK_HIP(hipStreamSynchronize(s));
+  bp.collect();
   ctx->stats.ms_bh_traverse +=
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (!finish_batch(ctx, bp, lk, err, flags)) bh_batch_host(ctx, pairs, idx, prm, lk, err, flags);
@@ -2290,7 +2610,7 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
       BatchPlan &bp = NG->batches.back();
       plan_batch(ctx, pairs, std::move(idx), prm, bp);
       if (!bp.device) return false;
-      bp.land_pinned(s);
+      bp.upload(s);
     }
     if (!ds_idx.empty()) {
       // Beside the Barnes-Hut branch the direct-sum kernel takes a share of

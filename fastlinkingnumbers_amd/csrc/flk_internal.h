@@ -195,11 +195,10 @@ struct BhScratch {
   // forest
   DevBuf geo, mom, order, m64, range, child, flag, flag2, scan, keys0, keys1, ids0, tmp, seg, vtx, box, sp, rtiles, rcurve;
   // traversal: root items of a pass, re-run list, per-pair sums and results
-  DevBuf roots_a, roots_b, beta2, cnt, leaves, pred, sum, err, items0, redo, outv, oute, outf;
+  DevBuf roots_a, roots_b, beta2, cnt, leaves, pred, sum, err, items0, redo, out;
   std::vector<std::unique_ptr<DevBuf>> levels;
   unsigned long long *host_cnt = nullptr;  // pinned, 2 words per level of a traversal round trip
-  int64_t dev_cap = 0;                     // items per level buffer of the device-scheduled pass
-  std::vector<unsigned long long> dev_counts;  // its per-level counts, read back once per pass
+  int64_t dev_cap = 0;                     // leaf items of a device-scheduled pass
   BhScratch() {
     each([](DevBuf &b) { b.tracked = true; });
   }
@@ -210,7 +209,7 @@ struct BhScratch {
   template <typename Fn> void each(Fn fn) {
     DevBuf *all[] = {&geo, &mom, &order, &m64, &range, &child, &flag, &flag2, &scan, &keys0, &keys1, &ids0,
                      &tmp, &seg, &vtx, &box, &sp, &rtiles, &rcurve, &roots_a, &roots_b, &beta2, &cnt, &leaves, &pred,
-                     &sum, &err, &items0, &redo, &outv, &oute, &outf};
+                     &sum, &err, &items0, &redo, &out};
     for (DevBuf *b : all) fn(*b);
     for (auto &b : levels) fn(*b);
   }

@@ -1,0 +1,70 @@
+"""The depth-first walk of batches with few segments a pair, against the
+host-driven level-by-level schedule (timing = 1): the same node pairs visited,
+far fields, leaf pairs and re-runs, and the same FP32 terms summed in another
+order in FP64 (1e-9, as the other schedules' tests)."""
+import numpy as np
+import pytest
+
+flk = pytest.importorskip("fastlinkingnumbers_amd")
+from fastlinkingnumbers_amd import workloads as W  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = ("bh_visits", "bh_far", "bh_leaf_pairs", "retries")
+
+
+def _check(engine, pairs, **kw):
+    kw = dict(method="barneshut", fallback_tol=0.0, **kw)
+    walked = engine.linking_numbers(pairs, **kw)
+    levels = engine.linking_numbers(pairs, timing=1, **kw)
+    assert walked.stats["bh_host_passes"] == 0 and levels.stats["bh_host_passes"] >= 1
+    for key in COUNTS:
+        assert walked.stats[key] == levels.stats[key], key
+    np.testing.assert_allclose(walked.lk, levels.lk, rtol=0, atol=1e-9)
+    np.testing.assert_allclose(walked.err, levels.err, rtol=1e-9, atol=1e-300)
+    assert np.array_equal(walked.flags, levels.flags)
+    return walked
+
+
+@pytest.mark.parametrize("n,m", [(2, 2), (2, 3), (5, 4), (63, 65), (64, 1000), (1023, 1025), (9000, 700),
+                                 (20000, 12000)])
+def test_one_pair(engine, n, m):
+    t, u = 2 * np.pi * np.arange(n) / n, 2 * np.pi * np.arange(m) / m
+    a = np.stack([np.cos(t), np.sin(t), 0.05 * np.sin(5 * t)], 1)
+    b = np.stack([1 + np.cos(u), 0.05 * np.cos(3 * u), np.sin(u)], 1)
+    engine.set_curves([a, b])
+    for leaf in (1, 4):
+        _check(engine, [[0, 1], [1, 0]], leaf_size=leaf)
+
+
+def test_tangled_pair_is_re_run(engine):
+    """One root pair with much work: it spreads over every wave through the
+    queues, and the adaptive re-run walks again."""
+    engine.set_curves(W.random_walk_pair(seed=3, n=16000, rg=25.0, workload=3))
+    assert _check(engine, [[0, 1]]).stats["retries"] == 1
+
+
+@pytest.mark.parametrize("copies", [8, 1])
+def test_many_pairs(engine, copies):
+    """Chain mail; with every pair of curves (more than 4,096) the sums have one
+    copy instead of eight."""
+    curves = W.chainmail(seed=5, grid=10, nmin=16, nmax=700)
+    engine.set_curves(curves)
+    pairs = engine.potential_links() if copies == 8 else np.array(
+        [(i, j) for i in range(100) for j in range(i + 1, 100)], dtype=np.int32)
+    assert (len(pairs) <= 4096) == (copies == 8)
+    _check(engine, pairs)
+
+
+def test_overflow_goes_to_the_host(engine):
+    engine.set_curves(W.random_walk_pair(seed=1, n=15000, rg=25.0, workload=3))
+    kw = dict(method="barneshut", fallback_tol=0.0)
+    base = engine.linking_numbers([[0, 1]], **kw)
+    assert base.stats["bh_host_passes"] == 0
+    for capacity in (64, 4096):
+        engine.set_tune(bh_level_capacity=capacity)
+        small = engine.linking_numbers([[0, 1]], **kw)
+        assert small.stats["bh_host_passes"] >= 1
+        for key in COUNTS:
+            assert small.stats[key] == base.stats[key], key
+        np.testing.assert_allclose(small.lk, base.lk, rtol=0, atol=1e-9)

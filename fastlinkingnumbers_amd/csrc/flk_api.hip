@@ -460,18 +460,10 @@ int32_t flk_discretize(flk_ctx *ctx, const double *ctrl_xyz, const int64_t *offs
   try {
     FLK_HIP(hipSetDevice(ctx->device));
     if (ncurves > 0 && offsets[0] != 0) throw Error(FLK_ERR_ARG, "offsets[0] must be 0");
-    std::vector<double> current;
-    if (!ctrl_xyz && ncurves > 0 && offsets[ncurves] > 0) {
-      // the control points are the current curve set's input array; the
-      // reference's guard and extent loops read them on the host
+    if (!ctrl_xyz && ncurves > 0 && offsets[ncurves] > 0) {  // the current curve set's input array
       const flk::Curves &cv = ctx->curves;
       if (cv.ncurves != ncurves || !std::equal(offsets, offsets + ncurves + 1, cv.in_off.begin()))
         throw Error(FLK_ERR_ARG, "offsets do not match the current curve set");
-      current.resize(3 * (size_t)offsets[ncurves]);
-      FLK_HIP(hipMemcpyAsync(current.data(), cv.raw.ptr, sizeof(double) * current.size(), hipMemcpyDeviceToHost,
-                             ctx->stream));
-      FLK_HIP(hipStreamSynchronize(ctx->stream));
-      ctrl_xyz = current.data();
     }
     flk::discretize_run(ctx, ctrl_xyz, offsets, segment_types, looped, ncurves, pairs, npairs, ctx->disc,
                         out_xyz != nullptr);

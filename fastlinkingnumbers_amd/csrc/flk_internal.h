@@ -272,6 +272,16 @@ struct DiscResult {
   double small_size = 0.0;
 };
 
+// Scratch of a discretization, kept by the context between calls (grow-only).
+struct DiscScratch {
+  struct Gen {  // pieces: curve, segment, parameter range, box
+    DevBuf c, s, lo, hi, box;
+  } gen[2], ret;
+  DevBuf q, land, cs, links, cnt, diag, part;
+  DevBuf keys0, keys1, ids0, ids1, heap, hit, flag, scan, tmp;
+  DevBuf k0, k1, i0, i1, i2, ob, open, out, per_curve;
+};
+
 struct MlpState {
   std::vector<float> params;  // FLK_MLP_NPARAM FP32 masters
   std::vector<float> norm;    // mean[12], std[12]
@@ -307,6 +317,7 @@ struct flk_ctx {
   flk::DsGraph ds_graph[2];      // FP32, FP64 batches
   std::shared_ptr<flk::CertGraph> cert_graph;  // last Barnes–Hut certificate graph
   flk::DiscResult disc;          // last flk_discretize result
+  flk::DiscScratch disc_scratch;
   flk::BccLoad bcc;              // last flk_load_bcc result
   flk::DevBuf bcc_land;          // FP32 landing area of flk_load_bcc
   uint64_t curves_version = 0;   // bumped by every flk_set_curves
@@ -373,8 +384,9 @@ void *noalloc_scratch_init(int device);
 void ds_run_noalloc(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, std::vector<double> &lk_out,
                     float *ms_kernel);
 
-// Spline-to-polyline discretization of the given curves against the given
-// potentially linked pairs (see disc.hip); the polylines become the context's
+// Spline-to-polyline discretization of the given curves (ctrl null: the current
+// curve set's input points, with these offsets) against the given potentially
+// linked pairs (see disc.hip); the polylines become the context's
 // curve set, and res.xyz a host copy of them when host_copy is set.
 void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, const int32_t *types,
                     const uint8_t *looped, int32_t nc, const int32_t *pairs, int64_t npairs, DiscResult &res,

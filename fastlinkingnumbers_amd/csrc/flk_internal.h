@@ -278,7 +278,7 @@ struct DiscScratch {
     DevBuf c, s, lo, hi, box;
   } gen[2], ret;
   DevBuf q, land, cs, links, cnt, diag, part;
-  DevBuf keys0, keys1, ids0, ids1, heap, hit, flag, scan, tmp;
+  DevBuf heap, curve_end, hit, flag, scan, tmp;
   DevBuf k0, k1, i0, i1, i2, ob, open, out, per_curve;
 };
 

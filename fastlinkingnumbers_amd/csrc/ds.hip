@@ -803,22 +803,14 @@ float ds_eager(flk_ctx *ctx, const DsPlan &P, std::vector<double> *lk_out) {
   return ms;
 }
 
-uint64_t fnv1a(uint64_t h, const void *p, size_t n) {
-  const unsigned char *c = static_cast<const unsigned char *>(p);
-  for (size_t i = 0; i < n; ++i) h = (h ^ c[i]) * 0x100000001b3ULL;
-  return h;
-}
-
-// Graph run: the batch is captured once per (pairs, shape, precision, curve
-// set) and replayed after that.  The graph is timed whole (its uploads and
+// Graph run: the batch is captured once per (pairs, curves' sizes, shape,
+// precision) and replayed after that.  The graph is timed whole (its uploads and
 // the reduction add well under a percent to a batch worth a launch).
 float ds_graph_run(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, std::vector<double> &lk_out,
                    int64_t *work) {
   const flk_tune &t = ctx->tune;
-  uint64_t key = fnv1a(0xcbf29ce484222325ULL, pairs, sizeof(int32_t) * 2 * (size_t)npairs);
-  const int64_t meta[7] = {npairs, t.ds_rows_per_lane, t.ds_blocks_per_cu, t.ds_tasks_per_wave, fp64 ? 1 : 0,
-                           (int64_t)ctx->curves_version, ctx->curves.inexact ? 1 : 0};
-  key = fnv1a(key, meta, sizeof meta);
+  GraphKey key(ctx, pairs, npairs);
+  key.add(std::array<int32_t, 3>{t.ds_rows_per_lane, t.ds_blocks_per_cu, t.ds_tasks_per_wave});
   DsGraph &G = ctx->ds_graph[fp64 ? 1 : 0];
   hipStream_t s = ctx->stream;
   if (!(G.exec && G.key == key)) {
@@ -862,7 +854,7 @@ float ds_graph_run(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64
       G.exec = nullptr;
       throw Error(FLK_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
     }
-    G.key = key;
+    G.key = std::move(key);
   }
   FLK_HIP(hipEventRecord(ctx->ev0, s));
   FLK_HIP(hipGraphLaunch(G.exec, s));

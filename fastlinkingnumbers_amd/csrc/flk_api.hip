@@ -63,9 +63,6 @@ int64_t curves_layout(flk_ctx *ctx, const int64_t *offsets, int32_t ncurves) {
   cv.ed.reserve(sizeof(float4) * nd);
   cv.inexact = false;
   cv.bh_budget = 0;
-  ++ctx->curves_version;
-  for (auto &g : ctx->ds_graph) g.reset();
-  ctx->cert_graph.reset();
   return nv;
 }
 
@@ -79,7 +76,6 @@ void curves_clear(flk_ctx *ctx) {
   cv.nvert_dev = 0;
   cv.inexact = false;
   cv.bh_budget = 0;
-  ++ctx->curves_version;
   for (auto &g : ctx->ds_graph) g.reset();
   ctx->cert_graph.reset();
 }

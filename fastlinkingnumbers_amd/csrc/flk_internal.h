@@ -4,9 +4,11 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <atomic>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 #include <memory>
 #include <vector>
 
@@ -193,10 +195,11 @@ struct HostStage {
 // FP64 build records and the traversal queues.
 struct BhScratch {
   // forest
-  DevBuf geo, mom, order, m64, range, child, loff, vals, keys0, keys1, ids0, tmp, seg, vtx, box, sp, rtiles, rcurve;
+  DevBuf geo, mom, order, m64, range, child, loff, vals, keys0, keys1, ids0, tmp, sp, pack;
   // traversal: root items of a pass, re-run list, per-pair sums and results
   DevBuf roots_a, roots_b, beta2, cnt, leaves, pred, sum, err, items0, redo, out;
   std::vector<std::unique_ptr<DevBuf>> levels;
+  HostBuf pack_host;                       // pinned: the plans' arrays on their way to `pack`
   unsigned long long *host_cnt = nullptr;  // pinned, 2 words per level of a traversal round trip
   int64_t dev_cap = 0;                     // leaf items of a device-scheduled pass
   BhScratch() {
@@ -208,7 +211,7 @@ struct BhScratch {
   }
   template <typename Fn> void each(Fn fn) {
     DevBuf *all[] = {&geo, &mom, &order, &m64, &range, &child, &loff, &vals, &keys0, &keys1, &ids0,
-                     &tmp, &seg, &vtx, &box, &sp, &rtiles, &rcurve, &roots_a, &roots_b, &beta2, &cnt, &leaves, &pred,
+                     &tmp, &sp, &pack, &roots_a, &roots_b, &beta2, &cnt, &leaves, &pred,
                      &sum, &err, &items0, &redo, &out};
     for (DevBuf *b : all) fn(*b);
     for (auto &b : levels) fn(*b);
@@ -226,12 +229,29 @@ struct BhScratch {
   }
 };
 
-// A captured direct-sum batch (uploads, tile kernel, per-pair reduction,
-// read-back) for replay when the same pairs come again with the same shape
-// and curves.  It owns its device buffers and host staging, so reallocations
-// elsewhere cannot leave dangling pointers in the graph.
+// What a captured graph was made for, all compared in full: the pairs, the
+// curves' sizes (and so their places in the vertex arrays), those arrays'
+// addresses, and what else its plan or its kernels' arguments depend on.  The
+// coordinates are not part of it: kernels read them where they are.
+struct GraphKey {
+  std::vector<int32_t> pairs, sizes;
+  std::vector<unsigned char> rest;
+  GraphKey() = default;
+  GraphKey(const flk_ctx *ctx, const int32_t *p, int64_t npairs);
+  template <typename T> void add(const T &v) {
+    static_assert(std::is_trivially_copyable_v<T>);
+    const auto *b = reinterpret_cast<const unsigned char *>(&v);
+    rest.insert(rest.end(), b, b + sizeof v);
+  }
+  bool operator==(const GraphKey &o) const { return rest == o.rest && sizes == o.sizes && pairs == o.pairs; }
+};
+
+// A captured direct-sum batch (tile kernel, per-pair reduction, read-back) for
+// replay when the same pairs of curves of the same sizes come again.  It owns
+// its device buffers and host staging, so reallocations elsewhere cannot leave
+// dangling pointers in the graph.
 struct DsGraph {
-  uint64_t key = 0;
+  GraphKey key;
   hipGraphExec_t exec = nullptr;
   int64_t work = 0;
   int32_t waves = 0;
@@ -247,7 +267,12 @@ struct DsGraph {
   void reset() {
     if (exec) (void)hipGraphExecDestroy(exec);
     exec = nullptr;
-    key = 0;
+  }
+  void take_buffers(DsGraph &o) {
+    DevBuf *mine[] = {&d_pairs, &d_tasks, &d_cost, &d_theta, &d_corr, &d_task0, &d_out};
+    DevBuf *from[] = {&o.d_pairs, &o.d_tasks, &o.d_cost, &o.d_theta, &o.d_corr, &o.d_task0, &o.d_out};
+    for (int k = 0; k < 7; ++k) std::swap(*mine[k], *from[k]);
+    std::swap(h_out, o.h_out);
   }
   ~DsGraph() { reset(); }
 };
@@ -320,13 +345,19 @@ struct flk_ctx {
   flk::DiscScratch disc_scratch;
   flk::BccLoad bcc;              // last flk_load_bcc result
   flk::DevBuf bcc_land;          // FP32 landing area of flk_load_bcc
-  uint64_t curves_version = 0;   // bumped by every flk_set_curves
   void *noalloc_scratch = nullptr;  // this device's fixed direct-sum array (ds.hip)
   // scratch
   flk::DevBuf d_pairs, d_tasks, d_cost, d_task_theta, d_task_corr, d_pair_task0,
       d_pair_out, d_pair_corr, d_boxes, d_pls, d_pls_boxes, d_count, d_misc;
   flk::HostBuf pls_host;         // pinned: the potential-link search's total and pairs
 };
+
+inline flk::GraphKey::GraphKey(const flk_ctx *ctx, const int32_t *p, int64_t npairs)
+    : pairs(p, p + 2 * npairs), sizes(ctx->curves.n) {
+  const Curves &cv = ctx->curves;
+  add(std::array<const void *, 4>{cv.dpts.ptr, cv.hi.ptr, cv.lo.ptr, cv.ed.ptr});
+  add(cv.inexact);
+}
 
 namespace flk {
 

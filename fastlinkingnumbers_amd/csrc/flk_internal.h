@@ -307,7 +307,15 @@ struct DiscScratch {
   DevBuf k0, k1, i0, i1, i2, ob, open, out, per_curve;
 };
 
+// Scratch of a gradient or a training, kept between calls (grow-only): the set,
+// the batch order, Adam's moments (m also a gradient's sum), the blocks' sums
+// and the loss.
+struct MlpScratch {
+  DevBuf x, t, idx, m, v, part, loss;
+};
+
 struct MlpState {
+  MlpScratch scratch;
   std::vector<float> params;  // FLK_MLP_NPARAM FP32 masters
   std::vector<float> norm;    // mean[12], std[12]
   bool loaded = false;

@@ -72,23 +72,38 @@ __device__ __forceinline__ bf16x8 a_frag(const __bf16 *m, int ld, int k0) {
   return v;
 }
 
-// Loads the weights into LDS (bf16 copies are made here from FP32 masters).
+// Loads the weights into LDS (bf16 copies are made here from FP32 masters),
+// every global load of a thread in flight at once.  256 threads.
 __device__ void load_weights(BlockLds &L, const float *__restrict__ P, const float *__restrict__ norm) {
-  for (int t = threadIdx.x; t < H * KP; t += blockDim.x) {
-    const int j = t / KP, i = t % KP;
-    L.w1[j][i] = (__bf16)(i < FLK_MLP_NFEAT ? P[OFF_W1 + j * FLK_MLP_NFEAT + i] : 0.0f);
+  static_assert(FLK_MLP_NFEAT % 4 == 0 && FLK_MLP_NFEAT * H / 4 <= 256 && OFF_W2 % 4 == 0, "whole float4 rows");
+  constexpr int kRow = FLK_MLP_NFEAT / 4;  // float4s of a row of W1
+  const int t = threadIdx.x;
+  const float4 *w1 = reinterpret_cast<const float4 *>(P + OFF_W1), *w2 = reinterpret_cast<const float4 *>(P + OFF_W2);
+  float4 v2[H * H / 1024], v1{};
+#pragma unroll
+  for (int q = 0; q < H * H / 1024; ++q) v2[q] = w2[t + 256 * q];
+  if (t < kRow * H) v1 = w1[t];
+  // the biases and W3 (a thread each), and the normalisation
+  const int j = t & (H - 1);
+  const float b = t < H ? P[OFF_B1 + j] : t < 2 * H ? P[OFF_B2 + j] : t < 3 * H ? P[OFF_W3 + j] : t == 3 * H ? P[OFF_B3] : 0.f;
+  const float nm = t < 2 * FLK_MLP_NFEAT ? norm[t] : 1.f;
+#pragma unroll
+  for (int q = 0; q < H * H / 1024; ++q) {
+    __bf16 *d = &L.w2[0][0] + 4 * (t + 256 * q);
+    d[0] = (__bf16)v2[q].x; d[1] = (__bf16)v2[q].y; d[2] = (__bf16)v2[q].z; d[3] = (__bf16)v2[q].w;
   }
-  for (int t = threadIdx.x; t < H * H; t += blockDim.x) L.w2[t / H][t % H] = (__bf16)P[OFF_W2 + t];
-  for (int t = threadIdx.x; t < H; t += blockDim.x) {
-    L.b1[t] = P[OFF_B1 + t];
-    L.b2[t] = P[OFF_B2 + t];
-    L.w3[t] = P[OFF_W3 + t];
+  if (t < kRow * H) {
+    __bf16 *d = &L.w1[t / kRow][4 * (t % kRow)];
+    d[0] = (__bf16)v1.x; d[1] = (__bf16)v1.y; d[2] = (__bf16)v1.z; d[3] = (__bf16)v1.w;
   }
-  if (threadIdx.x == 0) L.b3 = P[OFF_B3];
-  for (int t = threadIdx.x; t < FLK_MLP_NFEAT; t += blockDim.x) {
-    L.mean[t] = norm[t];
-    L.istd[t] = 1.0f / norm[FLK_MLP_NFEAT + t];
-  }
+  for (int k = t; k < H * (KP - FLK_MLP_NFEAT); k += 256)
+    L.w1[k / (KP - FLK_MLP_NFEAT)][FLK_MLP_NFEAT + k % (KP - FLK_MLP_NFEAT)] = (__bf16)0.0f;
+  if (t < H) L.b1[j] = b;
+  else if (t < 2 * H) L.b2[j] = b;
+  else if (t < 3 * H) L.w3[j] = b;
+  else if (t == 3 * H) L.b3 = b;
+  if (t < FLK_MLP_NFEAT) L.mean[t] = nm;
+  else if (t < 2 * FLK_MLP_NFEAT) L.istd[t - FLK_MLP_NFEAT] = 1.0f / nm;
   __syncthreads();
 }
 
@@ -147,19 +162,32 @@ __device__ void forward16(const BlockLds &L, WaveLds &W, f32x4 (&z1)[4], f32x4 (
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
-// Stages 16 rows of raw features (rows >= n are zero) normalised into W.x.
-__device__ void stage_x(const BlockLds &L, WaveLds &W, const float *__restrict__ x,
-                        const int64_t *__restrict__ idx, int64_t r0, int64_t n) {
+// 16 rows of a wave: lane l holds features 3 (l / 16) to + 2 of row l % 16, and
+// the row's target.
+struct WaveRows {
+  float x[3], t;
+};
+__device__ __forceinline__ WaveRows load_rows(const float *__restrict__ x, const float *__restrict__ t,
+                                              const int64_t *__restrict__ idx, int64_t r0, int64_t n) {
+  static_assert(FLK_MLP_NFEAT == 12, "three features a lane");
   const int l = threadIdx.x & 63;
-  for (int t = l; t < 16 * KP; t += 64) {
-    const int r = t / KP, i = t % KP;
-    float v = 0.f;
-    if (i < FLK_MLP_NFEAT && r0 + r < n) {
-      const int64_t row = idx ? idx[r0 + r] : r0 + r;
-      v = (x[row * FLK_MLP_NFEAT + i] - L.mean[i]) * L.istd[i];
-    }
-    W.x[r][i] = (__bf16)v;
+  WaveRows v{{0.f, 0.f, 0.f}, 0.f};
+  if (r0 + l % 16 < n) {
+    const int64_t row = idx ? idx[r0 + l % 16] : r0 + l % 16;
+    const float *p = x + row * FLK_MLP_NFEAT + 3 * (l / 16);
+    v = WaveRows{{p[0], p[1], p[2]}, t[row]};
   }
+  return v;
+}
+
+// Stages the rows (those at or past n are zero) normalised into W.x, whose
+// columns past the features are zero already.
+__device__ __forceinline__ void stage_x(const BlockLds &L, WaveLds &W, const WaveRows &v, int64_t r0, int64_t n) {
+  const int l = threadIdx.x & 63, i0 = 3 * (l / 16);
+  const bool live = r0 + l % 16 < n;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    W.x[l % 16][i0 + k] = (__bf16)(live ? (v.x[k] - L.mean[i0 + k]) * L.istd[i0 + k] : 0.f);
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
@@ -189,38 +217,51 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const float *__restric
   }
 }
 
+// A block's sums: every gradient, then the squared error.
+constexpr int kSums = FLK_MLP_NPARAM + 1;
+
 // Forward + backward of the mean squared error over rows idx[0..n) (or 0..n):
-// accumulates d(loss)/d(params) into grad (FP32 atomics, one set per wave)
-// and the summed squared error into loss.  inv_n = 1 / total rows.
+// d(loss)/d(params) and the summed squared error, one set of kSums per block in
+// `part`, the waves' added in LDS in order.  inv_n = 1 / total rows.
+// Bound by latency (a wave has one to a few 16-row tiles): FP32 atomics of every
+// wave on the 5,057 gradients took 56 us for 8,192 rows.
 __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__ P,
                                                        const float *__restrict__ norm,
                                                        const float *__restrict__ x,
                                                        const float *__restrict__ t,
                                                        const int64_t *__restrict__ idx, int64_t n,
-                                                       float inv_n, float *__restrict__ grad,
-                                                       float *__restrict__ loss) {
-  __shared__ BlockLds L;
-  load_weights(L, P, norm);
+                                                       float inv_n, float *__restrict__ part) {
+  __shared__ union {
+    BlockLds L;
+    float sums[2][kSums];
+  } lds;
+  BlockLds &L = lds.L;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   WaveLds &W = L.wv[w];
   const int64_t nwaves = (int64_t)gridDim.x * 4;
+  const int64_t row0 = ((int64_t)blockIdx.x * 4 + w) * 16;
+  WaveRows rows = load_rows(x, t, idx, row0, n);  // in flight beside the weights
+  for (int k = l; k < 16 * (KP - FLK_MLP_NFEAT); k += 64)
+    W.x[k / (KP - FLK_MLP_NFEAT)][FLK_MLP_NFEAT + k % (KP - FLK_MLP_NFEAT)] = (__bf16)0.0f;
+  load_weights(L, P, norm);
   // per-lane gradient accumulators in C layout
   f32x4 gW2[4][4], gW1[4];  // gW2[mb][nb]: rows mb*16.. (output j), cols nb*16.. (input k)
   for (int a = 0; a < 4; ++a) {
     gW1[a] = f32x4{0, 0, 0, 0};
     for (int b = 0; b < 4; ++b) gW2[a][b] = f32x4{0, 0, 0, 0};
   }
-  float gb1 = 0, gb2[4] = {0, 0, 0, 0}, gw3[4] = {0, 0, 0, 0}, gb3 = 0, lsum = 0;
+  float gb2[4] = {0, 0, 0, 0}, gw3[4] = {0, 0, 0, 0}, gb3 = 0, lsum = 0;
   float gb1v[4] = {0, 0, 0, 0};
-  for (int64_t r0 = ((int64_t)blockIdx.x * 4 + w) * 16; r0 < n; r0 += nwaves * 16) {
-    stage_x(L, W, x, idx, r0, n);
+  for (int64_t r0 = row0; r0 < n; r0 += nwaves * 16) {
+    stage_x(L, W, rows, r0, n);
+    const float target = rows.t;
+    rows = load_rows(x, t, idx, r0 + nwaves * 16, n);
     f32x4 z1[4], z2[4];
     forward16(L, W, z1, z2);
     if (l < 16) {
       float dy = 0.f;
       if (r0 + l < n) {
-        const int64_t row = idx ? idx[r0 + l] : r0 + l;
-        const float e = W.y[l] - t[row];
+        const float e = W.y[l] - target;
         lsum += e * e;
         dy = 2.0f * e * inv_n;
       }
@@ -302,58 +343,95 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
     }
     __builtin_amdgcn_wave_barrier();
   }
-  (void)gb1;
-  // flush: C layout row = 4*(l/16)+i within block mb, col = l%16 within nb
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = mb * 16 + 4 * (l / 16) + i;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        atomicAdd(grad + OFF_W2 + j * H + nb * 16 + l % 16, gW2[mb][nb][i]);
-      if (l % 16 < FLK_MLP_NFEAT) atomicAdd(grad + OFF_W1 + j * FLK_MLP_NFEAT + l % 16, gW1[mb][i]);
-    }
-  }
   // bias / w3 sums: reduce over the 4 row groups (lane bits 4,5)
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) {
-    float a = gb2[nb], b = gw3[nb], c = gb1v[nb];
-    a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64);
-    b += __shfl_xor(b, 16, 64); b += __shfl_xor(b, 32, 64);
-    c += __shfl_xor(c, 16, 64); c += __shfl_xor(c, 32, 64);
-    if (l < 16) {
-      atomicAdd(grad + OFF_B2 + nb * 16 + l, a);
-      atomicAdd(grad + OFF_W3 + nb * 16 + l, b);
-      atomicAdd(grad + OFF_B1 + nb * 16 + l, c);
-    }
+    gb2[nb] += __shfl_xor(gb2[nb], 16, 64);
+    gb2[nb] += __shfl_xor(gb2[nb], 32, 64);
+    gw3[nb] += __shfl_xor(gw3[nb], 16, 64);
+    gw3[nb] += __shfl_xor(gw3[nb], 32, 64);
+    gb1v[nb] += __shfl_xor(gb1v[nb], 16, 64);
+    gb1v[nb] += __shfl_xor(gb1v[nb], 32, 64);
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     gb3 += __shfl_xor(gb3, o, 64);
     lsum += __shfl_xor(lsum, o, 64);
   }
-  if (l == 0) {
-    atomicAdd(grad + OFF_B3, gb3);
-    atomicAdd(loss, lsum);
+  // waves 0 and 1 write their sums, waves 2 and 3 add to them; C layout: row =
+  // 4*(l/16)+i within block mb, col = l%16 within nb
+  auto flush = [&](float *dst, auto put) {
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = mb * 16 + 4 * (l / 16) + i;
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) put(dst[OFF_W2 + j * H + nb * 16 + l % 16], gW2[mb][nb][i]);
+        if (l % 16 < FLK_MLP_NFEAT) put(dst[OFF_W1 + j * FLK_MLP_NFEAT + l % 16], gW1[mb][i]);
+      }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+      if (l < 16) {
+        put(dst[OFF_B2 + nb * 16 + l], gb2[nb]);
+        put(dst[OFF_W3 + nb * 16 + l], gw3[nb]);
+        put(dst[OFF_B1 + nb * 16 + l], gb1v[nb]);
+      }
+    if (l == 0) {
+      put(dst[OFF_B3], gb3);
+      put(dst[FLK_MLP_NPARAM], lsum);
+    }
+  };
+  __syncthreads();
+  if (w < 2) flush(lds.sums[w], [](float &d, float v) { d = v; });
+  __syncthreads();
+  if (w >= 2) flush(lds.sums[w - 2], [](float &d, float v) { d += v; });
+  __syncthreads();
+  for (int k = threadIdx.x; k < kSums; k += 256)
+    part[(int64_t)blockIdx.x * kSums + k] = lds.sums[0][k] + lds.sums[1][k];
+}
+
+// The blocks' sums added, 64 parameters a block, a quarter of the sums a wave;
+// then either the gradient itself (grad) or an Adam step (FP32 masters; m, v
+// moments, zero before the first step; bias-corrected).  The squared error goes
+// to, or with `more` is added to, *loss.
+constexpr int kStepBlocks = (kSums + 63) / 64;
+__global__ __launch_bounds__(256) void mlp_step_kernel(const float *__restrict__ part, int nparts,
+                                                       float *__restrict__ grad, float *__restrict__ P,
+                                                       float *__restrict__ m, float *__restrict__ v, int first,
+                                                       float lr, float b1t, float b2t, float *__restrict__ loss,
+                                                       int more) {
+  __shared__ float sums[4][64];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, t = blockIdx.x * 64 + l;
+  float s = 0.f;
+  if (t < kSums) {
+    const float *p = part + t;
+    int k = w;
+    for (; k + 28 < nparts; k += 32) {  // eight loads in flight
+      float u[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) u[i] = p[(int64_t)(k + 4 * i) * kSums];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += u[i];
+    }
+    for (; k < nparts; k += 4) s += p[(int64_t)k * kSums];
   }
-}
-
-__global__ void zero_kernel(float *p, int n) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0.f;
-}
-
-// Adam (FP32 masters): m, v moments, bias-corrected step.
-__global__ void adam_kernel(float *__restrict__ P, const float *__restrict__ g, float *__restrict__ m,
-                            float *__restrict__ v, int n, float lr, float b1t, float b2t) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float b1 = 0.9f, b2 = 0.999f;
-  m[t] = b1 * m[t] + (1 - b1) * g[t];
-  v[t] = b2 * v[t] + (1 - b2) * g[t] * g[t];
-  const float mh = m[t] / (1 - b1t), vh = v[t] / (1 - b2t);
-  P[t] -= lr * mh / (sqrtf(vh) + 1e-8f);
+  sums[w][l] = s;
+  __syncthreads();
+  if (w || t >= kSums) return;
+  const float g = (sums[0][l] + sums[1][l]) + (sums[2][l] + sums[3][l]);
+  if (t == FLK_MLP_NPARAM) {
+    *loss = more ? *loss + g : g;
+  } else if (grad) {
+    grad[t] = g;
+  } else {
+    const float b1 = 0.9f, b2 = 0.999f;
+    const float mt = (first ? 0.f : b1 * m[t]) + (1 - b1) * g, vt = (first ? 0.f : b2 * v[t]) + (1 - b2) * g * g;
+    m[t] = mt;
+    v[t] = vt;
+    const float mh = mt / (1 - b1t), vh = vt / (1 - b2t);
+    P[t] -= lr * mh / (sqrtf(vh) + 1e-8f);
+  }
 }
 
 // The level kernel's LDS image of the network, one wave.
@@ -407,30 +485,54 @@ void mlp_forward_device(flk_ctx *ctx, const float *dx, int64_t n, float *dy) {
   FLK_HIP(hipGetLastError());
 }
 
+namespace {
+
+// Sets of more than this are given back after the call: their upload takes
+// many times what allocating them does.
+constexpr size_t kKeptBytes = size_t(64) << 20;
+void give_back(MlpScratch &D) {
+  for (DevBuf *b : {&D.x, &D.t, &D.idx})
+    if (b->bytes > kKeptBytes) b->release();
+}
+
+// One set of gradients of the n rows at idx (or the first n): the blocks' sums
+// into D.part; returns their number.  More blocks than are resident would add
+// sets to read without adding waves.
+int enqueue_gradient(flk_ctx *ctx, const float *x, const float *t, const int64_t *idx, int64_t n) {
+  MlpScratch &D = ctx->mlp.scratch;
+  const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((n + 63) / 64, 2 * std::max(1, ctx->num_cus)));
+  D.part.reserve(sizeof(float) * kSums * blocks);
+  hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, ctx->stream, ctx->mlp.d_params.as<float>(),
+                     ctx->mlp.d_norm.as<float>(), x, t, idx, n, 1.0f / (float)std::max<int64_t>(n, 1),
+                     D.part.as<float>());
+  FLK_HIP(hipGetLastError());
+  return blocks;
+}
+
+}  // namespace
+
 float mlp_gradient(flk_ctx *ctx, const float *x, const float *y, int64_t n, float *grad) {
   mlp_upload(ctx);
   hipStream_t s = ctx->stream;
-  DevBuf dx, dt, dg, dl;
-  dx.reserve(sizeof(float) * FLK_MLP_NFEAT * std::max<int64_t>(n, 1));
-  dt.reserve(sizeof(float) * std::max<int64_t>(n, 1));
-  dg.reserve(sizeof(float) * FLK_MLP_NPARAM);
-  dl.reserve(sizeof(float));
+  MlpScratch &D = ctx->mlp.scratch;
+  D.x.reserve(sizeof(float) * FLK_MLP_NFEAT * std::max<int64_t>(n, 1));
+  D.t.reserve(sizeof(float) * std::max<int64_t>(n, 1));
+  D.m.reserve(sizeof(float) * FLK_MLP_NPARAM);
+  D.loss.reserve(sizeof(float));
   if (n) {
-    FLK_HIP(hipMemcpyAsync(dx.ptr, x, sizeof(float) * FLK_MLP_NFEAT * n, hipMemcpyHostToDevice, s));
-    FLK_HIP(hipMemcpyAsync(dt.ptr, y, sizeof(float) * n, hipMemcpyHostToDevice, s));
+    FLK_HIP(hipMemcpyAsync(D.x.ptr, x, sizeof(float) * FLK_MLP_NFEAT * n, hipMemcpyHostToDevice, s));
+    FLK_HIP(hipMemcpyAsync(D.t.ptr, y, sizeof(float) * n, hipMemcpyHostToDevice, s));
   }
-  hipLaunchKernelGGL(zero_kernel, dim3((FLK_MLP_NPARAM + 255) / 256), dim3(256), 0, s, dg.as<float>(),
-                     FLK_MLP_NPARAM);
-  hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, dl.as<float>(), 1);
-  const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((n + 63) / 64, 8 * std::max(1, ctx->num_cus)));
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, s, ctx->mlp.d_params.as<float>(),
-                     ctx->mlp.d_norm.as<float>(), dx.as<float>(), dt.as<float>(), nullptr, n,
-                     1.0f / (float)std::max<int64_t>(n, 1), dg.as<float>(), dl.as<float>());
+  const int parts = enqueue_gradient(ctx, D.x.as<float>(), D.t.as<float>(), nullptr, n);
+  hipLaunchKernelGGL(mlp_step_kernel, dim3(kStepBlocks), dim3(256), 0, s, (const float *)D.part.as<float>(), parts,
+                     D.m.as<float>(), (float *)nullptr, (float *)nullptr, (float *)nullptr, 0, 0.f, 0.f, 0.f,
+                     D.loss.as<float>(), 0);
   FLK_HIP(hipGetLastError());
   float loss = 0;
-  FLK_HIP(hipMemcpyAsync(grad, dg.ptr, sizeof(float) * FLK_MLP_NPARAM, hipMemcpyDeviceToHost, s));
-  FLK_HIP(hipMemcpyAsync(&loss, dl.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
+  FLK_HIP(hipMemcpyAsync(grad, D.m.ptr, sizeof(float) * FLK_MLP_NPARAM, hipMemcpyDeviceToHost, s));
+  FLK_HIP(hipMemcpyAsync(&loss, D.loss.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
   FLK_HIP(hipStreamSynchronize(s));
+  give_back(D);
   return loss / (float)std::max<int64_t>(n, 1);
 }
 
@@ -439,48 +541,40 @@ float mlp_train(flk_ctx *ctx, const float *x, const float *y, int64_t n, int epo
   if (n <= 0 || epochs <= 0 || batch <= 0) throw Error(FLK_ERR_ARG, "empty training set");
   mlp_upload(ctx);
   hipStream_t s = ctx->stream;
-  DevBuf dx, dt, dg, dl, dm, dv, didx;
-  dx.reserve(sizeof(float) * FLK_MLP_NFEAT * n);
-  dt.reserve(sizeof(float) * n);
-  dg.reserve(sizeof(float) * FLK_MLP_NPARAM);
-  dm.reserve(sizeof(float) * FLK_MLP_NPARAM);
-  dv.reserve(sizeof(float) * FLK_MLP_NPARAM);
-  dl.reserve(sizeof(float));
-  didx.reserve(sizeof(int64_t) * n);
-  FLK_HIP(hipMemcpyAsync(dx.ptr, x, sizeof(float) * FLK_MLP_NFEAT * n, hipMemcpyHostToDevice, s));
-  FLK_HIP(hipMemcpyAsync(dt.ptr, y, sizeof(float) * n, hipMemcpyHostToDevice, s));
-  const unsigned zb = (FLK_MLP_NPARAM + 255) / 256;
-  hipLaunchKernelGGL(zero_kernel, dim3(zb), dim3(256), 0, s, dm.as<float>(), FLK_MLP_NPARAM);
-  hipLaunchKernelGGL(zero_kernel, dim3(zb), dim3(256), 0, s, dv.as<float>(), FLK_MLP_NPARAM);
+  MlpScratch &D = ctx->mlp.scratch;
+  D.x.reserve(sizeof(float) * FLK_MLP_NFEAT * n);
+  D.t.reserve(sizeof(float) * n);
+  D.m.reserve(sizeof(float) * FLK_MLP_NPARAM);
+  D.v.reserve(sizeof(float) * FLK_MLP_NPARAM);
+  D.loss.reserve(sizeof(float));
+  D.idx.reserve(sizeof(int64_t) * n);
+  FLK_HIP(hipMemcpyAsync(D.x.ptr, x, sizeof(float) * FLK_MLP_NFEAT * n, hipMemcpyHostToDevice, s));
+  FLK_HIP(hipMemcpyAsync(D.t.ptr, y, sizeof(float) * n, hipMemcpyHostToDevice, s));
   std::vector<int64_t> perm(n);
   for (int64_t k = 0; k < n; ++k) perm[k] = k;
   std::mt19937_64 rng(seed);
   float b1t = 1.f, b2t = 1.f, last = 0.f;
-  const int blocks_max = 4 * std::max(1, ctx->num_cus);
   for (int e = 0; e < epochs; ++e) {
     for (int64_t k = n - 1; k > 0; --k) std::swap(perm[k], perm[rng() % (uint64_t)(k + 1)]);
-    FLK_HIP(hipMemcpyAsync(didx.ptr, perm.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, s, dl.as<float>(), 1);
+    FLK_HIP(hipMemcpyAsync(D.idx.ptr, perm.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice, s));
     for (int64_t b0 = 0; b0 < n; b0 += batch) {
-      const int64_t nb = std::min<int64_t>(batch, n - b0);
-      hipLaunchKernelGGL(zero_kernel, dim3(zb), dim3(256), 0, s, dg.as<float>(), FLK_MLP_NPARAM);
-      const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((nb + 63) / 64, blocks_max));
-      hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, s, ctx->mlp.d_params.as<float>(),
-                         ctx->mlp.d_norm.as<float>(), dx.as<float>(), dt.as<float>(),
-                         didx.as<int64_t>() + b0, nb, 1.0f / (float)nb, dg.as<float>(), dl.as<float>());
+      const int parts = enqueue_gradient(ctx, D.x.as<float>(), D.t.as<float>(), D.idx.as<int64_t>() + b0,
+                                         std::min<int64_t>(batch, n - b0));
       b1t *= 0.9f;
       b2t *= 0.999f;
-      hipLaunchKernelGGL(adam_kernel, dim3(zb), dim3(256), 0, s, ctx->mlp.d_params.as<float>(),
-                         dg.as<float>(), dm.as<float>(), dv.as<float>(), FLK_MLP_NPARAM, lr, b1t, b2t);
+      hipLaunchKernelGGL(mlp_step_kernel, dim3(kStepBlocks), dim3(256), 0, s, (const float *)D.part.as<float>(),
+                         parts, (float *)nullptr, ctx->mlp.d_params.as<float>(), D.m.as<float>(), D.v.as<float>(),
+                         (int)(e == 0 && b0 == 0), lr, b1t, b2t, D.loss.as<float>(), (int)(b0 > 0));
+      FLK_HIP(hipGetLastError());
     }
-    FLK_HIP(hipGetLastError());
-    FLK_HIP(hipMemcpyAsync(&last, dl.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
+    FLK_HIP(hipMemcpyAsync(&last, D.loss.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
     FLK_HIP(hipStreamSynchronize(s));
     last /= (float)n;
   }
   FLK_HIP(hipMemcpyAsync(ctx->mlp.params.data(), ctx->mlp.d_params.ptr, sizeof(float) * FLK_MLP_NPARAM,
                          hipMemcpyDeviceToHost, s));
   FLK_HIP(hipStreamSynchronize(s));
+  give_back(D);
   return last;
 }
 

@@ -83,6 +83,19 @@ __device__ __forceinline__ uint64_t spread16(uint64_t v) {
 // VP: the FP64 coordinates (double4), or, when every stored coordinate is
 // exact in FP32, their FP32 copies (float4, half the bytes, the same values).
 template <typename VP>
+__device__ __forceinline__ uint32_t segment_key(const VP &p, const VP &q, const double *__restrict__ cb) {
+  const double m[3] = {0.5 * ((double)p.x + (double)q.x), 0.5 * ((double)p.y + (double)q.y),
+                       0.5 * ((double)p.z + (double)q.z)};
+  uint32_t code = 0;
+  for (int d = 0; d < 3; ++d) {
+    const double u = (m[d] - cb[d]) * cb[3 + d];
+    const uint64_t qd = (uint64_t)fmin(fmax(u, 0.0), 1023.0);
+    code |= (uint32_t)(spread16(qd) << (2 - d));
+  }
+  return code;
+}
+
+template <typename VP>
 __global__ __launch_bounds__(256) void bh_keys(const VP *__restrict__ pts, const int64_t *__restrict__ seg_off,
                                                const int64_t *__restrict__ vtx_off, const double *__restrict__ cbox,
                                                const RadixTile *__restrict__ tiles,
@@ -91,21 +104,10 @@ __global__ __launch_bounds__(256) void bh_keys(const VP *__restrict__ pts, const
   const RadixTile tl = tiles[blockIdx.x];
   const int c = tcurve[blockIdx.x];
   const int64_t v0 = vtx_off[c] - seg_off[c];
-  const double lo[3] = {cbox[6 * c], cbox[6 * c + 1], cbox[6 * c + 2]};
-  const double sc[3] = {cbox[6 * c + 3], cbox[6 * c + 4], cbox[6 * c + 5]};
   for (int o = threadIdx.x; o < tl.count; o += 256) {
     const int64_t g = (int64_t)tl.start + o;
     const int64_t v = v0 + g;
-    const VP p = pts[v], q = pts[v + 1];
-    const double m[3] = {0.5 * ((double)p.x + (double)q.x), 0.5 * ((double)p.y + (double)q.y),
-                         0.5 * ((double)p.z + (double)q.z)};
-    uint32_t code = 0;
-    for (int d = 0; d < 3; ++d) {
-      const double u = (m[d] - lo[d]) * sc[d];
-      const uint64_t qd = (uint64_t)fmin(fmax(u, 0.0), 1023.0);
-      code |= (uint32_t)(spread16(qd) << (2 - d));
-    }
-    keys[g] = code;
+    keys[g] = segment_key(pts[v], pts[v + 1], cbox + 6 * c);
     vals[g] = (uint32_t)v;
   }
 }
@@ -248,16 +250,103 @@ __device__ __forceinline__ double2 mk2(double2, double x, double y) { return mak
 __device__ __forceinline__ float2 mk2(float2, double x, double y) { return make_float2((float)x, (float)y); }
 
 template <typename SP, typename VP>
+__device__ __forceinline__ void stage_segment(const VP &a, const VP &b, SP *__restrict__ sp) {
+  sp[0] = mk2(SP{}, a.x, a.y);
+  sp[1] = mk2(SP{}, a.z, b.x);
+  sp[2] = mk2(SP{}, b.y, b.z);
+}
+
+template <typename SP, typename VP>
 __global__ __launch_bounds__(256) void bh_stage_segments(const uint32_t *__restrict__ order,
                                                          const VP *__restrict__ pts, int64_t nseg,
                                                          SP *__restrict__ sp) {
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nseg) return;
   const uint32_t v = order[s];
-  const VP a = pts[v], b = pts[v + 1];
-  sp[3 * s] = mk2(SP{}, a.x, a.y);
-  sp[3 * s + 1] = mk2(SP{}, a.z, b.x);
-  sp[3 * s + 2] = mk2(SP{}, b.y, b.z);
+  stage_segment(pts[v], pts[v + 1], sp + 3 * s);
+}
+
+// Keys, sort and (sp not null) staged end points of a curve of at most CAP
+// segments in one block, list[b] its rank: the same order as the segmented
+// sort's.  Key and place make one number, so every two differ: each wave sorts
+// runs of 64 across its lanes, and runs are merged by each element finding its
+// place in the other run, a thread's E elements side by side.  Bound by latency,
+// as the segmented sort's 14-18 launches are, which took 110 us for ten curves of
+// 24,000 segments and 165 for 400 of 4e5: 42 and 41 here, sorted within 64 bits
+// of LDS a segment.  8,192 is what 64 KB hold, two blocks a CU.
+constexpr int kSmallSorts = 3;
+constexpr int kSmallSort[kSmallSorts] = {1024, 4096, 8192}, kSmallThreads[kSmallSorts] = {256, 1024, 1024};
+template <typename SP, typename VP, int THREADS, int CAP>
+__global__ __launch_bounds__(THREADS) void bh_sort_small(const VP *__restrict__ pts,
+                                                         const int64_t *__restrict__ seg_off,
+                                                         const int64_t *__restrict__ vtx_off,
+                                                         const double *__restrict__ cbox,
+                                                         const int32_t *__restrict__ list,
+                                                         uint32_t *__restrict__ order, SP *__restrict__ sp) {
+  constexpr int E = CAP / THREADS;
+  constexpr int kPlaceBits = 13;
+  static_assert(CAP <= 1 << kPlaceBits && THREADS % 64 == 0, "places fit, whole waves");
+  __shared__ uint64_t a[CAP];
+  const int c = list[blockIdx.x], lane = threadIdx.x & 63;
+  const int64_t g0 = seg_off[c], v0 = vtx_off[c];
+  const int n = (int)(seg_off[c + 1] - g0), padded = (n + 63) / 64 * 64;
+  const int sets = max(0, (n - ((int)threadIdx.x - lane) + THREADS - 1) / THREADS);  // of 64, this wave's
+  uint64_t x[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = e * THREADS + (int)threadIdx.x;
+    x[e] = 1ull << (30 + kPlaceBits) | (uint64_t)i;  // behind every segment
+    if (i < n) x[e] = (uint64_t)segment_key(pts[v0 + i], pts[v0 + i + 1], cbox + 6 * c) << kPlaceBits | (uint64_t)i;
+  }
+#pragma unroll
+  for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+    for (int d = k / 2; d > 0; d >>= 1) {
+      const bool low = ((lane & d) == 0) == ((lane & k) == 0);  // keeps the smaller
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        if (e >= sets) break;
+        const uint64_t y = __shfl_xor(x[e], d, 64);
+        x[e] = (x[e] < y) == low ? x[e] : y;
+      }
+    }
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e < sets) a[e * THREADS + (int)threadIdx.x] = x[e];
+  for (int run = 64; run < n; run *= 2) {
+    __syncthreads();
+    int start[E], len[E], to[E];  // the other run, and how many of it are smaller
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = e * THREADS + (int)threadIdx.x;
+      const int other = min((i & ~(run - 1)) ^ run, padded);
+      start[e] = other;
+      len[e] = min(padded - other, run);
+      to[e] = 0;
+      if (e < sets) x[e] = a[i];
+    }
+    for (int h = run; h > 0; h >>= 1)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        if (e >= sets) break;
+        if (to[e] + h <= len[e] && a[start[e] + to[e] + h - 1] < x[e]) to[e] += h;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = e * THREADS + (int)threadIdx.x;
+      if (e < sets) a[(i & ~(2 * run - 1)) + (i & (run - 1)) + to[e]] = x[e];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = e * THREADS + (int)threadIdx.x;
+    if (i >= n) continue;
+    const int64_t v = v0 + (int64_t)(a[i] & ((1u << kPlaceBits) - 1));
+    order[g0 + i] = (uint32_t)v;
+    if (sp) stage_segment(pts[v], pts[v + 1], sp + 3 * (g0 + i));
+  }
 }
 
 template <typename SP>
@@ -495,8 +584,7 @@ __global__ __launch_bounds__(256) void bh_moments_direct(const BhRange *__restri
 // FP64 moments of a node above `direct` segments from its two children.
 template <typename SP>
 __device__ void node_moments(BhRange rr, int2 ch, int32_t direct, const BhRange *__restrict__ range,
-                             const SP *__restrict__ sp, const Mom64 *__restrict__ m64,
-                             const BhMom *__restrict__ mom, Mom64 &M) {
+                             const SP *__restrict__ sp, const Mom64 *m64, const BhMom *mom, Mom64 &M) {
   for (int t = 0; t < 3; ++t) M.c[t] = 0;
   for (int t = 0; t < 9; ++t) M.D[t] = 0;
   for (int t = 0; t < 18; ++t) M.Q[t] = 0;
@@ -550,17 +638,11 @@ __device__ void node_moments(BhRange rr, int2 ch, int32_t direct, const BhRange 
 // `direct` segments write FP64 records, so the bottom levels never round-trip
 // them through memory.  Children are read one at a time.
 template <typename SP>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3))) void bh_moments(const BhRange *__restrict__ range, int32_t n,
-                                                  int32_t base, int32_t direct,
-                                                  const int2 *__restrict__ child,
-                                                  const SP *__restrict__ sp,
-                                                  Mom64 *__restrict__ m64, BhGeo *__restrict__ geo,
-                                                  BhMom *__restrict__ mom) {
-  __shared__ float4 stage[2][18 * 16];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int k0 = blockIdx.x * blockDim.x + w * 64;  // this wave's first node past base
-  if (k0 >= n) return;                                // whole wave: no LDS exchange to join
-  const int k = k0 + lane, nw = min(64, n - k0);
+__device__ __forceinline__ void moments_wave(const BhRange *__restrict__ range, int32_t k0, int32_t n, int32_t base,
+                                             int32_t direct, const int2 *__restrict__ child,
+                                             const SP *__restrict__ sp, Mom64 *m64, BhGeo *geo, BhMom *mom,
+                                             float4 *stage) {
+  const int k = k0 + (threadIdx.x & 63), nw = min(64, n - k0);
   BhGeo gr;
   BhMom m;
   Mom64 M;
@@ -577,10 +659,41 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3))) void b
       node_records(M, ch, rr, gr, m);
     }
   }
-  wave_store_m64(M, __ballot(fp64), m64 + base + k0, nw, stage[w]);
-  wave_store_records(gr, m, geo + base + k0, mom + base + k0, nw, stage[w]);
+  wave_store_m64(M, __ballot(fp64), m64 + base + k0, nw, stage);
+  wave_store_records(gr, m, geo + base + k0, mom + base + k0, nw, stage);
 }
 
+template <typename SP>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3))) void bh_moments(
+    const BhRange *__restrict__ range, int32_t n, int32_t base, int32_t direct, const int2 *__restrict__ child,
+    const SP *__restrict__ sp, Mom64 *__restrict__ m64, BhGeo *__restrict__ geo, BhMom *__restrict__ mom) {
+  __shared__ float4 stage[2][18 * 16];
+  const int w = threadIdx.x >> 6;
+  const int k0 = blockIdx.x * blockDim.x + w * 64;  // this wave's first node past base
+  if (k0 >= n) return;                                // whole wave: no LDS exchange to join
+  moments_wave(range, k0, n, base, direct, child, sp, m64, geo, mom, stage[w]);
+}
+
+// The top levels, `top` to 0, in one launch: a block takes a curve's levels of at
+// most 128 nodes one after the other, its own stores read back after a barrier.
+// A launch each they took 5-17 us a level, most of it latency and the launch:
+// 400 curves of 4e5 segments 115 -> 63 us, 1,000 of 3.1e7 141 -> 114.
+constexpr int kTopLevels = 8;
+template <typename SP>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3))) void bh_moments_top(
+    const BhRange *__restrict__ range, int32_t nc, BhLevels L, const int32_t *__restrict__ loff, int32_t top,
+    int32_t direct, const int2 *__restrict__ child, const SP *__restrict__ sp, Mom64 *m64, BhGeo *geo, BhMom *mom) {
+  static_assert(1 << (kTopLevels - 1) <= 128, "a level's nodes fit the block");
+  __shared__ float4 stage[2][18 * 16];
+  const int w = threadIdx.x >> 6, c = blockIdx.x;
+  for (int lev = top; lev >= 0; --lev) {
+    const int32_t *row = loff + (int64_t)lev * nc;
+    const int32_t first = row[c], n = (c + 1 < nc ? row[c + 1] : L.base[lev + 1] - L.base[lev]) - first;
+    if (64 * w < n)
+      moments_wave(range, 64 * w, n, L.base[lev] + first, direct, child, sp, m64, geo, mom, stage[w]);
+    __syncthreads();
+  }
+}
 
 // ---------------------------------------------------------------- far field
 struct F3 {
@@ -1645,6 +1758,7 @@ struct ForestPlan {
   std::vector<double> cbox;
   std::vector<RadixTile> tiles;  // the segmented sort's tiles (one curve each)
   std::vector<int32_t> tcurve;   // each tile's curve rank
+  std::vector<int32_t> small[kSmallSorts];  // ranks of the curves that one block sorts (see kSmallSort)
   int64_t S = 0;
   std::vector<int32_t> level_base, level_n;
   std::vector<int64_t> level_split, level_max;
@@ -1654,7 +1768,7 @@ struct ForestPlan {
   const int64_t *d_seg = nullptr, *d_vtx = nullptr;
   const double *d_box = nullptr;
   const RadixTile *d_tiles = nullptr;
-  const int32_t *d_tcurve = nullptr;
+  const int32_t *d_tcurve = nullptr, *d_small[kSmallSorts] = {};
 };
 
 // Host arrays of the plans on their way to the device: gathered in one pinned
@@ -1694,6 +1808,7 @@ void add_forest(PlanUpload &up, ForestPlan &P) {
   up.add(P.cbox, P.d_box);
   up.add(P.tiles, P.d_tiles);
   up.add(P.tcurve, P.d_tcurve);
+  for (int k = 0; k < kSmallSorts; ++k) up.add(P.small[k], P.d_small[k]);
 }
 
 // The planned curves' key boxes, the one part of a plan that their coordinates
@@ -1732,10 +1847,23 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   plan_boxes(cv, P);
   const int64_t S = P.S = P.seg_off[nc];
   if (S >= INT32_MAX / 2) throw Error(FLK_ERR_ARG, "too many Barnes-Hut segments");
-  const int64_t ntiles = segmented_tiles(P.seg_off.data(), nc, P.tiles);
+  for (int32_t k = 0; k < nc; ++k) {
+    const int64_t n = P.seg_off[k + 1] - P.seg_off[k];
+    int cls = 0;
+    while (cls < kSmallSorts && n > kSmallSort[cls]) ++cls;
+    if (cls < kSmallSorts) P.small[cls].push_back(k);
+  }
+  // the shortest join the next class's launch where both are resident at once
+  if (!P.small[1].empty() && P.small[0].size() + P.small[1].size() <= 2 * (size_t)std::max(1, ctx->num_cus)) {
+    P.small[1].insert(P.small[1].end(), P.small[0].begin(), P.small[0].end());
+    P.small[0].clear();
+  }
+  const int64_t ntiles = segmented_tiles(P.seg_off.data(), nc, kSmallSort[kSmallSorts - 1], P.tiles);
   P.tcurve.resize(ntiles);
-  for (int32_t k = 0, t = 0; k < nc; ++k)
-    for (; t < ntiles && P.tiles[t].start < P.seg_off[k + 1]; ++t) P.tcurve[t] = k;
+  for (int32_t k = 0, t = 0; t < ntiles; ++t) {
+    while (P.seg_off[k + 1] <= P.tiles[t].start) ++k;
+    P.tcurve[t] = k;
+  }
   // Splits per level from the segment counts alone: a range of m > leaf
   // segments splits into floor(m/2) and m - floor(m/2), so every level of a
   // curve's tree holds at most two distinct range sizes (m and m + 1).  With
@@ -1804,22 +1932,39 @@ void plan_forest(flk_ctx *ctx, const std::vector<int32_t> &curves_in, int leaf, 
   B.mom.reserve(sizeof(BhMom) * total);
 }
 
-// The end-point gather, the nodes' ranges and children and the moments of a
-// planned forest, with the segments' end points staged as SP.
+// Every curve's segments in the order of their keys, and the end points staged
+// in it.  Curves within kSmallSort are sorted by a block each, the others by the
+// segmented sort.
+template <typename SP, typename VP>
+void enqueue_sort(flk_ctx *ctx, const ForestPlan &P, const VP *pts, SP *sp, hipStream_t s) {
+  BhScratch &B = ctx->bh;
+  const int64_t ntiles = (int64_t)P.tiles.size();
+  const auto sort = [&](auto kernel, int k) {
+    if (!P.small[k].empty())
+      hipLaunchKernelGGL(kernel, dim3((unsigned)P.small[k].size()), dim3(kSmallThreads[k]), 0, s, pts, P.d_seg,
+                         P.d_vtx, P.d_box, P.d_small[k], B.order.as<uint32_t>(), ntiles ? (SP *)nullptr : sp);
+  };
+  sort(bh_sort_small<SP, VP, kSmallThreads[0], kSmallSort[0]>, 0);
+  sort(bh_sort_small<SP, VP, kSmallThreads[1], kSmallSort[1]>, 1);
+  sort(bh_sort_small<SP, VP, kSmallThreads[2], kSmallSort[2]>, 2);
+  FLK_HIP(hipGetLastError());
+  if (ntiles == 0) return;
+  hipLaunchKernelGGL(bh_keys<VP>, dim3((unsigned)ntiles), dim3(256), 0, s, pts, P.d_seg, P.d_vtx, P.d_box, P.d_tiles,
+                     P.d_tcurve, B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
+  FLK_HIP(hipGetLastError());
+  radix_sort_pairs<uint32_t>(B.keys0.as<uint32_t>(), B.keys1.as<uint32_t>(), B.ids0.as<uint32_t>(),
+                             B.vals.as<uint32_t>(), B.order.as<uint32_t>(), P.S, 30, B.tmp.ptr, s, P.d_tiles, ntiles);
+  hipLaunchKernelGGL((bh_stage_segments<SP, VP>), dim3((unsigned)((P.S + 255) / 256)), dim3(256), 0, s,
+                     B.order.as<uint32_t>(), pts, P.S, sp);
+  FLK_HIP(hipGetLastError());
+}
+
+// The nodes' ranges and children and the moments of a planned forest, with the
+// segments' end points staged as SP.
 template <typename SP>
 void enqueue_moments(flk_ctx *ctx, const ForestPlan &P, SP *sp, hipStream_t s) {
-  Curves &cv = ctx->curves;
   BhScratch &B = ctx->bh;
-  const int64_t S = P.S;
   const int32_t nc = (int32_t)P.cs.size();
-  // FP32 staging means every coordinate is exact in FP32: read the FP32 copies
-  if constexpr (std::is_same_v<SP, float2>)
-    hipLaunchKernelGGL((bh_stage_segments<SP, float4>), dim3((unsigned)((S + 255) / 256)), dim3(256), 0, s,
-                       B.order.as<uint32_t>(), cv.hi.as<float4>(), S, sp);
-  else
-    hipLaunchKernelGGL((bh_stage_segments<SP, double4>), dim3((unsigned)((S + 255) / 256)), dim3(256), 0, s,
-                       B.order.as<uint32_t>(), cv.dpts.as<double4>(), S, sp);
-  FLK_HIP(hipGetLastError());
   BhLevels L{};
   L.depth = (int32_t)P.level_base.size();
   int64_t units = nc;
@@ -1840,13 +1985,17 @@ void enqueue_moments(flk_ctx *ctx, const ForestPlan &P, SP *sp, hipStream_t s) {
                        B.mom.as<BhMom>());
     FLK_HIP(hipGetLastError());
   }
-  for (int lev = P.lev_top - 1; lev >= 0; --lev) {
+  for (int lev = P.lev_top - 1; lev >= kTopLevels; --lev) {
     const int32_t n = P.level_n[lev];
     hipLaunchKernelGGL(bh_moments<SP>, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, s, B.range.as<BhRange>(),
                        n, P.level_base[lev], P.direct, B.child.as<int2>(), (const SP *)sp, B.m64.as<Mom64>(),
                        B.geo.as<BhGeo>(), B.mom.as<BhMom>());
-    FLK_HIP(hipGetLastError());
   }
+  if (P.lev_top > 0)
+    hipLaunchKernelGGL(bh_moments_top<SP>, dim3((unsigned)nc), dim3(128), 0, s, B.range.as<BhRange>(), nc, L,
+                       B.loff.as<int32_t>(), std::min(P.lev_top, kTopLevels) - 1, P.direct, B.child.as<int2>(),
+                       (const SP *)sp, B.m64.as<Mom64>(), B.geo.as<BhGeo>(), B.mom.as<BhMom>());
+  FLK_HIP(hipGetLastError());
 }
 
 void enqueue_forest(flk_ctx *ctx, const ForestPlan &P, hipStream_t s) {
@@ -1854,20 +2003,13 @@ void enqueue_forest(flk_ctx *ctx, const ForestPlan &P, hipStream_t s) {
   if (nc == 0) return;
   Curves &cv = ctx->curves;
   BhScratch &B = ctx->bh;
-  const int64_t S = P.S;
-  const int64_t ntiles = (int64_t)P.tiles.size();
-  if (cv.inexact)
-    hipLaunchKernelGGL(bh_keys<double4>, dim3((unsigned)ntiles), dim3(256), 0, s, cv.dpts.as<double4>(),
-                       P.d_seg, P.d_vtx, P.d_box, P.d_tiles, P.d_tcurve, B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
-  else  // every coordinate exact in FP32: the FP32 copies, the same values
-    hipLaunchKernelGGL(bh_keys<float4>, dim3((unsigned)ntiles), dim3(256), 0, s, cv.hi.as<float4>(),
-                       P.d_seg, P.d_vtx, P.d_box, P.d_tiles, P.d_tcurve, B.keys0.as<uint32_t>(), B.ids0.as<uint32_t>());
-  FLK_HIP(hipGetLastError());
-  radix_sort_pairs<uint32_t>(B.keys0.as<uint32_t>(), B.keys1.as<uint32_t>(), B.ids0.as<uint32_t>(),
-                             B.vals.as<uint32_t>(), B.order.as<uint32_t>(), S, 30, B.tmp.ptr, s,
-                             P.d_tiles, ntiles);
-  if (cv.inexact) enqueue_moments(ctx, P, B.sp.as<double2>(), s);
-  else enqueue_moments(ctx, P, B.sp.as<float2>(), s);
+  if (cv.inexact) {
+    enqueue_sort(ctx, P, cv.dpts.as<double4>(), B.sp.as<double2>(), s);
+    enqueue_moments(ctx, P, B.sp.as<double2>(), s);
+  } else {  // every coordinate exact in FP32: the FP32 copies, the same values
+    enqueue_sort(ctx, P, cv.hi.as<float4>(), B.sp.as<float2>(), s);
+    enqueue_moments(ctx, P, B.sp.as<float2>(), s);
+  }
 }
 
 void forest_from_plan(flk_ctx *ctx, const ForestPlan &P, Forest &F) {

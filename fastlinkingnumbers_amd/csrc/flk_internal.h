@@ -406,11 +406,12 @@ void exclusive_scan(const int32_t *in, int32_t *out, int64_t n, int32_t *temp, h
 struct RadixTile {
   int32_t start, count;  // keys [start, start + count), count <= 4096
   int32_t cbase, stride; // digit d's count at cbase + d * stride
+  int32_t skipped;       // keys before `start` that are in no tile
 };
 size_t radix_temp_bytes(int64_t n, int64_t table_tiles = 0);
-// Tiles of the segments [seg_off[c], seg_off[c+1]) (host table); returns
-// their number.
-int64_t segmented_tiles(const int64_t *seg_off, int64_t nseg, std::vector<RadixTile> &table);
+// Tiles of the segments [seg_off[c], seg_off[c+1]) of more than `skip` keys
+// (host table); returns their number.
+int64_t segmented_tiles(const int64_t *seg_off, int64_t nseg, int64_t skip, std::vector<RadixTile> &table);
 template <typename K>
 void radix_sort_pairs(K *keys, K *keys_alt, uint32_t *vals, uint32_t *vals_alt, uint32_t *vals_out, int64_t n,
                       int end_bit, void *temp, hipStream_t s, const RadixTile *table = nullptr,

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void scan_tiles(const int32_t *in, int32_t 
 __device__ __forceinline__ RadixTile tile_of(const RadixTile *__restrict__ table, int64_t n, int64_t tiles) {
   if (table) return table[blockIdx.x];
   const int64_t start = (int64_t)blockIdx.x * kTile;
-  return RadixTile{(int32_t)start, (int32_t)min<int64_t>(kTile, n - start), (int32_t)blockIdx.x, (int32_t)tiles};
+  return RadixTile{(int32_t)start, (int32_t)min<int64_t>(kTile, n - start), (int32_t)blockIdx.x, (int32_t)tiles, 0};
 }
 
 // Digit histogram of one tile: per-wave LDS counters, summed into
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void radix_scatter(const K *__restrict__ ki
       run += c[k];
     }
     dstart[d] = start;
-    gbase[d] = offsets[(int64_t)tl.cbase + (int64_t)d * tl.stride];
+    gbase[d] = offsets[(int64_t)tl.cbase + (int64_t)d * tl.stride] + tl.skipped;
   }
   __syncthreads();
 #pragma unroll
@@ -324,15 +324,20 @@ size_t radix_temp_bytes(int64_t n, int64_t table_tiles) {
   return sizeof(int32_t) * (size_t)cells + scan_temp_bytes(cells);
 }
 
-int64_t segmented_tiles(const int64_t *seg_off, int64_t nseg, std::vector<RadixTile> &table) {
+int64_t segmented_tiles(const int64_t *seg_off, int64_t nseg, int64_t skip, std::vector<RadixTile> &table) {
   table.clear();
+  int64_t skipped = 0;
   for (int64_t c = 0; c < nseg; ++c) {
     const int64_t len = seg_off[c + 1] - seg_off[c];
+    if (len <= skip) {
+      skipped += len;
+      continue;
+    }
     const int64_t nt = (len + kTile - 1) / kTile;
     const int64_t first = (int64_t)table.size();
     for (int64_t j = 0; j < nt; ++j)
       table.push_back(RadixTile{(int32_t)(seg_off[c] + j * kTile), (int32_t)std::min<int64_t>(kTile, len - j * kTile),
-                                (int32_t)(256 * first + j), (int32_t)nt});
+                                (int32_t)(256 * first + j), (int32_t)nt, (int32_t)skipped});
   }
   return (int64_t)table.size();
 }

@@ -2462,7 +2462,7 @@ struct BatchPlan {
   std::vector<double> v, e;
   std::vector<uint32_t> f;
   std::vector<unsigned long long> counts;  // both passes' heads
-  // The read-back's end: pinned, in the device buffer's layout (v, e, counts, f).
+  // What bh_merge writes, pinned: v, e, counts, f.
   HostBuf res;
   size_t res_bytes() const { return 20 * idx.size() + 8 * counts.size(); }
   // the arrays' device addresses (PlanUpload)
@@ -2474,7 +2474,7 @@ struct BatchPlan {
     up.add(rb, d_rb);
     up.add(beta2, d_beta2);
   }
-  void collect() {  // pinned read-back into the vectors
+  void collect() {  // res into the vectors
     const double *hv = res.as<double>();
     std::copy(hv, hv + v.size(), v.begin());
     hv += v.size();
@@ -2520,16 +2520,15 @@ void plan_batch(flk_ctx *ctx, const int32_t *pairs, std::vector<int64_t> idx, co
   bp.e.assign(nb, 0.0);
   bp.f.assign(nb, 0u);
   bp.counts.assign(2 * kPassHead, 0ull);
-  B.out.reserve(bp.res_bytes());
   bp.res.reserve(bp.res_bytes());
 }
 
-// The batch's merge of both passes into per-pair results, and their read-back.
+// The batch's merge of both passes into per-pair results, in pinned memory.
 // cnt: the device-scheduled passes' counters, null for a host-driven batch.
 void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, unsigned long long *cnt, hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size();
-  double *v = B.out.as<double>(), *e = v + nb;
+  double *v = bp.res.as<double>(), *e = v + nb;
   auto *heads = reinterpret_cast<unsigned long long *>(e + nb);
   auto *f = reinterpret_cast<uint32_t *>(heads + bp.counts.size());
   hipLaunchKernelGGL(bh_merge, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, nb,
@@ -2538,7 +2537,6 @@ void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, unsigned 
                      prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, v, e, f, heads, cnt, bp.shape.cap,
                      bp.shape.D);
   FLK_HIP(hipGetLastError());
-  FLK_HIP(hipMemcpyAsync(bp.res.ptr, B.out.ptr, bp.res_bytes(), hipMemcpyDeviceToHost, s));
 }
 
 void enqueue_adapt(flk_ctx *ctx, const BatchPlan &bp, const flk_params &prm, unsigned long long *n_redo,

@@ -559,49 +559,7 @@ __global__ __launch_bounds__(256) void ds_pair_reduce(const double *__restrict__
   if (lane == 0) lk[p] = th * 0.15915494309189533576888376337251436 + (double)cr;
 }
 
-// Converts the uploaded FP64 vertices (already shifted and scaled) into the
-// FP32 hi/lo split and FP32 edge vectors; flags any vertex not exactly
-// representable in FP32.
-__global__ __launch_bounds__(256) void convert_vertices(const double4 *__restrict__ d, int64_t n,
-                                                        float4 *__restrict__ hi,
-                                                        float4 *__restrict__ lo,
-                                                        float4 *__restrict__ ed,
-                                                        int32_t *__restrict__ inexact) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool bad = false;
-  if (v < n) {
-    const double4 p = d[v];
-    const float hx = (float)p.x, hy = (float)p.y, hz = (float)p.z;
-    const float lx = (float)(p.x - (double)hx), ly = (float)(p.y - (double)hy),
-                lz = (float)(p.z - (double)hz);
-    hi[v] = make_float4(hx, hy, hz, 0.f);
-    lo[v] = make_float4(lx, ly, lz, 0.f);
-    bad = (lx != 0.f) || (ly != 0.f) || (lz != 0.f);
-    if (v + 1 < n) {
-      const double4 q = d[v + 1];
-      const double ex = q.x - p.x, ey = q.y - p.y, ez = q.z - p.z;
-      ed[v] = make_float4((float)ex, (float)ey, (float)ez, (float)(-0.5 * (ex * ex + ey * ey + ez * ez)));
-    } else {
-      ed[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  }
-  // One plain store for the blocks that read the flag clear (writers agree, and
-  // a stale read costs another store): an atomic for every wave serialises on
-  // its address, 180 us for the 8.8e5 vertices of a discretized knit.
-  if (__syncthreads_or(bad) && threadIdx.x == 0 &&
-      __hip_atomic_load(inexact, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
-    __hip_atomic_store(inexact, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 }  // namespace
-
-void convert_vertices_launch(hipStream_t s, const double4 *d, int64_t n, float4 *hi, float4 *lo,
-                             float4 *ed, int32_t *inexact) {
-  const int64_t blocks = (n + 255) / 256;
-  hipLaunchKernelGGL(convert_vertices, dim3((unsigned)blocks), dim3(256), 0, s, d, n, hi, lo, ed,
-                     inexact);
-  FLK_HIP(hipGetLastError());
-}
 
 // Rows per lane of the FP32 tile kernel, and rows per wave.
 constexpr int kRowsPerLane64 = 2;
@@ -731,8 +689,9 @@ DsBufs reserve_bufs(DevBuf &pairs, DevBuf &tasks, DevBuf &cost, DevBuf &theta, D
 }
 
 // Uploads of the plan arrays, the tile kernel (between ev_a and ev_b when
-// given) and, with `out`, the per-pair reduction and read-back: one stream-
-// ordered sequence, launched eagerly or captured into a graph.
+// given) and, with `out`, the per-pair reduction and read-back (or, without
+// d.out, the reduction straight into `out`, pinned memory): one stream-ordered
+// sequence, launched eagerly or captured into a graph.
 void ds_upload(const DsPair *dp, const DsTask *tasks, const int64_t *prefix, const int64_t *task0, int64_t npairs,
                int64_t ntasks, const DsBufs &d, hipStream_t s) {
   FLK_HIP(hipMemcpyAsync(d.pairs, dp, sizeof(DsPair) * npairs, hipMemcpyHostToDevice, s));
@@ -781,9 +740,9 @@ void ds_enqueue(flk_ctx *ctx, const DsPlan &P, const DsPair *dp, const DsTask *t
   if (out) {
     const int64_t rblocks = (npairs * 64 + 255) / 256;
     hipLaunchKernelGGL(ds_pair_reduce, dim3((unsigned)rblocks), dim3(256), 0, s, d.theta, d.corr, d.task0,
-                       npairs, d.out);
+                       npairs, d.out ? d.out : out);
     FLK_HIP(hipGetLastError());
-    FLK_HIP(hipMemcpyAsync(out, d.out, sizeof(double) * npairs, hipMemcpyDeviceToHost, s));
+    if (d.out) FLK_HIP(hipMemcpyAsync(out, d.out, sizeof(double) * npairs, hipMemcpyDeviceToHost, s));
   }
 }
 
@@ -831,8 +790,8 @@ float ds_graph_run(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64
     G.work = P.work;
     G.waves = P.blocks * 4;
     const int64_t nt = (int64_t)G.tasks.size();
-    const DsBufs d =
-        reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, G.d_out, npairs, nt);
+    DsBufs d = reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, G.d_out, npairs, nt);
+    d.out = nullptr;
     G.h_out.reserve(sizeof(double) * npairs);
     // the plan goes to the device once; the graph reads it there
     ds_upload(G.dp.data(), G.tasks.data(), G.prefix.data(), G.task0.data(), npairs, nt, d, s);
@@ -904,7 +863,7 @@ void ds_capture_enqueue(flk_ctx *ctx, DsGraph &G, hipStream_t s) {
   P.precise = G.precise;
   const int64_t nt = (int64_t)G.tasks.size();
   const DsBufs d = DsBufs{G.d_pairs.as<DsPair>(), G.d_tasks.as<DsTask>(), G.d_cost.as<int64_t>(),
-                          G.d_task0.as<int64_t>(), G.d_theta.as<double>(), G.d_out.as<double>(),
+                          G.d_task0.as<int64_t>(), G.d_theta.as<double>(), nullptr,
                           G.d_corr.as<int32_t>()};
   ds_enqueue(ctx, P, nullptr, nullptr, nullptr, nullptr, G.npairs, nt, d, s, nullptr, nullptr, G.h_out.as<double>());
 }

@@ -11,7 +11,6 @@
 #include "flk_internal.h"
 
 namespace flk {
-void stage_vertices_launch(flk_ctx *ctx);
 }
 
 using flk::Error;
@@ -56,7 +55,6 @@ int64_t curves_layout(flk_ctx *ctx, const int64_t *offsets, int32_t ncurves) {
   cv.nvert_dev = nv + ncurves;
   const int64_t nd = std::max<int64_t>(cv.nvert_dev, 1);
   cv.raw.reserve(sizeof(double) * 3 * std::max<int64_t>(nv, 1));
-  cv.d_off.reserve(sizeof(int64_t) * (ncurves + 1));
   cv.dpts.reserve(sizeof(double4) * nd);
   cv.hi.reserve(sizeof(float4) * nd);  // also the FP32 landing area of the upload
   cv.lo.reserve(sizeof(float4) * nd);
@@ -128,17 +126,7 @@ void curves_finish(flk_ctx *ctx) {
   const double ref = dmax > 0 ? 2.0 * dmax : span;
   cv.scale = ref > 0 ? std::ldexp(1.0, -(int)std::ceil(std::log2(ref))) : 1.0;
   if (!std::isfinite(cv.scale) || cv.scale == 0) cv.scale = 1.0;
-  if (cv.nvert_dev > 0) {
-    stage_vertices_launch(ctx);
-    ctx->d_count.reserve(sizeof(int32_t));
-    FLK_HIP(hipMemsetAsync(ctx->d_count.ptr, 0, sizeof(int32_t), s));
-    convert_vertices_launch(s, cv.dpts.as<double4>(), cv.nvert_dev, cv.hi.as<float4>(), cv.lo.as<float4>(),
-                            cv.ed.as<float4>(), ctx->d_count.as<int32_t>());
-    int32_t flag = 0;
-    FLK_HIP(hipMemcpyAsync(&flag, ctx->d_count.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    FLK_HIP(hipStreamSynchronize(s));
-    cv.inexact = flag != 0;
-  }
+  if (cv.nvert_dev > 0) cv.inexact = stage_vertices_run(ctx);
 }
 
 }  // namespace flk
@@ -247,7 +235,7 @@ void flk_destroy(flk_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   flk::DevBuf *bufs[] = {&ctx->curves.raw, &ctx->curves.dpts, &ctx->curves.hi, &ctx->curves.lo,
-                         &ctx->curves.ed, &ctx->curves.d_off, &ctx->d_pairs, &ctx->d_tasks,
+                         &ctx->curves.ed, &ctx->d_pairs, &ctx->d_tasks,
                          &ctx->d_cost, &ctx->d_task_theta, &ctx->d_task_corr,
                          &ctx->d_pair_task0, &ctx->d_pair_out, &ctx->d_pair_corr,
                          &ctx->d_boxes, &ctx->d_pls, &ctx->d_pls_boxes, &ctx->d_count, &ctx->d_misc,

@@ -173,7 +173,6 @@ struct Curves {
   DevBuf raw;                    // input FP64 AoS (no closing vertex)
   DevBuf dpts;                   // double4 per vertex, shifted+scaled, +1 closing vertex per curve
   DevBuf hi, lo, ed;             // float4 per vertex (+1 closing vertex per curve)
-  DevBuf d_off;                  // int64 device offsets (ncurves + 1)
   int64_t nvert_dev = 0;
   bool inexact = false;          // some stored coordinate needs the FP32 lo part
   int64_t bh_budget = 0;         // Barnes–Hut batch size in segments, fixed per curve set
@@ -197,7 +196,7 @@ struct BhScratch {
   // forest
   DevBuf geo, mom, order, m64, range, child, loff, vals, keys0, keys1, ids0, tmp, sp, pack;
   // traversal: root items of a pass, re-run list, per-pair sums and results
-  DevBuf roots_a, roots_b, beta2, cnt, leaves, pred, sum, err, items0, redo, out;
+  DevBuf roots_a, roots_b, beta2, cnt, leaves, pred, sum, err, items0, redo;
   std::vector<std::unique_ptr<DevBuf>> levels;
   HostBuf pack_host;                       // pinned: the plans' arrays on their way to `pack`
   unsigned long long *host_cnt = nullptr;  // pinned, 2 words per level of a traversal round trip
@@ -212,7 +211,7 @@ struct BhScratch {
   template <typename Fn> void each(Fn fn) {
     DevBuf *all[] = {&geo, &mom, &order, &m64, &range, &child, &loff, &vals, &keys0, &keys1, &ids0,
                      &tmp, &sp, &pack, &roots_a, &roots_b, &beta2, &cnt, &leaves, &pred,
-                     &sum, &err, &items0, &redo, &out};
+                     &sum, &err, &items0, &redo};
     for (DevBuf *b : all) fn(*b);
     for (auto &b : levels) fn(*b);
   }
@@ -358,6 +357,8 @@ struct flk_ctx {
   flk::DevBuf d_pairs, d_tasks, d_cost, d_task_theta, d_task_corr, d_pair_task0,
       d_pair_out, d_pair_corr, d_boxes, d_pls, d_pls_boxes, d_count, d_misc;
   flk::HostBuf pls_host;         // pinned: the potential-link search's total and pairs
+  flk::HostBuf curve_host;       // pinned: an upload's tables, its boxes and (inexact_host) its flag
+  int32_t *inexact_host = nullptr;
 };
 
 inline flk::GraphKey::GraphKey(const flk_ctx *ctx, const int32_t *p, int64_t npairs)
@@ -443,6 +444,9 @@ void tree_export(flk_ctx *ctx, int32_t curve, int32_t leaf, std::vector<flk_tree
 void pls_run(flk_ctx *ctx, const double *boxes, int32_t ncurves, std::vector<int32_t> &out);
 
 void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes);
+// Vertices, their FP32 forms and edges of the current curve set, after
+// curve_boxes_run; true when FP32 cannot hold some coordinate.
+bool stage_vertices_run(flk_ctx *ctx);
 
 // A new curve set: validates the offsets and sizes the device arrays; the
 // caller then fills curves.raw (input FP64 AoS) and calls curves_finish, which
@@ -465,8 +469,6 @@ void widen_launch(flk_ctx *ctx, const float *land, int64_t nval, double *dst);
 
 // Reads a BCC file into the context's curve set (see ingest.hip).
 void load_bcc(flk_ctx *ctx, const char *path, BccLoad &out);
-void convert_vertices_launch(hipStream_t s, const double4 *d, int64_t n, float4 *hi, float4 *lo,
-                             float4 *ed, int32_t *inexact);
 
 int64_t mlp_samples(flk_ctx *ctx, int32_t a, int32_t b, int64_t cap, uint64_t seed, float *x,
                     float *y);

@@ -39,13 +39,17 @@ __device__ __forceinline__ bool box_overlap(const Box6 &a, const Box6 &b) {
 // curve.cpp:331-343; an empty curve gets the empty box) in two passes: one
 // block per chunk of at most kBoxChunk vertices of one curve, then one thread
 // per curve folding its chunks, so a curve of millions of vertices is spread
-// over the whole chip.
+// over the whole chip; where every curve is one chunk the first pass is all.
+// The boxes also go to pinned memory (`host`) without a copy, and the last pass
+// clears the flag that stage_vertices sets.
 constexpr int64_t kBoxChunk = 16384;
 
 __global__ __launch_bounds__(256) void curve_box_chunks(const double *__restrict__ xyz,
                                                         const int64_t *__restrict__ chunk_v,
-                                                        double *__restrict__ part) {
+                                                        double *__restrict__ part, double *__restrict__ host,
+                                                        int32_t *__restrict__ inexact) {
   const int64_t c = blockIdx.x;
+  if (host && c == 0 && threadIdx.x == 0) *inexact = 0;
   const int64_t v0 = chunk_v[2 * c], v1 = chunk_v[2 * c + 1];
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
   for (int64_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
@@ -79,14 +83,20 @@ __global__ __launch_bounds__(256) void curve_box_chunks(const double *__restrict
       }
       part[6 * c + d] = lo;
       part[6 * c + 3 + d] = hi;
+      if (host) {
+        host[6 * c + d] = lo;
+        host[6 * c + 3 + d] = hi;
+      }
     }
   }
 }
 
 __global__ __launch_bounds__(256) void curve_box_merge(const double *__restrict__ part,
                                                        const int64_t *__restrict__ coff, int32_t ncurves,
-                                                       double *__restrict__ boxes) {
+                                                       double *__restrict__ boxes, double *__restrict__ host,
+                                                       int32_t *__restrict__ inexact) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c == 0) *inexact = 0;
   if (c >= ncurves) return;
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
   for (int64_t k = coff[c]; k < coff[c + 1]; ++k)
@@ -95,37 +105,65 @@ __global__ __launch_bounds__(256) void curve_box_merge(const double *__restrict_
       mx[d] = fmax(mx[d], part[6 * k + 3 + d]);
     }
   for (int d = 0; d < 3; ++d) {
-    boxes[6 * c + d] = mn[d];
-    boxes[6 * c + 3 + d] = mx[d];
+    boxes[6 * c + d] = host[6 * c + d] = mn[d];
+    boxes[6 * c + 3 + d] = host[6 * c + 3 + d] = mx[d];
   }
 }
 
 // Device vertex v (curve c, local index l <= n_c) takes input vertex l, or
 // vertex 0 for the closing copy l == n_c; coordinates are (x - origin) * scale.
+// Beside the FP64 vertex go its FP32 hi/lo split and the FP32 edge to the next
+// vertex of the array (the FP64 difference rounded, with -|edge|^2 / 2); any
+// vertex that FP32 cannot hold sets the flag.  One pass instead of a second over
+// the FP64 vertices: 3.1e7 vertices took 523 + 433 us in two.
 __global__ __launch_bounds__(256) void stage_vertices(const double *__restrict__ xyz,
                                                       const int64_t *__restrict__ in_off,
                                                       const int64_t *__restrict__ dev_off,
                                                       int32_t ncurves, int64_t ndev, double ox,
                                                       double oy, double oz, double scale,
-                                                      double4 *__restrict__ out) {
+                                                      double4 *__restrict__ out, float4 *__restrict__ hi,
+                                                      float4 *__restrict__ lo, float4 *__restrict__ ed,
+                                                      int32_t *__restrict__ inexact,
+                                                      int32_t *__restrict__ inexact_host) {
   const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= ndev) return;
-  int lo = 0, hi = ncurves;  // last c with dev_off[c] <= v
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (dev_off[mid] <= v) lo = mid;
-    else hi = mid;
+  bool bad = false;
+  if (v < ndev) {
+    int c = 0, end = ncurves;  // last c with dev_off[c] <= v
+    while (end - c > 1) {
+      const int mid = (c + end) >> 1;
+      if (dev_off[mid] <= v) c = mid;
+      else end = mid;
+    }
+    auto staged = [&](int k, int64_t l) {  // vertex l of curve k, (0, 0, 0) for an empty one
+      const int64_t first = in_off[k], n = in_off[k + 1] - first;
+      if (n == 0) return make_double4(0, 0, 0, 0);
+      const double *p = xyz + 3 * (first + (l < n ? l : 0));
+      return make_double4((p[0] - ox) * scale, (p[1] - oy) * scale, (p[2] - oz) * scale, 0.0);
+    };
+    const int64_t l = v - dev_off[c];
+    const double4 p = staged(c, l);
+    out[v] = p;
+    const float hx = (float)p.x, hy = (float)p.y, hz = (float)p.z;
+    const float lx = (float)(p.x - (double)hx), ly = (float)(p.y - (double)hy), lz = (float)(p.z - (double)hz);
+    hi[v] = make_float4(hx, hy, hz, 0.f);
+    lo[v] = make_float4(lx, ly, lz, 0.f);
+    bad = (lx != 0.f) || (ly != 0.f) || (lz != 0.f);
+    if (v + 1 < ndev) {
+      const double4 q = v + 1 < dev_off[c + 1] ? staged(c, l + 1) : staged(c + 1, 0);
+      const double ex = q.x - p.x, ey = q.y - p.y, ez = q.z - p.z;
+      ed[v] = make_float4((float)ex, (float)ey, (float)ez, (float)(-0.5 * (ex * ex + ey * ey + ez * ez)));
+    } else {
+      ed[v] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
   }
-  const int c = lo;
-  const int64_t l = v - dev_off[c];
-  const int64_t n = in_off[c + 1] - in_off[c];
-  if (n == 0) {
-    out[v] = make_double4(0, 0, 0, 0);
-    return;
+  // Plain stores by the blocks that read the flag clear (writers agree, and a
+  // stale read costs another store): an atomic for every wave serialises on its
+  // address, 180 us for the 8.8e5 vertices of a discretized knit.
+  if (__syncthreads_or(bad) && threadIdx.x == 0 &&
+      __hip_atomic_load(inexact, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) {
+    __hip_atomic_store(inexact, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    *inexact_host = 1;
   }
-  const int64_t src = in_off[c] + (l < n ? l : 0);
-  out[v] = make_double4((xyz[3 * src] - ox) * scale, (xyz[3 * src + 1] - oy) * scale,
-                        (xyz[3 * src + 2] - oz) * scale, 0.0);
 }
 
 __device__ __forceinline__ uint32_t spread10(uint32_t v) {
@@ -298,17 +336,85 @@ __global__ __launch_bounds__(256) void pls_all_pairs(const double *__restrict__ 
 // 16,384, 1,052 and 636 for 30,000; the sweep grows with the square.
 constexpr int32_t kAllPairsCurves = 32768;
 
+// Up to kOneBlockCurves curves in one launch: the boxes in LDS, a row a wave at a
+// time, counted and, after a scan of the rows' counts, written.  For ten curves
+// the three launches were most of the call.
+constexpr int32_t kOneBlockCurves = 256;
+__global__ __launch_bounds__(1024) void pls_one_block(const double *__restrict__ boxes, int32_t n, int64_t cap,
+                                                      int2 *__restrict__ out, int64_t *__restrict__ total) {
+  __shared__ double box[6][kOneBlockCurves];
+  __shared__ int first[kOneBlockCurves];
+  __shared__ int sum[kOneBlockCurves / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, waves = (int)(blockDim.x >> 6);
+  for (int t = threadIdx.x; t < 6 * n; t += (int)blockDim.x) box[t % 6][t / 6] = boxes[t];
+  __syncthreads();
+  auto row = [&](int i, auto found) {  // found(mask of the overlaps from column j0)
+    Box6 a;
+    for (int d = 0; d < 3; ++d) {
+      a.mn[d] = box[d][i];
+      a.mx[d] = box[3 + d][i];
+    }
+    for (int j0 = (i + 1) / 64 * 64; j0 < n; j0 += 64) {
+      const int j = j0 + lane;
+      Box6 b;
+      for (int d = 0; d < 3; ++d) {
+        b.mn[d] = box[d][min(j, n - 1)];
+        b.mx[d] = box[3 + d][min(j, n - 1)];
+      }
+      found(j0, __ballot(j > i && j < n && box_overlap(a, b)));
+    }
+  };
+  for (int i = w; i < n; i += waves) {
+    int cnt = 0;
+    row(i, [&](int, uint64_t m) { cnt += __popcll(m); });
+    if (lane == 0) first[i] = cnt;
+  }
+  __syncthreads();
+  int mine = 0, inc = 0;  // the rows' counts, scanned
+  if (threadIdx.x < kOneBlockCurves) {
+    mine = inc = (int)threadIdx.x < n ? first[threadIdx.x] : 0;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += u;
+    }
+    if (lane == 63) sum[w] = inc;
+  }
+  __syncthreads();
+  if (threadIdx.x < kOneBlockCurves) {
+    for (int k = 0; k < w; ++k) inc += sum[k];
+    first[threadIdx.x] = inc - mine;
+    if (threadIdx.x == kOneBlockCurves - 1) *total = inc;
+  }
+  __syncthreads();
+  for (int i = w; i < n; i += waves) {
+    int at = first[i];
+    row(i, [&](int j0, uint64_t m) {
+      const int slot = at + __popcll(m & ((1ull << lane) - 1ull));
+      if (((m >> lane) & 1ull) && slot < cap) out[slot] = make_int2(i, j0 + lane);
+      at += __popcll(m);
+    });
+  }
+}
+
+// Pinned memory of the search that a call may leave behind.
+constexpr size_t kKeptPinned = size_t(64) << 20;
+
 void pls_small(flk_ctx *ctx, const double *d_boxes, int32_t n, std::vector<int32_t> &out) {
   hipStream_t s = ctx->stream;
+  const bool one = n <= kOneBlockCurves;
   const int32_t chunks = (n + kColChunk - 1) / kColChunk;
   const int64_t ncells = (int64_t)n * chunks;
-  ctx->d_pls.reserve(sizeof(int32_t) * (ncells + 1) + scan_temp_bytes(ncells + 1));
-  int32_t *cells = ctx->d_pls.as<int32_t>(), *tmp = cells + ncells + 1;
   const dim3 grid((unsigned)((n + 4 * kRowsPerWave - 1) / (4 * kRowsPerWave)), (unsigned)chunks);
-  hipLaunchKernelGGL(pls_all_pairs<false>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, (int64_t)0,
-                     (int2 *)nullptr, (int64_t *)nullptr);
-  FLK_HIP(hipGetLastError());
-  exclusive_scan(cells, cells, ncells + 1, tmp, s);
+  int32_t *cells = nullptr;
+  if (!one) {
+    ctx->d_pls.reserve(sizeof(int32_t) * (ncells + 1) + scan_temp_bytes(ncells + 1));
+    cells = ctx->d_pls.as<int32_t>();
+    hipLaunchKernelGGL(pls_all_pairs<false>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, (int64_t)0,
+                       (int2 *)nullptr, (int64_t *)nullptr);
+    FLK_HIP(hipGetLastError());
+    exclusive_scan(cells, cells, ncells + 1, cells + ncells + 1, s);
+  }
   // the pairs land in pinned memory behind their total; a second sweep only
   // when there are more than eight pairs a curve (and than ever before)
   int64_t cap = std::max<int64_t>(1024, 8 * (int64_t)n);
@@ -317,12 +423,16 @@ void pls_small(flk_ctx *ctx, const double *d_boxes, int32_t n, std::vector<int32
     cap = (int64_t)(ctx->pls_host.bytes / sizeof(int64_t)) - 1;
     int64_t *total = ctx->pls_host.as<int64_t>();
     int2 *pairs = reinterpret_cast<int2 *>(total + 1);
-    hipLaunchKernelGGL(pls_all_pairs<true>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, cap, pairs, total);
+    if (one)
+      hipLaunchKernelGGL(pls_one_block, dim3(1), dim3(1024), 0, s, d_boxes, n, cap, pairs, total);
+    else
+      hipLaunchKernelGGL(pls_all_pairs<true>, grid, dim3(256), 0, s, d_boxes, n, chunks, cells, cap, pairs, total);
     FLK_HIP(hipGetLastError());
     FLK_HIP(hipStreamSynchronize(s));
     if (*total <= cap) {
       const int32_t *p = reinterpret_cast<const int32_t *>(pairs);
       out.assign(p, p + 2 * *total);
+      if (ctx->pls_host.bytes > kKeptPinned) ctx->pls_host.release();
       return;
     }
     cap = *total;
@@ -333,53 +443,69 @@ void pls_small(flk_ctx *ctx, const double *d_boxes, int32_t n, std::vector<int32
 
 void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes) {
   Curves &cv = ctx->curves;
-  boxes.assign(6 * (size_t)cv.ncurves, 0.0);
-  if (cv.ncurves == 0) return;
-  // chunk table: (first, end) vertex of every chunk, and each curve's chunks
-  std::vector<int64_t> meta(cv.ncurves + 1);
-  std::vector<int64_t> chunk_v;
-  for (int32_t c = 0; c < cv.ncurves; ++c) {
-    meta[c] = (int64_t)chunk_v.size() / 2;
-    for (int64_t v = cv.in_off[c]; v < cv.in_off[c + 1]; v += kBoxChunk) {
-      chunk_v.push_back(v);
-      chunk_v.push_back(std::min(v + kBoxChunk, cv.in_off[c + 1]));
+  const size_t nc = (size_t)cv.ncurves;
+  boxes.assign(6 * nc, 0.0);
+  if (nc == 0) return;
+  // input and device offsets, the chunk table ((first, end) vertex of every
+  // chunk) and each curve's chunks, in pinned memory on their way to the device
+  int64_t nchunks = 0;
+  for (size_t c = 0; c < nc; ++c) nchunks += (cv.in_off[c + 1] - cv.in_off[c] + kBoxChunk - 1) / kBoxChunk;
+  bool single = nchunks <= (int64_t)nc;  // then empty curves have a chunk too
+  for (size_t c = 0; single && c < nc; ++c) single = cv.in_off[c + 1] - cv.in_off[c] <= kBoxChunk;
+  if (single) nchunks = (int64_t)nc;
+  const size_t words = 3 * (nc + 1) + 2 * (size_t)nchunks;
+  ctx->curve_host.reserve(sizeof(int64_t) * words + sizeof(double) * 6 * nc + sizeof(int32_t));
+  int64_t *meta = ctx->curve_host.as<int64_t>();
+  double *host = reinterpret_cast<double *>(meta + words);
+  ctx->inexact_host = reinterpret_cast<int32_t *>(host + 6 * nc);
+  *ctx->inexact_host = 0;
+  std::copy(cv.in_off.begin(), cv.in_off.end(), meta);
+  std::copy(cv.off.begin(), cv.off.end(), meta + nc + 1);
+  int64_t *coff = meta + 2 * (nc + 1), *chunk = coff + nc + 1, k = 0;
+  for (size_t c = 0; c < nc; ++c) {
+    coff[c] = k;
+    int64_t v = cv.in_off[c];
+    const int64_t end = cv.in_off[c + 1];
+    if (single && v == end) {
+      chunk[2 * k] = chunk[2 * k + 1] = v;
+      ++k;
+    }
+    for (; v < end; v += kBoxChunk, ++k) {
+      chunk[2 * k] = v;
+      chunk[2 * k + 1] = std::min(v + kBoxChunk, end);
     }
   }
-  const int64_t nchunks = (int64_t)chunk_v.size() / 2;
-  meta[cv.ncurves] = nchunks;
-  meta.insert(meta.end(), chunk_v.begin(), chunk_v.end());
-  ctx->d_boxes.reserve(sizeof(double) * 6 * (cv.ncurves + std::max<int64_t>(nchunks, 1)));
-  ctx->d_misc.reserve(sizeof(int64_t) * meta.size());
-  FLK_HIP(hipMemcpyAsync(ctx->d_misc.ptr, meta.data(), sizeof(int64_t) * meta.size(), hipMemcpyHostToDevice,
-                         ctx->stream));
-  double *d_boxes = ctx->d_boxes.as<double>(), *d_part = d_boxes + 6 * (size_t)cv.ncurves;
-  const int64_t *d_coff = ctx->d_misc.as<int64_t>(), *d_chunk = d_coff + cv.ncurves + 1;
-  if (nchunks > 0) {
-    hipLaunchKernelGGL(curve_box_chunks, dim3((unsigned)nchunks), dim3(256), 0, ctx->stream,
-                       cv.raw.as<double>(), d_chunk, d_part);
-    FLK_HIP(hipGetLastError());
-  }
-  hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((cv.ncurves + 255) / 256)), dim3(256), 0, ctx->stream,
-                     d_part, d_coff, cv.ncurves, d_boxes);
+  coff[nc] = nchunks;
+  hipStream_t s = ctx->stream;
+  ctx->d_boxes.reserve(sizeof(double) * 6 * (nc + std::max<int64_t>(nchunks, 1)));
+  ctx->d_misc.reserve(sizeof(int64_t) * words);
+  ctx->d_count.reserve(sizeof(int32_t));
+  FLK_HIP(hipMemcpyAsync(ctx->d_misc.ptr, meta, sizeof(int64_t) * words, hipMemcpyHostToDevice, s));
+  double *d_boxes = ctx->d_boxes.as<double>(), *d_part = d_boxes + 6 * nc;
+  const int64_t *d_coff = ctx->d_misc.as<int64_t>() + 2 * (nc + 1), *d_chunk = d_coff + nc + 1;
+  int32_t *flag = ctx->d_count.as<int32_t>();
+  if (nchunks > 0)
+    hipLaunchKernelGGL(curve_box_chunks, dim3((unsigned)nchunks), dim3(256), 0, s, cv.raw.as<double>(), d_chunk,
+                       single ? d_boxes : d_part, single ? host : (double *)nullptr, flag);
+  if (!single)
+    hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, d_part, d_coff,
+                       cv.ncurves, d_boxes, host, flag);
   FLK_HIP(hipGetLastError());
-  FLK_HIP(hipMemcpyAsync(boxes.data(), d_boxes, sizeof(double) * 6 * cv.ncurves, hipMemcpyDeviceToHost,
-                         ctx->stream));
-  FLK_HIP(hipStreamSynchronize(ctx->stream));
+  FLK_HIP(hipStreamSynchronize(s));
+  boxes.assign(host, host + 6 * nc);
 }
 
-void stage_vertices_launch(flk_ctx *ctx) {
+bool stage_vertices_run(flk_ctx *ctx) {
   Curves &cv = ctx->curves;
-  ctx->d_misc.reserve(sizeof(int64_t) * (cv.ncurves + 1));
-  FLK_HIP(hipMemcpyAsync(ctx->d_misc.ptr, cv.in_off.data(), sizeof(int64_t) * (cv.ncurves + 1),
-                         hipMemcpyHostToDevice, ctx->stream));
-  FLK_HIP(hipMemcpyAsync(cv.d_off.ptr, cv.off.data(), sizeof(int64_t) * (cv.ncurves + 1),
-                         hipMemcpyHostToDevice, ctx->stream));
   const int64_t blocks = (cv.nvert_dev + 255) / 256;
-  hipLaunchKernelGGL(stage_vertices, dim3((unsigned)blocks), dim3(256), 0, ctx->stream,
-                     cv.raw.as<double>(), ctx->d_misc.as<int64_t>(), cv.d_off.as<int64_t>(),
-                     cv.ncurves, cv.nvert_dev, cv.origin[0], cv.origin[1], cv.origin[2],
-                     cv.scale, cv.dpts.as<double4>());
+  const int64_t *d_in = ctx->d_misc.as<int64_t>();
+  hipLaunchKernelGGL(stage_vertices, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, cv.raw.as<double>(), d_in,
+                     d_in + cv.ncurves + 1, cv.ncurves, cv.nvert_dev, cv.origin[0], cv.origin[1], cv.origin[2],
+                     cv.scale, cv.dpts.as<double4>(), cv.hi.as<float4>(), cv.lo.as<float4>(), cv.ed.as<float4>(),
+                     ctx->d_count.as<int32_t>(), ctx->inexact_host);
   FLK_HIP(hipGetLastError());
+  FLK_HIP(hipStreamSynchronize(ctx->stream));
+  return *ctx->inexact_host != 0;
 }
 
 void pls_run(flk_ctx *ctx, const double *boxes, int32_t n, std::vector<int32_t> &out) {

@@ -1,0 +1,46 @@
+"""An upload's boxes and vertices at the edges of their kernels: curves of one and
+of several box chunks (16,384 vertices), empty and short ones among them, and
+the one-block potential-link search at the ends of its range."""
+import numpy as np
+import pytest
+
+flk = pytest.importorskip("fastlinkingnumbers_amd")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("sizes", [[1, 0, 2, 16384, 3], [16385, 0, 5], [0, 40000, 1, 16384], [0, 0]], ids=str)
+def test_boxes_and_direct_sums(engine, sizes, dtype):
+    """The boxes are the vertices' extrema exactly; a Hopf link appended behind
+    the curves has its integer by either precision."""
+    rng = np.random.default_rng(len(sizes))
+    t = 2 * np.pi * np.arange(300) / 300
+    ring = np.stack([np.cos(t), np.sin(t), 0 * t], 1) + 20
+    curves = [rng.normal(size=(n, 3)) for n in sizes] + [ring, ring[:, [0, 2, 1]] * [1, 1, 1] + [1, 0, 0]]
+    packed = np.concatenate(curves).astype(dtype)
+    offsets = np.concatenate([[0], np.cumsum([len(c) for c in curves])])
+    engine.set_curves_packed(packed, offsets)
+    boxes = engine.curve_boxes()
+    for k, (a, b) in enumerate(zip(offsets[:-1], offsets[1:])):
+        if b > a:
+            v = packed[a:b].astype(np.float64)
+            assert np.array_equal(boxes[k], np.concatenate([v.min(0), v.max(0)])), k
+    n = len(sizes)
+    for fp64 in (0, 1):
+        lk = engine.linking_numbers([[n, n + 1]], method="directsum", fp64=fp64, fallback_tol=0.0).lk[0]
+        assert abs(abs(lk) - 1) < 1e-4, lk
+
+
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 128, 255, 256, 257])
+def test_one_block_search_is_every_overlapping_pair(engine, n):
+    """All pairs in ascending order; touching, empty and all-overlapping boxes,
+    more pairs than the first pinned array holds among them."""
+    rng = np.random.default_rng(n)
+    lo = np.round(rng.uniform(0, 4, size=(n, 3)))
+    for size in (0.0, 1.0, 10.0):
+        boxes = np.concatenate([lo, lo + size], 1)
+        boxes[n // 2] = [1, 1, 1, 0, 0, 0]  # empty
+        i, j = np.triu_indices(n, 1)
+        near = np.all((boxes[i, :3] <= boxes[j, 3:]) & (boxes[j, :3] <= boxes[i, 3:]), axis=1)
+        assert np.array_equal(engine.potential_links(boxes), np.stack([i[near], j[near]], 1)), size

@@ -146,8 +146,8 @@ __device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
 // the split nodes' ranks need no scan).
 struct BhShape {
   int32_t n, full, m;
-  __device__ __forceinline__ BhShape(int32_t n_, int32_t leaf) : n(n_), full(0) {
-    while ((n >> full) > leaf) ++full;
+  __device__ __forceinline__ BhShape(int32_t n_, int32_t leaf) : n(n_), full(max(0, __clz(leaf) - __clz(n_))) {
+    full += (n >> full) > leaf;  // as many bits as leaf, so at most one level more
     m = n >> full;
   }
   __device__ __forceinline__ int32_t big() const { return n - (m << full); }
@@ -1056,16 +1056,18 @@ __device__ __forceinline__ void load_infer_image(const InferImage *__restrict__ 
 // as (pair with the split side in its sign, unsplit node, child 0, child 1)
 // from the front of the block's stage, leaf-bucket items from the back; after
 // the block has classified its 256 * IPT items the stage is copied out
-// coalesced behind one queue atomic each.  MLP: the learned criterion, its
+// coalesced behind one queue atomic each.  A queue past the roots holds these
+// records as they are, one for the two items of a split: bound by the bytes it
+// moves, a visit reads and writes 8 of the queue instead of 16.  MLP: the learned criterion, its
 // network evaluated here on the node records the level already holds (the
 // weight fragments in LDS, loaded once per block); *evals counts the
 // evaluations.
 template <int IPT, bool MLP>
 __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4))) void bh_level(
-    const BhItem *__restrict__ items, int64_t n, const unsigned long long *__restrict__ n_dev,
+    const int4 *__restrict__ items, int64_t n, const unsigned long long *__restrict__ n_dev, int roots,
     const BhGeo *__restrict__ geo, const BhMom *__restrict__ mom, const float *__restrict__ beta2,
     float eps, const InferImage *__restrict__ mlp_img, float log_tol, unsigned long long *__restrict__ evals,
-    BhItem *__restrict__ next, unsigned long long *__restrict__ next_count, int64_t next_cap,
+    int4 *__restrict__ next, unsigned long long *__restrict__ next_count, int64_t next_cap,
     BhItem *__restrict__ leaves, unsigned long long *__restrict__ leaf_count, int64_t leaf_cap,
     double *__restrict__ psum, double *__restrict__ perr) {
   constexpr int kTravItems = kTravBlock * IPT;
@@ -1104,7 +1106,15 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
   for (int k = 0; k < IPT && k * kTravBlock < csz; ++k) {
     const int64_t t = b0 + (int64_t)k * kTravBlock;
     const bool live = t < n;
-    BhItem it = live ? items[t] : BhItem{0, 0, 0, 0};
+    BhItem it{0, 0, 0, 0};
+    if (live && roots) {
+      const int4 r = items[t];
+      it = BhItem{r.x, r.y, r.z, 0};
+    } else if (live) {  // one of a split node's two children with the other side's node
+      const int4 r = items[t >> 1];
+      const int c = t & 1 ? r.w : r.z;
+      it = r.x < 0 ? BhItem{~r.x, c, r.y, 0} : BhItem{r.x, r.y, c, 0};
+    }
     const BhVisit v = bh_visit<MLP>(it, live, geo, mom, beta2, eps, log_tol, ms, wave_evals);
     if (v.kind == 1) {
       if (tp < 0 || tp == it.pair) {
@@ -1130,19 +1140,8 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
   }
   __syncthreads();
   const int64_t bn = (int64_t)sh.base[0], bl = (int64_t)sh.base[1];
-  for (int i = threadIdx.x; i < ns; i += kTravBlock) {
-    const int4 r = stage[i];
-    const int64_t s = bn + 2 * (int64_t)i;
-    if (s + 1 < next_cap) {
-      if (r.x < 0) {  // node 1 split: (child, unsplit node 2)
-        next[s] = BhItem{~r.x, r.z, r.y, 0};
-        next[s + 1] = BhItem{~r.x, r.w, r.y, 0};
-      } else {
-        next[s] = BhItem{r.x, r.y, r.z, 0};
-        next[s + 1] = BhItem{r.x, r.y, r.w, 0};
-      }
-    }
-  }
+  for (int i = threadIdx.x; i < ns; i += kTravBlock)
+    if (bn + 2 * (int64_t)i + 1 < next_cap) next[bn / 2 + i] = stage[i];
   for (int i = threadIdx.x; i < nl; i += kTravBlock) {
     const int64_t s = bl + i;
     if (s < leaf_cap) {
@@ -2042,9 +2041,9 @@ int items_per_thread(const flk_ctx *ctx, bool use_mlp) {
 }
 
 // The level kernel for a criterion and a number of items per thread.
-using LevelKernel = void (*)(const BhItem *, int64_t, const unsigned long long *, const BhGeo *, const BhMom *,
+using LevelKernel = void (*)(const int4 *, int64_t, const unsigned long long *, int, const BhGeo *, const BhMom *,
                              const float *, float, const InferImage *, float, unsigned long long *,
-                             BhItem *, unsigned long long *, int64_t, BhItem *, unsigned long long *, int64_t,
+                             int4 *, unsigned long long *, int64_t, BhItem *, unsigned long long *, int64_t,
                              double *, double *);
 LevelKernel level_kernel(int ipt, bool use_mlp) {
   if (use_mlp) return ipt == 2 ? bh_level<2, true> : ipt == 8 ? bh_level<8, true> : bh_level<4, true>;
@@ -2088,6 +2087,7 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
   struct Level {
     DevBuf *buf;
     int64_t n;
+    bool roots;
   };
   std::vector<Level> stack;
   size_t used = 0;  // level buffers handed out from B.levels
@@ -2097,7 +2097,7 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
     b->reserve(sizeof(BhItem) * std::max<int64_t>(items, 1));
     return b;
   };
-  stack.push_back(Level{level_buf(np), np});
+  stack.push_back(Level{level_buf(np), np, true});
   hipLaunchKernelGGL(bh_roots, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s,
                      B.roots_a.as<int32_t>(), B.roots_b.as<int32_t>(), np, stack[0].buf->as<BhItem>());
   FLK_HIP(hipGetLastError());
@@ -2116,7 +2116,8 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
     }
     const int64_t take = std::min<int64_t>(top.n, kChunk);
     top.n -= take;
-    const BhItem *src = top.buf->as<BhItem>() + top.n;
+    const int4 *src = top.buf->as<int4>() + (top.roots ? top.n : top.n / 2);  // two items a record past the roots
+    const bool roots = top.roots;
     // Levels enqueued before the next read-back: the first from its exact
     // count and, when it is consumed whole, up to kRound - 1 more, level d
     // sized for its bound take * 2^d (a level at most doubles) and reading
@@ -2146,15 +2147,15 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
     DevBuf *outb[kRound];
     for (int d = 0; d < D; ++d) {
       outb[d] = (d % 2 == 0) ? spare : alt;
-      const BhItem *in = d == 0 ? src : outb[d - 1]->as<BhItem>();
+      const int4 *in = d == 0 ? src : outb[d - 1]->as<int4>();
       const int64_t bound = take << d;
       const unsigned long long *n_dev = d == 0 ? nullptr : qc + 2 * (d - 1);
       // with timing, start/stop events ride on the dispatch itself
       const dim3 grid((unsigned)((bound + ipt * kTravBlock - 1) / (ipt * kTravBlock)));
       launch_timed(timing ? ctx->ev1 : nullptr, timing ? ctx->ev2 : nullptr, level_kernel(ipt, use_mlp), grid,
-                   dim3(kTravBlock), s, in, bound, n_dev, F.geo.as<BhGeo>(), F.mom.as<BhMom>(),
+                   dim3(kTravBlock), s, in, bound, n_dev, (int)(roots && d == 0), F.geo.as<BhGeo>(), F.mom.as<BhMom>(),
                    (const float *)B.beta2.as<float>(), eps, mlp_img, log_tol, cnt + 3,
-                   outb[d]->as<BhItem>(), qc + 2 * d, 2 * bound, B.leaves.as<BhItem>(), qc + 1, leaf_cap, d_sum,
+                   outb[d]->as<int4>(), qc + 2 * d, 2 * bound, B.leaves.as<BhItem>(), qc + 1, leaf_cap, d_sum,
                    d_err);
       FLK_HIP(hipGetLastError());
     }
@@ -2194,10 +2195,11 @@ void traverse(flk_ctx *ctx, Forest &F, const std::vector<int32_t> &ra, const std
       DevBuf *consumed = top.buf;
       top.buf = last;
       top.n = in_n;
+      top.roots = false;
       if (D > 1) alt = (last == spare) ? alt : spare;
       spare = consumed;
     } else if (in_n > 0) {
-      stack.push_back(Level{last, in_n});  // D == 1: last is spare
+      stack.push_back(Level{last, in_n, false});  // D == 1: last is spare
       spare = level_buf(2 * kChunk);
     }
   }
@@ -2272,8 +2274,10 @@ bool plan_device_passes(flk_ctx *ctx, int64_t nb, int64_t segments, int depth, b
   P.ipt = items_per_thread(ctx, use_mlp);
   P.copies = P.walk && nb <= 4096 ? 8 : 1;
   while (B.levels.size() < 2) B.add_level();
-  B.levels[0]->reserve(sizeof(BhItem) * P.cap);
-  B.levels[1]->reserve(sizeof(BhItem) * P.cap);
+  // a walk's items, or a level's records of two items each
+  const size_t level_bytes = P.walk ? sizeof(BhItem) * P.cap : sizeof(int4) * (P.cap / 2 + 1);
+  B.levels[0]->reserve(level_bytes);
+  B.levels[1]->reserve(level_bytes);
   B.leaves.reserve(sizeof(BhItem) * P.cap);
   auto leafk = P.ipt == 2 ? bh_leaf_pairs<2> : P.ipt == 8 ? bh_leaf_pairs<8> : bh_leaf_pairs<4>;
   const int64_t items_per_block = (int64_t)P.ipt * kTravBlock;
@@ -2311,9 +2315,9 @@ void enqueue_pass(flk_ctx *ctx, const PassShape &P, const BhItem *items0, const 
                          B.mom.as<BhMom>(), beta2, eps, cnt, d, buf[d & 1], B.leaves.as<BhItem>(), d_sum, d_err,
                          P.copies, copy_stride);
     else
-      hipLaunchKernelGGL(lev, dim3(P.grid_lev), dim3(kTravBlock), 0, s, in, P.cap,
-                         (const unsigned long long *)(cnt + 4 + 2 * d), B.geo.as<BhGeo>(), B.mom.as<BhMom>(), beta2,
-                         eps, mlp_img, log_tol, cnt + 3, buf[d & 1], cnt + 4 + 2 * (d + 1), P.cap,
+      hipLaunchKernelGGL(lev, dim3(P.grid_lev), dim3(kTravBlock), 0, s, reinterpret_cast<const int4 *>(in), P.cap,
+                         (const unsigned long long *)(cnt + 4 + 2 * d), (int)(d == 0), B.geo.as<BhGeo>(), B.mom.as<BhMom>(), beta2,
+                         eps, mlp_img, log_tol, cnt + 3, reinterpret_cast<int4 *>(buf[d & 1]), cnt + 4 + 2 * (d + 1), P.cap,
                          B.leaves.as<BhItem>(), cnt + 5, P.cap, d_sum, d_err);
     FLK_HIP(hipGetLastError());
   }

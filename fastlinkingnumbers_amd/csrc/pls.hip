@@ -37,8 +37,8 @@ __device__ __forceinline__ bool box_overlap(const Box6 &a, const Box6 &b) {
 
 // FP64 min/max of each curve's vertices (the polyline case of reference
 // curve.cpp:331-343; an empty curve gets the empty box) in two passes: one
-// block per chunk of at most kBoxChunk vertices of one curve, then one thread
-// per curve folding its chunks, so a curve of millions of vertices is spread
+// block per chunk of at most kBoxChunk vertices of one curve, then one wave per
+// curve folding its chunks (a thread took 115 us for 490 chunks), so a curve of millions of vertices is spread
 // over the whole chip; where every curve is one chunk the first pass is all.
 // The boxes also go to pinned memory (`host`) without a copy, and the last pass
 // clears the flag that stage_vertices sets.
@@ -95,15 +95,22 @@ __global__ __launch_bounds__(256) void curve_box_merge(const double *__restrict_
                                                        const int64_t *__restrict__ coff, int32_t ncurves,
                                                        double *__restrict__ boxes, double *__restrict__ host,
                                                        int32_t *__restrict__ inexact) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c == 0) *inexact = 0;
+  const int c = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  if (c == 0 && lane == 0) *inexact = 0;
   if (c >= ncurves) return;
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  for (int64_t k = coff[c]; k < coff[c + 1]; ++k)
+  for (int64_t k = coff[c] + lane; k < coff[c + 1]; k += 64)
     for (int d = 0; d < 3; ++d) {
       mn[d] = fmin(mn[d], part[6 * k + d]);
       mx[d] = fmax(mx[d], part[6 * k + 3 + d]);
     }
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    for (int o = 32; o > 0; o >>= 1) {
+      mn[d] = fmin(mn[d], __shfl_xor(mn[d], o, 64));
+      mx[d] = fmax(mx[d], __shfl_xor(mx[d], o, 64));
+    }
+  if (lane) return;
   for (int d = 0; d < 3; ++d) {
     boxes[6 * c + d] = host[6 * c + d] = mn[d];
     boxes[6 * c + 3 + d] = host[6 * c + 3 + d] = mx[d];
@@ -488,7 +495,7 @@ void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes) {
     hipLaunchKernelGGL(curve_box_chunks, dim3((unsigned)nchunks), dim3(256), 0, s, cv.raw.as<double>(), d_chunk,
                        single ? d_boxes : d_part, single ? host : (double *)nullptr, flag);
   if (!single)
-    hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s, d_part, d_coff,
+    hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, d_part, d_coff,
                        cv.ncurves, d_boxes, host, flag);
   FLK_HIP(hipGetLastError());
   FLK_HIP(hipStreamSynchronize(s));

@@ -2478,6 +2478,9 @@ struct BatchPlan {
     up.add(rb, d_rb);
     up.add(beta2, d_beta2);
   }
+  const unsigned long long *heads() const {
+    return reinterpret_cast<const unsigned long long *>(res.as<double>() + 2 * idx.size());
+  }
   void collect() {  // res into the vectors
     const double *hv = res.as<double>();
     std::copy(hv, hv + v.size(), v.begin());
@@ -2566,9 +2569,11 @@ void enqueue_begin(flk_ctx *ctx, const BatchPlan &bp, hipStream_t s) {
 
 // Traversal of a planned batch on the device schedule, after its forest:
 // first pass, the re-run decision (bh_adapt), second pass over the re-run
-// list, the merge, and the read-back of results and counters.  Kernels and
-// copies only, so it can be captured.
-void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipStream_t s) {
+// list and the merge of results and counters.  Kernels only, so it can be
+// captured.  `first` and `second` pick the passes to enqueue (a merge follows
+// either).
+void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipStream_t s, bool first = true,
+                       bool second = true) {
   BhScratch &B = ctx->bh;
   const Curves &cv = ctx->curves;
   const bool use_mlp = prm.criterion == FLK_CRIT_MLP;
@@ -2577,12 +2582,15 @@ void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipSt
   const float eps = (float)(prm.eps_sq * cv.scale * cv.scale);
   const float log_tol = (float)prm.mlp_log_tol;
   double *sum = B.sum.as<double>(), *err = B.err.as<double>();
-  enqueue_begin(ctx, bp, s);
   unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + kPassWords;
-  enqueue_pass(ctx, P, B.items0.as<BhItem>(), bp.d_beta2, eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);
-  enqueue_adapt(ctx, bp, prm, c2 + 4, s);
-  enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, eps, use_mlp, log_tol - 1.0f, c2, sum + nb,
-               err + nb, 2 * nb, s);
+  if (first) {
+    enqueue_begin(ctx, bp, s);
+    enqueue_pass(ctx, P, B.items0.as<BhItem>(), bp.d_beta2, eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);
+    enqueue_adapt(ctx, bp, prm, c2 + 4, s);
+  }
+  if (second)
+    enqueue_pass(ctx, P, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, eps, use_mlp, log_tol - 1.0f, c2, sum + nb,
+                 err + nb, 2 * nb, s);
   enqueue_merge(ctx, bp, prm, c1, s);
 }
 
@@ -2773,20 +2781,47 @@ std::vector<std::vector<int64_t>> form_batches(flk_ctx *ctx, const int32_t *pair
 // from the pairs and the curves' sizes but for the key boxes, so new positions
 // of the same curves replay it too, with the plans sent again: capturing and
 // instantiating 50-100 nodes for each step of a simulation took longer than
-// running them.
+// running them.  With one Barnes–Hut batch the second pass is a graph of its own
+// (`again`), launched when the first has pairs to re-run, which is known after
+// it: 7 launches of a walk or 45-50 of levels that would find nothing take 36 or
+// 250 us.  A certificate that had re-runs is launched with it at once.
 struct CertGraph {
   GraphKey key;
   uint64_t epoch = 0;
-  hipGraphExec_t exec = nullptr;
+  hipGraphExec_t exec = nullptr, again = nullptr;
+  bool reran = false;  // the last launch had pairs to re-run
   std::vector<int64_t> ds_idx;
   DsGraph ds;
   std::vector<BatchPlan> batches;
   ~CertGraph() {
     if (exec) (void)hipGraphExecDestroy(exec);
+    if (again) (void)hipGraphExecDestroy(again);
   }
 };
 
 namespace {
+
+// What `body` enqueues on s, captured and instantiated.
+template <typename F> hipGraphExec_t captured(hipStream_t s, F &&body) {
+  hipGraph_t graph = nullptr;
+  FLK_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  t_capturing = true;
+  try {
+    body();
+  } catch (...) {
+    t_capturing = false;
+    (void)hipStreamEndCapture(s, &graph);
+    if (graph) (void)hipGraphDestroy(graph);
+    throw;
+  }
+  t_capturing = false;
+  FLK_HIP(hipStreamEndCapture(s, &graph));
+  hipGraphExec_t exec = nullptr;
+  const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(graph);
+  if (ie != hipSuccess) throw Error(FLK_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
+  return exec;
+}
 
 // Captures (or finds) the certificate graph for these pairs and launches it;
 // false when a batch does not fit the device schedule (the caller then runs
@@ -2840,51 +2875,38 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
       ds_capture_prepare(ctx, ds_pairs.data(), (int64_t)ds_idx.size(), prm.fp64 != 0, NG->ds, share);
     }
     FLK_HIP(hipStreamSynchronize(s));
-    hipGraph_t graph = nullptr;
-    FLK_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    t_capturing = true;
     // A hybrid certificate's direct-sum part (VALU-bound) and its Barnes-Hut
     // batches (memory-bound builds and traversals) share nothing they write:
     // the direct sum is a branch of its own, forked from the capture stream
     // onto the context's second stream and joined before the capture ends.
     const bool fork = !ds_idx.empty() && !NG->batches.empty();
-    bool forked = false, joined = false;
-    try {
-      if (fork) {
-        FLK_HIP(hipEventRecord(ctx->ev_fork, s));
-        FLK_HIP(hipStreamWaitEvent(ctx->aux, ctx->ev_fork, 0));
-        forked = true;
-        ds_capture_enqueue(ctx, NG->ds, ctx->aux);
-      } else if (!ds_idx.empty()) {
-        ds_capture_enqueue(ctx, NG->ds, s);
-      }
-      for (BatchPlan &bp : NG->batches) {
-        enqueue_forest(ctx, bp.forest, s);
-        enqueue_traversal(ctx, bp, prm, s);
+    NG->exec = captured(s, [&]() {
+      bool forked = false;
+      try {
+        if (fork) {
+          FLK_HIP(hipEventRecord(ctx->ev_fork, s));
+          FLK_HIP(hipStreamWaitEvent(ctx->aux, ctx->ev_fork, 0));
+          forked = true;
+          ds_capture_enqueue(ctx, NG->ds, ctx->aux);
+        } else if (!ds_idx.empty()) {
+          ds_capture_enqueue(ctx, NG->ds, s);
+        }
+        for (BatchPlan &bp : NG->batches) {
+          enqueue_forest(ctx, bp.forest, s);
+          enqueue_traversal(ctx, bp, prm, s, true, NG->batches.size() > 1);
+        }
+      } catch (...) {
+        if (forked) {  // the capture cannot end with a branch left open
+          (void)hipEventRecord(ctx->ev_join, ctx->aux);
+          (void)hipStreamWaitEvent(s, ctx->ev_join, 0);
+        }
+        throw;
       }
       if (forked) {
         FLK_HIP(hipEventRecord(ctx->ev_join, ctx->aux));
         FLK_HIP(hipStreamWaitEvent(s, ctx->ev_join, 0));
-        joined = true;
       }
-    } catch (...) {
-      t_capturing = false;
-      if (forked && !joined) {  // the capture cannot end with a branch left open
-        (void)hipEventRecord(ctx->ev_join, ctx->aux);
-        (void)hipStreamWaitEvent(s, ctx->ev_join, 0);
-      }
-      (void)hipStreamEndCapture(s, &graph);
-      if (graph) (void)hipGraphDestroy(graph);
-      throw;
-    }
-    t_capturing = false;
-    FLK_HIP(hipStreamEndCapture(s, &graph));
-    const hipError_t ie = hipGraphInstantiate(&NG->exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (ie != hipSuccess) {
-      NG->exec = nullptr;
-      throw Error(FLK_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
-    }
+    });
     NG->epoch = g_devbuf_epoch.load();
     ctx->cert_graph = NG;
     G = NG.get();
@@ -2901,8 +2923,21 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
   FLK_HIP(hipGraphLaunch(G->exec, s));
   ctx->stats.ms_graph_launch =
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+  const bool at_once = G->again && G->reran;
+  if (at_once) FLK_HIP(hipGraphLaunch(G->again, s));
   FLK_HIP(hipEventRecord(ctx->ev1, s));
   FLK_HIP(hipStreamSynchronize(s));
+  if (G->batches.size() == 1) {
+    const unsigned long long *head = G->batches[0].heads();
+    G->reran = head[kPassHead + 4] != 0;
+    if (G->reran && !at_once && head[6] == 0) {  // (an overflowed first pass goes to the host)
+      if (!G->again)
+        G->again = captured(s, [&]() { enqueue_traversal(ctx, G->batches[0], prm, s, false, true); });
+      FLK_HIP(hipGraphLaunch(G->again, s));
+      FLK_HIP(hipEventRecord(ctx->ev1, s));
+      FLK_HIP(hipStreamSynchronize(s));
+    }
+  }
   float ms = 0.f;
   FLK_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   ctx->stats.ms_kernel = ms;

@@ -98,7 +98,8 @@ typedef struct flk_stats {
                                (per-launch timing, or the device-scheduled pass's
                                buffers overflowed) instead of all levels enqueued at once */
   int64_t graph_launches;   /* Barnes–Hut certificates run as one captured HIP graph (params.graph:
-                               the direct-sum part, every tree build and both traversal passes);
+                               the direct-sum part, every tree build and the traversal passes; with
+                               one batch its re-runs, when there are any, are a second graph);
                                their device time is ms_kernel, and ms_bh_build/ms_bh_traverse
                                stay 0 */
   double ms_graph_launch;   /* host time of that hipGraphLaunch call */

@@ -64,13 +64,11 @@ namespace {
 constexpr float kInv2PiF = 0.15915494309189533577f;
 constexpr float kInv4PiF = 0.07957747154594766788f;
 
-__device__ __forceinline__ uint64_t spread16(uint64_t v) {
-  v &= 0xffff;
-  v = (v | (v << 16)) & 0x0000ff0000ffULL;
-  v = (v | (v << 8)) & 0x00f00f00f00fULL;
-  v = (v | (v << 4)) & 0x0c30c30c30c3ULL;
-  v = (v | (v << 2)) & 0x249249249249ULL;
-  return v;
+__device__ __forceinline__ uint32_t spread10(uint32_t v) {  // bits of v to every third place
+  v = (v | (v << 16)) & 0x030000ffu;
+  v = (v | (v << 8)) & 0x0300f00fu;
+  v = (v | (v << 4)) & 0x030c30c3u;
+  return (v | (v << 2)) & 0x09249249u;
 }
 
 // Sort keys of the Barnes–Hut segments, one block per tile of the segmented
@@ -89,8 +87,7 @@ __device__ __forceinline__ uint32_t segment_key(const VP &p, const VP &q, const 
   uint32_t code = 0;
   for (int d = 0; d < 3; ++d) {
     const double u = (m[d] - cb[d]) * cb[3 + d];
-    const uint64_t qd = (uint64_t)fmin(fmax(u, 0.0), 1023.0);
-    code |= (uint32_t)(spread16(qd) << (2 - d));
+    code |= spread10((uint32_t)fmin(fmax(u, 0.0), 1023.0)) << (2 - d);
   }
   return code;
 }
@@ -112,9 +109,9 @@ __global__ __launch_bounds__(256) void bh_keys(const VP *__restrict__ pts, const
   }
 }
 
-// Exclusive scan of one value per thread over a 256-thread block; *total
-// receives the sum.  sw: 4 ints of LDS.  Contains block barriers.
-__device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
+// Exclusive scan of one value per thread over a block of WAVES waves; *total
+// receives the sum.  sw: WAVES ints of LDS.  Contains block barriers.
+template <int WAVES> __device__ __forceinline__ int block_scan(int v, int *total, int *sw) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int inc = v;
 #pragma unroll
@@ -126,7 +123,7 @@ __device__ __forceinline__ int block_scan256(int v, int *total, int *sw) {
   __syncthreads();
   int off = 0, tot = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < WAVES; ++k) {
     off += k < w ? sw[k] : 0;
     tot += sw[k];
   }
@@ -167,7 +164,7 @@ __global__ __launch_bounds__(256) void bh_level_offsets(const int64_t *__restric
     const int32_t k = c0 + threadIdx.x;
     const int v = k < nc ? BhShape((int32_t)(seg_off[k + 1] - seg_off[k]), leaf).nodes(lev, leaf) : 0;
     int tot;
-    const int pos = carry + block_scan256(v, &tot, sw);
+    const int pos = carry + block_scan<4>(v, &tot, sw);
     if (k < nc) loff[(int64_t)lev * nc + k] = pos;
     carry += tot;
   }
@@ -1620,6 +1617,14 @@ __global__ __launch_bounds__(256) void bh_begin(const int32_t *__restrict__ ra, 
 // The copies of one sum, added in order.
 __device__ __forceinline__ double fold_copies(const double *p, int copies, int64_t stride) {
   double v = p[0];
+  if (copies == 8) {  // a walk's, in flight at once
+    double u[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) u[k] = p[(k + 1) * stride];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) v += u[k];
+    return v;
+  }
   for (int k = 1; k < copies; ++k) v += p[k * stride];
   return v;
 }
@@ -1634,22 +1639,25 @@ __device__ __forceinline__ double fold_copies(const double *p, int copies, int64
 // and compacts the re-runs with a block scan, so the list is deterministic:
 // root items (pair = position in the list), beta^2, and every pair's position
 // in it (-1: not re-run).  Sets the second pass's root count.
-__global__ __launch_bounds__(256) void bh_adapt(int64_t nb, const int32_t *__restrict__ ra,
+__global__ __launch_bounds__(1024) void bh_adapt(int64_t nb, const int32_t *__restrict__ ra,
                                                 const int32_t *__restrict__ rb, const double *__restrict__ err1,
                                                 int copies, int64_t copy_stride, int mlp, double err_scale,
                                                 double target_error, double beta_init, double beta_limit,
                                                 BhItem *__restrict__ items2, float *__restrict__ beta2_2,
                                                 int32_t *__restrict__ redo, unsigned long long *__restrict__ n_redo) {
-  __shared__ int sw[4];
+  __shared__ int sw[16];
   int carry = 0;
-  for (int64_t c0 = 0; c0 < nb; c0 += 256) {
+  for (int64_t c0 = 0; c0 < nb; c0 += 1024) {
     const int64_t t = c0 + threadIdx.x;
     int flag = 0;
     float b2 = 0.f;
     const double e1 = t < nb ? fold_copies(err1 + t, copies, copy_stride) : 0.0;
     if (t < nb) {
-      if (!mlp) {
-        const double want = pow(e1 * err_scale / target_error, 0.25) * beta_init;
+      const double excess = e1 * err_scale / target_error;
+      if (!mlp && excess < 0.99 && beta_init > 0.0) {
+        // a fourth root below 1: the target lies below beta_init, without the pow
+      } else if (!mlp) {
+        const double want = pow(excess, 0.25) * beta_init;
         const double target = beta_limit < want ? beta_limit : want;  // std::min: a NaN estimate stays NaN
         if (target > beta_init) {
           flag = 1;
@@ -1661,7 +1669,7 @@ __global__ __launch_bounds__(256) void bh_adapt(int64_t nb, const int32_t *__res
       }
     }
     int tot = 0;
-    const int pos = carry + block_scan256(flag, &tot, sw);
+    const int pos = carry + block_scan<16>(flag, &tot, sw);
     if (flag) {
       items2[pos] = BhItem{pos, ra[t], rb[t], 0};
       beta2_2[pos] = b2;
@@ -2550,7 +2558,7 @@ void enqueue_adapt(flk_ctx *ctx, const BatchPlan &bp, const flk_params &prm, uns
                    hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size();
-  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(256), 0, s, nb, bp.d_ra, bp.d_rb,
+  hipLaunchKernelGGL(bh_adapt, dim3(1), dim3(1024), 0, s, nb, bp.d_ra, bp.d_rb,
                      (const double *)B.err.as<double>(), bp.shape.copies,
                      2 * nb, prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, prm.target_error, prm.beta_init,
                      prm.beta_limit, B.items0.as<BhItem>(), B.beta2.as<float>() + nb, B.redo.as<int32_t>(), n_redo);

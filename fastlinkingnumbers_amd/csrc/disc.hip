@@ -174,7 +174,7 @@ __device__ __forceinline__ int curve_of(const DCurve *__restrict__ cs, int nc, i
 // One piece per segment: (curve, segment, 0, 1), its box and diagonal.
 // Also reduced per block: the sum of the segments' first points' norms, the
 // first smallest box diagonal and whether any is NaN,
-// so the host reads 32 bytes a block instead of every point and diagonal: with
+// and those by disc_fold, so the host reads 32 bytes instead of every point and diagonal: with
 // the scratch kept between calls, a discretization of 8.8e5 splines took 16.2 ms
 // and takes 2.3.
 struct InitPart {
@@ -182,6 +182,30 @@ struct InitPart {
   int64_t mg;
   int64_t nan;
 };
+__device__ __forceinline__ void fold_part(InitPart &a, const InitPart &b) {
+  a.sum += b.sum;
+  a.nan |= b.nan;
+  if (b.md < a.md || (b.md == a.md && b.mg < a.mg)) {
+    a.md = b.md;
+    a.mg = b.mg;
+  }
+}
+// Thread 0's r becomes the block's (WAVES waves, as many entries of LDS).
+template <int WAVES> __device__ __forceinline__ void fold_block(InitPart &r, InitPart *sp) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    InitPart u;
+    u.sum = __shfl_down(r.sum, o, 64);
+    u.md = __shfl_down(r.md, o, 64);
+    u.mg = __shfl_down(r.mg, o, 64);
+    u.nan = __shfl_down(r.nan, o, 64);
+    fold_part(r, u);
+  }
+  if ((threadIdx.x & 63) == 0) sp[threadIdx.x >> 6] = r;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int k = 1; k < WAVES; ++k) fold_part(r, sp[k]);
+}
 __global__ __launch_bounds__(256) void disc_init(const double *__restrict__ q, const DCurve *__restrict__ cs,
                                                  int32_t nc, int64_t nseg, int32_t *__restrict__ pc,
                                                  int32_t *__restrict__ ps, double *__restrict__ plo,
@@ -207,30 +231,26 @@ __global__ __launch_bounds__(256) void disc_init(const double *__restrict__ q, c
     r.md = d;
     r.mg = g;
   }
-  auto fold = [](InitPart &a, const InitPart &b) {
-    a.sum += b.sum;
-    a.nan |= b.nan;
-    if (b.md < a.md || (b.md == a.md && b.mg < a.mg)) {
-      a.md = b.md;
-      a.mg = b.mg;
-    }
-  };
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    InitPart u;
-    u.sum = __shfl_down(r.sum, o, 64);
-    u.md = __shfl_down(r.md, o, 64);
-    u.mg = __shfl_down(r.mg, o, 64);
-    u.nan = __shfl_down(r.nan, o, 64);
-    fold(r, u);
-  }
   __shared__ InitPart sp[4];
-  if ((threadIdx.x & 63) == 0) sp[threadIdx.x >> 6] = r;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < 4; ++k) fold(r, sp[k]);
-    part[blockIdx.x] = r;
-  }
+  fold_block<4>(r, sp);
+  if (threadIdx.x == 0) part[blockIdx.x] = r;
+}
+
+// The blocks' folded, straight into pinned memory.
+__global__ __launch_bounds__(1024) void disc_fold(const InitPart *__restrict__ part, int64_t n,
+                                                  InitPart *__restrict__ host) {
+  InitPart r{0.0, __builtin_inf(), INT64_MAX, 0};
+  for (int64_t k = threadIdx.x; k < n; k += 1024) fold_part(r, part[k]);
+  __shared__ InitPart sp[16];
+  fold_block<16>(r, sp);
+  if (threadIdx.x == 0) *host = r;
+}
+
+// A round's overlaps and marked pieces into pinned memory.
+__global__ void disc_report(const unsigned long long *__restrict__ cnt, const int32_t *__restrict__ nhit,
+                            unsigned long long *__restrict__ host) {
+  host[0] = cnt[0];
+  host[1] = (unsigned long long)*nhit;
 }
 
 // A node of the implicit tree: its box rounded outward to FP32 (32 bytes
@@ -546,9 +566,20 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
     return threshold_of(sum);
   };
   constexpr double kUnsure = 1e-6;  // far above either sum's rounding
-  FLK_HIP(hipMemcpyAsync(d_cs.ptr, cs.data(), sizeof(DCurve) * nc, hipMemcpyHostToDevice, s));
+  // everything small goes through pinned memory
+  D.host.reserve(sizeof(InitPart) + 2 * sizeof(unsigned long long) + sizeof(uint64_t) * lk.size() +
+                 (sizeof(DCurve) + 3 * sizeof(int32_t)) * (size_t)nc);
+  InitPart *h_part = D.host.as<InitPart>();
+  auto *h_report = reinterpret_cast<unsigned long long *>(h_part + 1);
+  auto *h_links = reinterpret_cast<uint64_t *>(h_report + 2);
+  auto *h_cs = reinterpret_cast<DCurve *>(h_links + lk.size());
+  auto *per_curve = reinterpret_cast<int32_t *>(h_cs + nc);
+  int32_t *open_before = per_curve + nc, *is_open = open_before + nc;
+  std::copy(lk.begin(), lk.end(), h_links);
+  std::copy(cs.begin(), cs.end(), h_cs);
+  FLK_HIP(hipMemcpyAsync(d_cs.ptr, h_cs, sizeof(DCurve) * nc, hipMemcpyHostToDevice, s));
   if (!lk.empty())
-    FLK_HIP(hipMemcpyAsync(d_links.ptr, lk.data(), sizeof(uint64_t) * lk.size(), hipMemcpyHostToDevice, s));
+    FLK_HIP(hipMemcpyAsync(d_links.ptr, h_links, sizeof(uint64_t) * lk.size(), hipMemcpyHostToDevice, s));
   const DCurve *dcs = d_cs.as<DCurve>();
   unsigned long long *cnt = d_cnt.as<unsigned long long>();  // [0] overlaps, [1] too-small flag
 
@@ -588,21 +619,13 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
                        gen[0].s.as<int32_t>(), gen[0].lo.as<double>(), gen[0].hi.as<double>(),
                        gen[0].box.as<PBox>(), D.diag.as<double>(), D.part.as<InitPart>());
     FLK_HIP(hipGetLastError());
-    std::vector<InitPart> part(nb);
-    FLK_HIP(hipMemcpyAsync(part.data(), D.part.ptr, sizeof(InitPart) * nb, hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(disc_fold, dim3(1), dim3(1024), 0, s, (const InitPart *)D.part.as<InitPart>(), nb, h_part);
+    FLK_HIP(hipGetLastError());
     FLK_HIP(hipStreamSynchronize(s));
-    double sum = 0.0, md = std::numeric_limits<double>::infinity();
-    int64_t mg = -1;
-    bool nan = false;
-    for (const InitPart &r : part) {
-      sum += r.sum;
-      nan = nan || r.nan;
-      if (r.md < md) {
-        md = r.md;
-        mg = r.mg;
-      }
-    }
-    threshold = threshold_of(sum) * (1 + kUnsure);
+    double md = h_part->md;
+    int64_t mg = h_part->mg;
+    const bool nan = h_part->nan != 0;
+    threshold = threshold_of(h_part->sum) * (1 + kUnsure);
     // the reference's input guard, in its order (first smallest, NaN taken)
     if (nan) {
       std::vector<double> diag(nseg);
@@ -662,10 +685,12 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
     FLK_HIP(hipMemsetAsync(d_flag.as<int32_t>() + n, 0, sizeof(int32_t), s));
     d_tmp.reserve(scan_temp_bytes(n + 1));
     exclusive_scan(d_flag.as<int32_t>(), d_scan.as<int32_t>(), n + 1, d_tmp.as<int32_t>(), s);
-    int32_t nhit = 0;
-    FLK_HIP(hipMemcpyAsync(&nhit, d_scan.as<int32_t>() + n, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    FLK_HIP(hipMemcpyAsync(host_cnt, cnt, sizeof host_cnt, hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(disc_report, dim3(1), dim3(1), 0, s, cnt, d_scan.as<int32_t>() + n, h_report);
+    FLK_HIP(hipGetLastError());
     FLK_HIP(hipStreamSynchronize(s));
+    const int32_t nhit = (int32_t)h_report[1];
+    host_cnt[0] = h_report[0];
+    host_cnt[1] = 0;
     res.overlaps.push_back((int64_t)host_cnt[0]);
     // bisect the marked pieces, retire the rest
     DiscScratch::Gen &N = gen[cur ^ 1];
@@ -704,7 +729,7 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
   const int R = res.rounds;
   int gbits = 1;
   while (gbits < 32 && ((int64_t)1 << gbits) < nseg) ++gbits;
-  DevBuf &d_k0 = D.k0, &d_k1 = D.k1, &d_i0 = D.i0, &d_i1 = D.i1, &d_i2 = D.i2, &d_ob = D.ob, &d_open = D.open,
+  DevBuf &d_k0 = D.k0, &d_k1 = D.k1, &d_i0 = D.i0, &d_i1 = D.i1, &d_i2 = D.i2, &d_open = D.open,
          &d_out = D.out, &d_per = D.per_curve;
   d_k0.reserve(sizeof(uint64_t) * nret);
   d_k1.reserve(sizeof(uint64_t) * nret);
@@ -730,10 +755,8 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
     radix_sort_pairs<uint32_t>(d_k0.as<uint32_t>(), d_k1.as<uint32_t>(), d_i2.as<uint32_t>(), d_i0.as<uint32_t>(),
                                d_i1.as<uint32_t>(), nret, gbits, d_tmp.ptr, s);
   }
-  std::vector<int32_t> per_curve(nc, 0);
-  FLK_HIP(hipMemcpyAsync(per_curve.data(), d_per.ptr, sizeof(int32_t) * nc, hipMemcpyDeviceToHost, s));
+  FLK_HIP(hipMemcpyAsync(per_curve, d_per.ptr, sizeof(int32_t) * nc, hipMemcpyDeviceToHost, s));
   FLK_HIP(hipStreamSynchronize(s));
-  std::vector<int32_t> open_before(nc, 0), is_open(nc, 0);
   int32_t opens = 0;
   res.out_offsets.assign(nc + 1, 0);
   for (int32_t c = 0; c < nc; ++c) {
@@ -744,14 +767,12 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
   }
   res.retired = nret;
   const int64_t nout = res.out_offsets[nc];
-  d_ob.reserve(sizeof(int32_t) * nc);
-  d_open.reserve(sizeof(int32_t) * nc);
+  d_open.reserve(sizeof(int32_t) * 2 * nc);
   d_out.reserve(sizeof(double) * 3 * std::max<int64_t>(nout, 1));
-  FLK_HIP(hipMemcpyAsync(d_ob.ptr, open_before.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice, s));
-  FLK_HIP(hipMemcpyAsync(d_open.ptr, is_open.data(), sizeof(int32_t) * nc, hipMemcpyHostToDevice, s));
+  FLK_HIP(hipMemcpyAsync(d_open.ptr, open_before, sizeof(int32_t) * 2 * nc, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(disc_points, dim3(blocks_for(nret)), dim3(256), 0, s, q, dcs, d_i1.as<int32_t>(),
                      ret.c.as<int32_t>(), ret.s.as<int32_t>(), ret.lo.as<double>(), ret.hi.as<double>(), nret,
-                     d_ob.as<int32_t>(), d_open.as<int32_t>(), d_out.as<double>());
+                     d_open.as<int32_t>(), d_open.as<int32_t>() + nc, d_out.as<double>());
   FLK_HIP(hipGetLastError());
   if (host_copy) {
     res.xyz.resize(3 * nout);

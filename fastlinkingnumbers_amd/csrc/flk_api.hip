@@ -78,11 +78,11 @@ void curves_clear(flk_ctx *ctx) {
   ctx->cert_graph.reset();
 }
 
-void curves_finish(flk_ctx *ctx) {
+void curves_finish(flk_ctx *ctx, const float *land) {
   Curves &cv = ctx->curves;
   const int32_t ncurves = cv.ncurves;
   hipStream_t s = ctx->stream;
-  curve_boxes_run(ctx, cv.box);
+  curve_boxes_run(ctx, cv.box, land);
   // Origin and power-of-two scale: stored = (x - origin) * scale with the
   // model extent near 1.  The origin stays 0 unless the model is far from it
   // (then it is snapped to a coarse grid so fp32 inputs remain exact).
@@ -274,8 +274,9 @@ int32_t flk_set_curves(flk_ctx *ctx, const double *xyz, const int64_t *offsets, 
     try {
       const int64_t nv = flk::curves_layout(ctx, offsets, ncurves);
       flk::Curves &cv = ctx->curves;
-      flk::ingest_points(ctx, xyz, false, nv, cv.raw.as<double>(), cv.hi.as<float>(), cv.hi.bytes);
-      flk::curves_finish(ctx);
+      bool landed;
+      flk::ingest_points(ctx, xyz, false, nv, cv.raw.as<double>(), cv.hi.as<float>(), cv.hi.bytes, &landed);
+      flk::curves_finish(ctx, landed ? cv.hi.as<float>() : nullptr);
     } catch (...) {
       flk::curves_clear(ctx);  // never leave a half-built curve set behind
       throw;
@@ -292,8 +293,9 @@ int32_t flk_set_curves_f32(flk_ctx *ctx, const float *xyz, const int64_t *offset
     try {
       const int64_t nv = flk::curves_layout(ctx, offsets, ncurves);
       flk::Curves &cv = ctx->curves;
-      flk::ingest_points(ctx, xyz, true, nv, cv.raw.as<double>(), cv.hi.as<float>(), cv.hi.bytes);
-      flk::curves_finish(ctx);
+      bool landed;
+      flk::ingest_points(ctx, xyz, true, nv, cv.raw.as<double>(), cv.hi.as<float>(), cv.hi.bytes, &landed);
+      flk::curves_finish(ctx, landed ? cv.hi.as<float>() : nullptr);
     } catch (...) {
       flk::curves_clear(ctx);  // never leave a half-built curve set behind
       throw;

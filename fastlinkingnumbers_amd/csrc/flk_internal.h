@@ -303,7 +303,8 @@ struct DiscScratch {
   } gen[2], ret;
   DevBuf q, land, cs, links, cnt, diag, part;
   DevBuf heap, curve_end, hit, flag, scan, tmp;
-  DevBuf k0, k1, i0, i1, i2, ob, open, out, per_curve;
+  DevBuf k0, k1, i0, i1, i2, open, out, per_curve;
+  HostBuf host;  // pinned: tables on their way to the device, results on their way back
 };
 
 // Scratch of a gradient or a training, kept between calls (grow-only): the set,
@@ -443,17 +444,18 @@ void tree_export(flk_ctx *ctx, int32_t curve, int32_t leaf, std::vector<flk_tree
 
 void pls_run(flk_ctx *ctx, const double *boxes, int32_t ncurves, std::vector<int32_t> &out);
 
-void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes);
+void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes, const float *land);
 // Vertices, their FP32 forms and edges of the current curve set, after
 // curve_boxes_run; true when FP32 cannot hold some coordinate.
 bool stage_vertices_run(flk_ctx *ctx);
 
 // A new curve set: validates the offsets and sizes the device arrays; the
-// caller then fills curves.raw (input FP64 AoS) and calls curves_finish, which
+// caller then fills curves.raw (input FP64 AoS), or has its values in land as
+// FP32, and calls curves_finish, which fills curves.raw from land (if any) and
 // computes the boxes, origin and scale and the staged vertex arrays.  Returns
 // the vertex count.
 int64_t curves_layout(flk_ctx *ctx, const int64_t *offsets, int32_t ncurves);
-void curves_finish(flk_ctx *ctx);
+void curves_finish(flk_ctx *ctx, const float *land = nullptr);
 // Resets to the empty curve set (after a failure part-way through a new one).
 void curves_clear(flk_ctx *ctx);
 
@@ -461,9 +463,10 @@ void curves_clear(flk_ctx *ctx);
 // exactly) to dst (device FP64 AoS) through the pinned staging buffers; land
 // is device scratch for the FP32 copy (>= 12 n bytes).  Enqueued on the
 // context's stream; the host array is no longer read on return.  Returns the
-// bytes sent.
+// bytes sent.  With `landed`, values sent as FP32 stay in land, *landed is set
+// and dst is the caller's to fill (curves_finish does).
 int64_t ingest_points(flk_ctx *ctx, const void *src, bool src_f32, int64_t n, double *dst, float *land,
-                      size_t land_bytes);
+                      size_t land_bytes, bool *landed = nullptr);
 // dst[i] = (double)land[i], i < nval, on the context's stream.
 void widen_launch(flk_ctx *ctx, const float *land, int64_t nval, double *dst);
 

@@ -88,7 +88,8 @@ int ingest_workers(const flk_ctx *ctx) {
 }
 
 int64_t ingest_points(flk_ctx *ctx, const void *src, bool src_f32, int64_t n, double *dst, float *land,
-                      size_t land_bytes) {
+                      size_t land_bytes, bool *landed) {
+  if (landed) *landed = false;
   if (n <= 0) return 0;
   hipStream_t s = ctx->stream;
   HostStage &st = ctx->stage;
@@ -157,7 +158,8 @@ int64_t ingest_points(flk_ctx *ctx, const void *src, bool src_f32, int64_t n, do
       for (auto &p : st.pending) p = 0;
       continue;
     }
-    if (wire_f32) widen_launch(ctx, land, nval, dst);
+    if (wire_f32 && landed) *landed = true;
+    else if (wire_f32) widen_launch(ctx, land, nval, dst);
     return (int64_t)esz * nval;
   }
   return 0;  // not reached
@@ -168,7 +170,7 @@ int64_t ingest_points(flk_ctx *ctx, const void *src, bool src_f32, int64_t n, do
 // FP32 xyz triples.  The coordinates are read straight into the pinned
 // staging buffers, the counts stripped on the way, and each full buffer is
 // sent while the next one is read; once the counts are known the curve set is
-// laid out and the FP32 array widened on the device.
+// laid out and the FP32 array widened by the pass that takes the boxes.
 void load_bcc(flk_ctx *ctx, const char *path, BccLoad &out) {
   out = BccLoad{};
   std::FILE *f = std::fopen(path, "rb");
@@ -261,8 +263,7 @@ void load_bcc(flk_ctx *ctx, const char *path, BccLoad &out) {
   // the curve set: layout from the counts, then the FP32 array widened
   try {
     curves_layout(ctx, out.offsets.data(), nc);
-    widen_launch(ctx, reinterpret_cast<const float *>(land), 3 * out.points, ctx->curves.raw.as<double>());
-    curves_finish(ctx);
+    curves_finish(ctx, reinterpret_cast<const float *>(land));
   } catch (...) {
     curves_clear(ctx);
     throw;

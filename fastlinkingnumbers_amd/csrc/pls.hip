@@ -42,9 +42,14 @@ __device__ __forceinline__ bool box_overlap(const Box6 &a, const Box6 &b) {
 // over the whole chip; where every curve is one chunk the first pass is all.
 // The boxes also go to pinned memory (`host`) without a copy, and the last pass
 // clears the flag that stage_vertices sets.
-constexpr int64_t kBoxChunk = 16384;
+constexpr int64_t kBoxChunk = 4096;
 
-__global__ __launch_bounds__(256) void curve_box_chunks(const double *__restrict__ xyz,
+// Coordinates that came as FP32 are read there and written to xyz as FP64 on the
+// way (a pass of its own read and wrote them again: 215 us for 3.1e7 vertices).
+// A block of 1,024 threads with four vertices each in flight: for a few curves of
+// thousands of vertices the pass is as long as one chunk.
+template <bool LANDED>
+__global__ __launch_bounds__(1024) void curve_box_chunks(double *__restrict__ xyz, const float *__restrict__ land,
                                                         const int64_t *__restrict__ chunk_v,
                                                         double *__restrict__ part, double *__restrict__ host,
                                                         int32_t *__restrict__ inexact) {
@@ -52,15 +57,24 @@ __global__ __launch_bounds__(256) void curve_box_chunks(const double *__restrict
   if (host && c == 0 && threadIdx.x == 0) *inexact = 0;
   const int64_t v0 = chunk_v[2 * c], v1 = chunk_v[2 * c + 1];
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  for (int64_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
+  for (int64_t base = v0 + threadIdx.x; base < v1; base += 4 * 1024) {
+    double x[4][3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const double x = xyz[3 * v + d];
-      mn[d] = fmin(mn[d], x);
-      mx[d] = fmax(mx[d], x);
+    for (int k = 0; k < 4; ++k) {
+      const int64_t v = min(base + 1024 * k, v1 - 1);  // the last again past the end
+#pragma unroll
+      for (int d = 0; d < 3; ++d) x[k][d] = LANDED ? (double)land[3 * v + d] : xyz[3 * v + d];
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if (LANDED && base + 1024 * k < v1) xyz[3 * (base + 1024 * k) + d] = x[k][d];
+        mn[d] = fmin(mn[d], x[k][d]);
+        mx[d] = fmax(mx[d], x[k][d]);
+      }
   }
-  __shared__ double smn[3][4], smx[3][4];
+  __shared__ double smn[3][16], smx[3][16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -448,7 +462,7 @@ void pls_small(flk_ctx *ctx, const double *d_boxes, int32_t n, std::vector<int32
 
 }  // namespace
 
-void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes) {
+void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes, const float *land) {
   Curves &cv = ctx->curves;
   const size_t nc = (size_t)cv.ncurves;
   boxes.assign(6 * nc, 0.0);
@@ -492,7 +506,8 @@ void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes) {
   const int64_t *d_coff = ctx->d_misc.as<int64_t>() + 2 * (nc + 1), *d_chunk = d_coff + nc + 1;
   int32_t *flag = ctx->d_count.as<int32_t>();
   if (nchunks > 0)
-    hipLaunchKernelGGL(curve_box_chunks, dim3((unsigned)nchunks), dim3(256), 0, s, cv.raw.as<double>(), d_chunk,
+    hipLaunchKernelGGL(land ? curve_box_chunks<true> : curve_box_chunks<false>, dim3((unsigned)nchunks), dim3(1024), 0,
+                       s, cv.raw.as<double>(), land, d_chunk,
                        single ? d_boxes : d_part, single ? host : (double *)nullptr, flag);
   if (!single)
     hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, d_part, d_coff,

@@ -44,3 +44,22 @@ def test_one_block_search_is_every_overlapping_pair(engine, n):
         i, j = np.triu_indices(n, 1)
         near = np.all((boxes[i, :3] <= boxes[j, 3:]) & (boxes[j, :3] <= boxes[i, 3:]), axis=1)
         assert np.array_equal(engine.potential_links(boxes), np.stack([i[near], j[near]], 1)), size
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("sizes", [[4096, 0, 4095, 1], [4097, 1, 0, 8193], [1024, 1025, 3]], ids=str)
+def test_boxes_around_a_chunk(engine, sizes, dtype):
+    """Curves within and beyond one chunk of 4,096 vertices, in whole and part
+    rounds of a block's 1,024 threads; extrema at the ends."""
+    rng = np.random.default_rng(sum(sizes))
+    packed = rng.normal(size=(sum(sizes), 3)).astype(dtype)
+    offsets = np.concatenate([[0], np.cumsum(sizes)])
+    for a, b in zip(offsets[:-1], offsets[1:]):
+        if b > a:
+            packed[a], packed[b - 1] = -9, 9
+    engine.set_curves_packed(packed, offsets)
+    boxes = engine.curve_boxes()
+    for k, (a, b) in enumerate(zip(offsets[:-1], offsets[1:])):
+        if b > a:
+            v = packed[a:b].astype(np.float64)
+            assert np.array_equal(boxes[k], np.concatenate([v.min(0), v.max(0)])), k

@@ -265,12 +265,14 @@ __global__ __launch_bounds__(256) void bh_stage_segments(const uint32_t *__restr
 
 // Keys, sort and (sp not null) staged end points of a curve of at most CAP
 // segments in one block, list[b] its rank: the same order as the segmented
-// sort's.  Key and place make one number, so every two differ: each wave sorts
-// runs of 64 across its lanes, and runs are merged by each element finding its
-// place in the other run, a thread's E elements side by side.  Bound by latency,
+// sort's.  Each wave sorts runs of 64 across its lanes, key and place as one
+// number, and runs are merged by each element finding its place in the other run
+// by its key alone (a left run's places are all below the right one's: an element
+// of the right follows the left's equal keys), a thread's E elements side by side
+// in 6 bytes of LDS each.  Bound by latency,
 // as the segmented sort's 14-18 launches are, which took 110 us for ten curves of
-// 24,000 segments and 165 for 400 of 4e5: 42 and 41 here, sorted within 64 bits
-// of LDS a segment.  8,192 is what 64 KB hold, two blocks a CU.
+// 24,000 segments and 165 for 400 of 4e5: 37 and 36 here (43 and 42 with a branch
+// for each of a thread's elements).  8,192 takes 48 KB, two blocks a CU.
 constexpr int kSmallSorts = 3;
 constexpr int kSmallSort[kSmallSorts] = {1024, 4096, 8192}, kSmallThreads[kSmallSorts] = {256, 1024, 1024};
 template <typename SP, typename VP, int THREADS, int CAP>
@@ -283,64 +285,92 @@ __global__ __launch_bounds__(THREADS) void bh_sort_small(const VP *__restrict__ 
   constexpr int E = CAP / THREADS;
   constexpr int kPlaceBits = 13;
   static_assert(CAP <= 1 << kPlaceBits && THREADS % 64 == 0, "places fit, whole waves");
-  __shared__ uint64_t a[CAP];
+  __shared__ uint32_t keys[CAP];
+  __shared__ uint16_t places[CAP];
   const int c = list[blockIdx.x], lane = threadIdx.x & 63;
   const int64_t g0 = seg_off[c], v0 = vtx_off[c];
   const int n = (int)(seg_off[c + 1] - g0), padded = (n + 63) / 64 * 64;
-  const int sets = max(0, (n - ((int)threadIdx.x - lane) + THREADS - 1) / THREADS);  // of 64, this wave's
-  uint64_t x[E];
+  // sets of 64 segments, this wave's
+  const int sets = __builtin_amdgcn_readfirstlane(max(0, (n - ((int)threadIdx.x - lane) + THREADS - 1) / THREADS));
+  // a wave with one set takes the code for one, any other that for E: without a
+  // branch for each set the sets' exchanges and searches overlap
+  auto sort_runs = [&](auto count) {
+    constexpr int N = decltype(count)::value;
+    uint64_t x[N];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int i = e * THREADS + (int)threadIdx.x;
-    x[e] = 1ull << (30 + kPlaceBits) | (uint64_t)i;  // behind every segment
-    if (i < n) x[e] = (uint64_t)segment_key(pts[v0 + i], pts[v0 + i + 1], cbox + 6 * c) << kPlaceBits | (uint64_t)i;
-  }
-#pragma unroll
-  for (int k = 2; k <= 64; k <<= 1)
-#pragma unroll
-    for (int d = k / 2; d > 0; d >>= 1) {
-      const bool low = ((lane & d) == 0) == ((lane & k) == 0);  // keeps the smaller
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        if (e >= sets) break;
-        const uint64_t y = __shfl_xor(x[e], d, 64);
-        x[e] = (x[e] < y) == low ? x[e] : y;
-      }
+    for (int e = 0; e < N; ++e) {
+      const int i = e * THREADS + (int)threadIdx.x;
+      x[e] = 1ull << (30 + kPlaceBits) | (uint64_t)i;  // behind every segment
+      if (i < n) x[e] = (uint64_t)segment_key(pts[v0 + i], pts[v0 + i + 1], cbox + 6 * c) << kPlaceBits | (uint64_t)i;
     }
 #pragma unroll
-  for (int e = 0; e < E; ++e)
-    if (e < sets) a[e * THREADS + (int)threadIdx.x] = x[e];
+    for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+      for (int d = k / 2; d > 0; d >>= 1) {
+        const bool low = ((lane & d) == 0) == ((lane & k) == 0);  // keeps the smaller
+        uint64_t y[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) y[e] = __shfl_xor(x[e], d, 64);
+#pragma unroll
+        for (int e = 0; e < N; ++e) x[e] = (x[e] < y[e]) == low ? x[e] : y[e];
+      }
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+      if (e < sets) {
+        keys[e * THREADS + (int)threadIdx.x] = (uint32_t)(x[e] >> kPlaceBits);
+        places[e * THREADS + (int)threadIdx.x] = (uint16_t)(x[e] & ((1u << kPlaceBits) - 1));
+      }
+  };
+  uint32_t key[E];
+  uint16_t place[E];
+  int to[E];  // the element's place in the merged run
+  auto find = [&](auto count, int run) {
+    constexpr int N = decltype(count)::value;
+    int start[N], len[N], before[N];  // the other run, and how many of it go before
+    uint32_t below[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const int i = min(e * THREADS + (int)threadIdx.x, padded - 1);
+      start[e] = min((i & ~(run - 1)) ^ run, padded);
+      len[e] = min(padded - start[e], run);
+      before[e] = 0;
+      key[e] = keys[i];
+      place[e] = places[i];
+      below[e] = key[e] + ((i & run) ? 1u : 0u);
+      to[e] = (i & ~(2 * run - 1)) + (i & (run - 1));
+    }
+    for (int h = run; h > 0; h >>= 1) {
+      uint32_t k[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) k[e] = keys[min(start[e] + before[e] + h, padded) - 1];
+#pragma unroll
+      for (int e = 0; e < N; ++e) before[e] += before[e] + h <= len[e] && k[e] < below[e] ? h : 0;
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) to[e] += before[e];
+  };
+  using One = std::integral_constant<int, 1>;
+  using All = std::integral_constant<int, E>;
+  if (sets == 1) sort_runs(One{});
+  else if (sets) sort_runs(All{});
   for (int run = 64; run < n; run *= 2) {
     __syncthreads();
-    int start[E], len[E], to[E];  // the other run, and how many of it are smaller
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int i = e * THREADS + (int)threadIdx.x;
-      const int other = min((i & ~(run - 1)) ^ run, padded);
-      start[e] = other;
-      len[e] = min(padded - other, run);
-      to[e] = 0;
-      if (e < sets) x[e] = a[i];
-    }
-    for (int h = run; h > 0; h >>= 1)
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        if (e >= sets) break;
-        if (to[e] + h <= len[e] && a[start[e] + to[e] + h - 1] < x[e]) to[e] += h;
-      }
+    if (sets == 1) find(One{}, run);
+    else if (sets) find(All{}, run);
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int i = e * THREADS + (int)threadIdx.x;
-      if (e < sets) a[(i & ~(2 * run - 1)) + (i & (run - 1)) + to[e]] = x[e];
-    }
+    for (int e = 0; e < E; ++e)
+      if (e < sets) {
+        keys[to[e]] = key[e];
+        places[to[e]] = place[e];
+      }
   }
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int i = e * THREADS + (int)threadIdx.x;
     if (i >= n) continue;
-    const int64_t v = v0 + (int64_t)(a[i] & ((1u << kPlaceBits) - 1));
+    const int64_t v = v0 + places[i];
     order[g0 + i] = (uint32_t)v;
     if (sp) stage_segment(pts[v], pts[v + 1], sp + 3 * (g0 + i));
   }

@@ -494,6 +494,15 @@ void discretize_run(flk_ctx *ctx, const double *ctrl, const int64_t *offsets, co
                     bool host_copy) {
   hipStream_t s = ctx->stream;
   DiscScratch &D = ctx->disc_scratch;
+  struct GiveBack {
+    DiscScratch &D;
+    hipStream_t s;
+    ~GiveBack() {
+      if (D.bytes() <= DiscScratch::kKept) return;
+      (void)hipStreamSynchronize(s);
+      D = DiscScratch{};
+    }
+  } give_back{D, s};
   res = DiscResult{};
   // curves and their segments
   std::vector<DCurve> cs(nc);

@@ -296,7 +296,7 @@ struct DiscResult {
   double small_size = 0.0;
 };
 
-// Scratch of a discretization, kept by the context between calls (grow-only).
+// Scratch of a discretization, kept by the context between calls.
 struct DiscScratch {
   struct Gen {  // pieces: curve, segment, parameter range, box
     DevBuf c, s, lo, hi, box;
@@ -305,6 +305,16 @@ struct DiscScratch {
   DevBuf heap, curve_end, hit, flag, scan, tmp;
   DevBuf k0, k1, i0, i1, i2, open, out, per_curve;
   HostBuf host;  // pinned: tables on their way to the device, results on their way back
+  static constexpr size_t kKept = size_t(1) << 30;  // more is given back after the call
+  size_t bytes() const {
+    size_t n = 0;
+    for (const Gen *g : {&gen[0], &gen[1], &ret})
+      for (const DevBuf *b : {&g->c, &g->s, &g->lo, &g->hi, &g->box}) n += b->bytes;
+    for (const DevBuf *b : {&q, &land, &cs, &links, &cnt, &diag, &part, &heap, &curve_end, &hit, &flag, &scan, &tmp, &k0,
+                            &k1, &i0, &i1, &i2, &open, &out, &per_curve})
+      n += b->bytes;
+    return n;
+  }
 };
 
 // Scratch of a gradient or a training, kept between calls (grow-only): the set,

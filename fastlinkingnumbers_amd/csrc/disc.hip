@@ -346,8 +346,9 @@ __global__ __launch_bounds__(256) void disc_query(const FBox *__restrict__ heap,
             k *= 2;
             continue;
           }
+          // (a box of all FP32 numbers overlaps the padding behind the last piece too)
           const int64_t o = (int64_t)k - L;
-          if (overlap(pbox[o], me) && linked(links, nlinks, c, pc[o])) {
+          if (o < n && overlap(pbox[o], me) && linked(links, nlinks, c, pc[o])) {
             ++found;
             hit[i] = 1;
             hit[o] = 1;

@@ -1,0 +1,38 @@
+"""The discretization's walk for overlapping pieces: what it finds does not
+depend on where the model lies, how large it is, or the curves' order."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+flk = pytest.importorskip("fastlinkingnumbers_amd")
+
+pytestmark = pytest.mark.gpu
+
+
+def _polygons(na, nb):
+    """Two linked polygons whose first segments each span most of the model on
+    every axis, 0.4 apart where they cross."""
+    a = np.array([[-1, -1, -1], [1, 1, 1]], float)
+    b = np.array([[-1, 1, 0.8], [1, -1, -1.1]], float) + [0.3, 0.3, 0]
+    arc = lambda p, q, n, bend: [p + (q - p) * t + bend * np.sin(np.pi * t)  # noqa: E731
+                                 for t in np.arange(n) / n]
+    return [np.array([a[0], *arc(a[1], a[0], na - 1, np.array([2.0, -2.0, 0.3]))]),
+            np.array([b[0], *arc(b[1], b[0], nb - 1, np.array([-1.5, -1.5, 0.4]))])]
+
+
+# numbers of pieces that are not powers of two, so the tree has padding; beyond
+# 2^128 a box that holds the origin is every FP32 number once rounded outward
+@pytest.mark.parametrize("na,nb", [(3, 4), (5, 6), (60, 201)])
+def test_models_beyond_fp32(engine, na, nb):
+    curves = _polygons(na, nb)
+    ref = O.Model.from_curves(curves).discretize().curves()
+    unit, du = engine.discretize(curves, flk.SEG_POLYLINE, True, [[0, 1]])
+    assert du["rounds"] > 1 and du["overlaps"][0] > 0 and du["overlaps"][-1] == 0
+    assert [len(c) for c in unit] == [len(c) for c in ref]
+    for u, r in zip(unit, ref):
+        np.testing.assert_allclose(u, r, rtol=0, atol=1e-12)
+    big, db = engine.discretize([2.0 ** 130 * c for c in curves], flk.SEG_POLYLINE, True, [[0, 1]])
+    assert db == du
+    for u, b in zip(unit, big):  # a power of two changes no rounding
+        np.testing.assert_array_equal(b, 2.0 ** 130 * u)

@@ -368,6 +368,19 @@ __device__ __forceinline__ double atan_short_f64(double zi, double zr) {
   return fma(t * s, p, t);
 }
 
+// What 1/16 x' - |y'| has to exceed on the short path.  It multiplies four x', up
+// to 16 r^6 each for vectors of length r, so curves whose vectors may be
+// longer than 1e11 (pairs that no search finds, their boxes being far apart)
+// always take the general path.  p0, q0: the curves' first vertices, with their
+// boxes' diagonals.
+__device__ __forceinline__ double short_path_limit(const double4 &p0, const double4 &q0) {
+  const double x = q0.x - p0.x, y = q0.y - p0.y, z = q0.z - p0.z;
+  const double longest = sqrt(x * x + y * y + z * z) + p0.w + q0.w;
+  const double limit = longest < 1e11 ? 1e-28 : __builtin_inf();
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(limit)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(limit)));  // the wave's, in scalar registers
+}
+
 template <int R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void ds_tile_f64(
     const double4 *__restrict__ pts, const DsPair *__restrict__ pairs,
@@ -414,6 +427,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
     };
     const double4 *__restrict__ cpt = pts + pr.off_c;
     const int ncl = pr.n_c;
+    const double limit = short_path_limit(rows[0], cpt[0]);
     double an[R + 1], al[R + 1], acol[R];
     double bn[R + 1], bl[R + 1], bcol[R];
     double qx, qy, qz;  // the previous column's vertex
@@ -476,7 +490,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
         // no branch correction, |y'/x'| <= 1/16, and x' clear of the rounding
         // noise of vertices that (nearly) touch: their denominators are at
         // most ~1e-16 each (relative vectors are at most 1 long), x' ~1e-32
-        small = small && (s12 > 0.0) && (fma(0.0625, xp, -fabs(yp)) > 1e-28);
+        small = small && (s12 > 0.0) && (fma(0.0625, xp, -fabs(yp)) > limit);
         if (k == 0) {
           yr = xp;
           yi = yp;

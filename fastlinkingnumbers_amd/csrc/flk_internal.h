@@ -171,7 +171,8 @@ struct Curves {
   double scale = 1.0;            // power of two
   std::vector<int64_t> in_off;   // input offsets
   DevBuf raw;                    // input FP64 AoS (no closing vertex)
-  DevBuf dpts;                   // double4 per vertex, shifted+scaled, +1 closing vertex per curve
+  DevBuf dpts;                   // double4 per vertex, shifted+scaled, +1 closing vertex per curve; the
+                                 // fourth of a curve's first: its box's diagonal, scaled
   DevBuf hi, lo, ed;             // float4 per vertex (+1 closing vertex per curve)
   int64_t nvert_dev = 0;
   bool inexact = false;          // some stored coordinate needs the FP32 lo part

@@ -134,12 +134,14 @@ __global__ __launch_bounds__(256) void curve_box_merge(const double *__restrict_
 // Device vertex v (curve c, local index l <= n_c) takes input vertex l, or
 // vertex 0 for the closing copy l == n_c; coordinates are (x - origin) * scale.
 // Beside the FP64 vertex go its FP32 hi/lo split and the FP32 edge to the next
-// vertex of the array (the FP64 difference rounded, with -|edge|^2 / 2); any
+// vertex of the array (the FP64 difference rounded, with -|edge|^2 / 2), and
+// with a curve's first vertex the scaled diagonal of its box; any
 // vertex that FP32 cannot hold sets the flag.  One pass instead of a second over
 // the FP64 vertices: 3.1e7 vertices took 523 + 433 us in two.
 __global__ __launch_bounds__(256) void stage_vertices(const double *__restrict__ xyz,
                                                       const int64_t *__restrict__ in_off,
                                                       const int64_t *__restrict__ dev_off,
+                                                      const double *__restrict__ boxes,
                                                       int32_t ncurves, int64_t ndev, double ox,
                                                       double oy, double oz, double scale,
                                                       double4 *__restrict__ out, float4 *__restrict__ hi,
@@ -162,7 +164,12 @@ __global__ __launch_bounds__(256) void stage_vertices(const double *__restrict__
       return make_double4((p[0] - ox) * scale, (p[1] - oy) * scale, (p[2] - oz) * scale, 0.0);
     };
     const int64_t l = v - dev_off[c];
-    const double4 p = staged(c, l);
+    double4 p = staged(c, l);
+    if (l == 0 && in_off[c + 1] > in_off[c]) {
+      const double *b = boxes + 6 * (int64_t)c;
+      const double dx = (b[3] - b[0]) * scale, dy = (b[4] - b[1]) * scale, dz = (b[5] - b[2]) * scale;
+      p.w = sqrt(dx * dx + dy * dy + dz * dz);
+    }
     out[v] = p;
     const float hx = (float)p.x, hy = (float)p.y, hz = (float)p.z;
     const float lx = (float)(p.x - (double)hx), ly = (float)(p.y - (double)hy), lz = (float)(p.z - (double)hz);
@@ -522,7 +529,7 @@ bool stage_vertices_run(flk_ctx *ctx) {
   const int64_t blocks = (cv.nvert_dev + 255) / 256;
   const int64_t *d_in = ctx->d_misc.as<int64_t>();
   hipLaunchKernelGGL(stage_vertices, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, cv.raw.as<double>(), d_in,
-                     d_in + cv.ncurves + 1, cv.ncurves, cv.nvert_dev, cv.origin[0], cv.origin[1], cv.origin[2],
+                     d_in + cv.ncurves + 1, ctx->d_boxes.as<double>(), cv.ncurves, cv.nvert_dev, cv.origin[0], cv.origin[1], cv.origin[2],
                      cv.scale, cv.dpts.as<double4>(), cv.hi.as<float4>(), cv.lo.as<float4>(), cv.ed.as<float4>(),
                      ctx->d_count.as<int32_t>(), ctx->inexact_host);
   FLK_HIP(hipGetLastError());

@@ -67,3 +67,16 @@ def test_planar_and_touching_curves_keep_their_signs(engine):
     print("got", got, "oracle", O.ds(a, b), O.ds(a, c), O.ds(c, a))
     assert abs(got[0] - O.ds(a, b)) < 1e-12
     assert min(abs(got[1] - O.ds(a, c)), abs(got[1] - O.ds(c, a))) < 1e-12
+
+
+@pytest.mark.parametrize("gap", [1e3, 1e10, 1e11, 3e12, 1e13, 1e15])
+@pytest.mark.parametrize("fp64", [1, 0])
+def test_curves_far_apart_sum_to_zero(engine, gap, fp64):
+    """Pairs that no search would list: the products of four denominators'
+    x', r^24 for vectors of length r, stay finite (in FP32, whose own range ends
+    first, the judge sums in FP64).  64 x 48 angles of at most 0.02 / r^2."""
+    a = _ring(64, [0, 0, 0], 0.0, 0.05, 1)
+    b = _ring(48, [gap, 0.3 * gap, -gap], 1.1, 0.05, 2)
+    engine.set_curves([a, b])
+    got = engine.linking_numbers([[0, 1]], method="directsum", fp64=fp64).lk[0]
+    assert abs(got) < 3072 * 0.02 / gap ** 2 + 1e-15

@@ -334,7 +334,7 @@ __global__ __launch_bounds__(256) void ds_tile_f32(
 // 175 -> 448 G pairs/s, where every pair took four roots and one library
 // atan2; the sums' error against a 64-bit reference 2.3e-15 -> 1.5e-16, as the
 // triple product comes from the edges instead of three long vectors.  Held to
-// 128 VGPRs, 4 waves per SIMD (the 12 spilled serve the general path): 17.4
+// 128 VGPRs, 4 waves per SIMD (the 14 spilled serve the general path): 17.4
 // ms at 140 and 3 waves; R = 4 at 2 waves takes 15.8 ms but pads the rows of
 // a curve to 256.
 __device__ __forceinline__ double sqrt_refined(double x) {
@@ -368,15 +368,22 @@ __device__ __forceinline__ double atan_short_f64(double zi, double zr) {
   return fma(t * s, p, t);
 }
 
-// What 1/16 x' - |y'| has to exceed on the short path.  It multiplies four x', up
-// to 16 r^6 each for vectors of length r, so curves whose vectors may be
-// longer than 1e11 (pairs that no search finds, their boxes being far apart)
-// always take the general path.  p0, q0: the curves' first vertices, with their
-// boxes' diagonals.
+// What 1/16 x' - |y'| has to exceed on the short path: x' clear of the rounding
+// noise of vertices that (nearly) touch, whose denominators are about 1e-16 of
+// the cubed longest vector each, x' 1e-32 of its sixth power.  Vectors are at
+// most 1 long where a search found the pair, but those of two small curves beside
+// a large one may all be far shorter: at 1e-28 whatever their length, such curves took
+// the general path on every step (two rings 1e-5 of the unit across, 2.7e8
+// pairs: 2.46 ms, 0.79 now, as without the large curve).  The four x' that are
+// multiplied, up to 16 r^6 each for vectors of length r, stay within 1e-69 and
+// 1e68: curves whose vectors may be longer than 1e11 (pairs that no search
+// finds, their boxes being far apart) always take the general path.  p0, q0: the
+// curves' first vertices, with their boxes' diagonals.
 __device__ __forceinline__ double short_path_limit(const double4 &p0, const double4 &q0) {
   const double x = q0.x - p0.x, y = q0.y - p0.y, z = q0.z - p0.z;
   const double longest = sqrt(x * x + y * y + z * z) + p0.w + q0.w;
-  const double limit = longest < 1e11 ? 1e-28 : __builtin_inf();
+  const double r2 = fmin(longest * longest, 1.0);
+  const double limit = longest < 1e11 ? fmax(1e-28 * r2 * r2 * r2, 1e-70) : __builtin_inf();
   return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(limit)),
                           __builtin_amdgcn_readfirstlane(__double2loint(limit)));  // the wave's, in scalar registers
 }
@@ -487,9 +494,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void d
         const double xp = fma(div1, div2, -dt[k] * dt[k]);
         const double s12 = div1 + div2;
         const double yp = dt[k] * s12;
-        // no branch correction, |y'/x'| <= 1/16, and x' clear of the rounding
-        // noise of vertices that (nearly) touch: their denominators are at
-        // most ~1e-16 each (relative vectors are at most 1 long), x' ~1e-32
+        // no branch correction, |y'/x'| <= 1/16, and x' clear of rounding noise
         small = small && (s12 > 0.0) && (fma(0.0625, xp, -fabs(yp)) > limit);
         if (k == 0) {
           yr = xp;

@@ -80,3 +80,33 @@ def test_curves_far_apart_sum_to_zero(engine, gap, fp64):
     engine.set_curves([a, b])
     got = engine.linking_numbers([[0, 1]], method="directsum", fp64=fp64).lk[0]
     assert abs(got) < 3072 * 0.02 / gap ** 2 + 1e-15
+
+
+@pytest.mark.parametrize("radius", [1.0, 1e-2, 1e-3, 1e-5, 1e-7, 1e-9])
+def test_small_curves_beside_a_large_one(engine, radius):
+    """The short path's limit follows the pair's own size, not that of the
+    model's largest curve (radius 500): the sums keep the tolerance above."""
+    a = radius * _ring(600, [0, 0, 0], 0.0, 0.07, 1)
+    b = radius * _ring(511, [0.9, 0.1, 0.2], 1.3, 0.05, 2)
+    c = radius * _ring(300, [2.0 + 1e-5, 0, 0], np.pi / 2, 0.0, 3)  # passes a at about 0.01 of its size
+    engine.set_curves([a, b, c, 500 * _ring(64, [0, 0, 0], 0.0, 0.0, 4)])
+    got = engine.linking_numbers([[0, 1], [0, 2]], method="directsum", fp64=1).lk
+    ref = [O.ds(a, b), O.ds(a, c)]
+    print(radius, "got", got, "oracle", ref)
+    assert np.abs(got - ref).max() < 1e-12
+
+
+def test_small_curves_take_no_longer_beside_a_large_one(engine):
+    """The general path on every step took 3.1 times as long."""
+    ring = [1e-2 * _ring(16384, [x, 0, 0], tilt, 0.05, 1) for x, tilt in ((0, 0.0), (0.9, 1.3))]
+    large = 500 * _ring(64, [0, 0, 0], 0.0, 0.0, 4)
+    ms = []
+    for curves in (ring, ring + [large]):
+        engine.set_curves(curves)
+        times = []
+        for _ in range(5):
+            engine.linking_numbers([[0, 1]], method="directsum", fp64=1)
+            times.append(engine.stats()["ms_ds_kernel"])
+        ms.append(min(times))
+    print("alone, beside", ms)
+    assert ms[1] < 1.6 * ms[0]

@@ -1194,8 +1194,8 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // ended, a wave still at work leaves its stack to the next round within
 // kWalkSteps steps, so a round ends with the chip full, and the first rounds,
 // whose few items widen twofold a step, take the work to every wave.  The last
-// round leaves nothing (a stack that overflows there fails the pass, as items
-// beyond the queue's capacity do, and the host re-runs the batch).
+// round leaves nothing.  Items beyond the queue's capacity fail the pass, and the
+// host re-runs the batch.
 // Level by level the 2 x depth + 1 launches cost 5-10 us each whatever they do:
 // device time of certificates of ten loops of 2,000-4,000 vertices (10 pairs)
 // 473 -> 336 us, 400 rings of 64-4,096 (1,038 pairs) 1,004 -> 706 us, 2,000
@@ -1209,7 +1209,7 @@ constexpr int kWalkSteps = 8;
 constexpr int kSegs = 64;
 constexpr int kLine = 16;  // words of a counter line (128 bytes)
 
-// Counter words of a pass.  Walked: [4] root items, [6] overflow, and lines of
+// Counter words of a pass.  Walked: [4] root items, and lines of
 // the segments' totals (visits, splits, -, leaf items, leaf segment pairs) and,
 // for each round, of its items, the chunks taken of it and the waves that have
 // ended.  Level by level: [2] leaf segment pairs, [3] network evaluations, [4 +
@@ -1228,6 +1228,9 @@ __host__ __device__ __forceinline__ unsigned long long *seg_round(unsigned long 
 }
 
 constexpr int kStack = 512, kLeaves = 128;
+constexpr int kDepth = 2 * 31;              // two trees of at most 2^30 segments
+constexpr int kWide = kStack - 64;
+static_assert(kWide + kDepth <= kStack, "a walk's stack holds what its newest item adds");
 struct WalkLds {  // a wave's stack (circular) and its leaf pairs waiting to leave
   int p[kStack], a[kStack], b[kStack];
   int lp[kLeaves], la[kLeaves], lb[kLeaves];
@@ -1335,7 +1338,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     }
     // the oldest items go to the next round when the stack could overflow, and
     // all of them kWalkSteps steps after the segment's chunks ran out
-    const int out = last ? 0 : steps <= 0 ? num : num > kStack - 64 ? num / 2 : 0;
+    const int out = last ? 0 : steps <= 0 ? num : num > kWide ? num / 2 : 0;
     if (out) {
       unsigned long long at = 0;
       if (lane == 0) at = atomicAdd(nextq, (unsigned long long)out);
@@ -1349,13 +1352,10 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
       num -= out;
       continue;
     }
-    // (in the last round a stack near its end goes on with its newest item
-    // alone, which adds no more than the trees' levels)
-    if (num > kStack - 2) {
-      if (lane == 0) atomicOr(cnt + 6, 1ull);
-      break;
-    }
-    const int take = num <= kStack - 64 ? min(num, 64) : 1;
+    // In the last round a filling stack narrows the steps: those of several items
+    // leave it at kWide at most, and the newest item alone adds no more than the
+    // splits above a leaf pair, kDepth, before it is done.
+    const int take = last ? max(1, min(min(num, 64), kWide - num)) : min(num, 64);
     num -= take;
     const int base = wrap(bot + num);
     const bool live = lane < take;
@@ -1755,7 +1755,7 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
     x[1] = tot[1];
     x[2] = tot[4];
     x[5] = tot[3];
-    if (c[6] || (int64_t)tot[3] > cap / kSegs) x[6] = 1;
+    if ((int64_t)tot[3] > cap / kSegs) x[6] = 1;
     for (int r = 1; r <= kWalkRounds; ++r)
       if ((int64_t)*seg_round(c, r, seg) > cap / kSegs) x[6] = 1;
   }

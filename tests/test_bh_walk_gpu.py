@@ -68,3 +68,18 @@ def test_overflow_goes_to_the_host(engine):
         for key in COUNTS:
             assert small.stats[key] == base.stats[key], key
         np.testing.assert_allclose(small.lk, base.lk, rtol=0, atol=1e-9)
+
+
+def test_deep_stacks_stay_in_the_walk(engine):
+    """Twenty tangled pairs, 360 node pairs a segment: in the last round the waves'
+    stacks fill to the end and the steps narrow; nothing goes to the host."""
+    curves = []
+    for k in range(20):
+        curves += [c + np.array([100.0 * k, 0, 0]) for c in W.random_walk_pair(seed=k, n=16000, rg=9.0, workload=3)]
+    engine.set_curves(curves)
+    pairs = [[2 * k, 2 * k + 1] for k in range(20)]
+    first = _check(engine, pairs)
+    for _ in range(3):
+        again = engine.linking_numbers(pairs, method="barneshut", fallback_tol=0.0)
+        assert again.stats["bh_host_passes"] == 0
+        np.testing.assert_allclose(again.lk, first.lk, rtol=0, atol=1e-9)

@@ -1204,7 +1204,6 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // 7 ns each on one address), so the queues, the leaf list and their counters
 // come in kSegs segments on lines of their own, one for every 16 blocks, each
 // of one XCD; a round takes its chunks from all segments alike.
-constexpr int kWalkRounds = 6;
 constexpr int kWalkSteps = 8;
 constexpr int kSegs = 64;
 constexpr int kLine = 16;  // words of a counter line (128 bytes)
@@ -1218,8 +1217,8 @@ constexpr int kLine = 16;  // words of a counter line (128 bytes)
 // evaluations, root items, leaf items, overflow.
 constexpr int kPassHead = 8;
 constexpr int kMaxLevels = 1000;
-constexpr int kPassWords = 16 + kLine * kSegs * (2 + kWalkRounds);
-static_assert(kPassWords >= 4 + 2 * (kMaxLevels + 1), "a level pass's counters fit");
+__host__ __device__ __forceinline__ int pass_words(int rounds) { return 16 + kLine * kSegs * (2 + rounds); }
+static_assert(16 + kLine * kSegs * 2 >= 4 + 2 * (kMaxLevels + 1), "a level pass's counters fit");
 __host__ __device__ __forceinline__ unsigned long long *seg_totals(unsigned long long *cnt, int seg) {
   return cnt + 16 + kLine * seg;
 }
@@ -1238,7 +1237,7 @@ struct WalkLds {  // a wave's stack (circular) and its leaf pairs waiting to lea
 
 __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4))) void bh_walk(
     const BhItem *__restrict__ items, int64_t cap, const BhGeo *__restrict__ geo, const BhMom *__restrict__ mom,
-    const float *__restrict__ beta2, float eps, unsigned long long *__restrict__ cnt, int round,
+    const float *__restrict__ beta2, float eps, unsigned long long *__restrict__ cnt, int round, int last,
     BhItem *__restrict__ next, BhItem *__restrict__ leaves, double *__restrict__ psum, double *__restrict__ perr,
     int copies, int64_t copy_stride) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -1271,7 +1270,6 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
   if (w == 0) ends[lane] = end;
   if (threadIdx.x < 2) sh.base[threadIdx.x] = 0;
   __syncthreads();
-  const bool last = round + 1 == kWalkRounds;
   const uint64_t below = (1ull << lane) - 1ull;
   unsigned long long *totals = seg_totals(cnt, seg);
   unsigned long long *taken = seg_round(cnt, round, seg) + 1, *nextq = seg_round(cnt, round + 1, seg);
@@ -1636,11 +1634,11 @@ __global__ void bh_roots(const int32_t *__restrict__ ra, const int32_t *__restri
 // captured), and the first pass's root count.
 __global__ __launch_bounds__(256) void bh_begin(const int32_t *__restrict__ ra, const int32_t *__restrict__ rb,
                                                 int64_t nb, BhItem *__restrict__ items,
-                                                unsigned long long *__restrict__ cnt, int64_t nsums,
+                                                unsigned long long *__restrict__ cnt, int words, int64_t nsums,
                                                 double *__restrict__ sum, double *__restrict__ err) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < nb) items[k] = BhItem{(int32_t)k, ra[k], rb[k], 0};
-  if (k < 2 * kPassWords) cnt[k] = k == 4 ? (unsigned long long)nb : 0ull;
+  if (k < 2 * words) cnt[k] = k == 4 ? (unsigned long long)nb : 0ull;
   if (k < nsums) sum[k] = err[k] = 0.0;
 }
 
@@ -1715,14 +1713,14 @@ __global__ __launch_bounds__(1024) void bh_adapt(int64_t nb, const int32_t *__re
 // second pass's for a re-run pair; sums of the second pass are at + nb.
 // Block 0 makes both device-scheduled passes' kPassHead words of their counters
 // (cnt, null for a host-driven batch; levels: how many a level pass has, 0 when
-// walked), with an overflow noted where a queue or a leaf list is over its
+// walked in `rounds`), with an overflow noted where a queue or a leaf list is over its
 // capacity (its segment's share of it) or items were left after the last level.
 __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__restrict__ redo,
                                                 const double *__restrict__ sum, const double *__restrict__ err,
                                                 int copies, int64_t copy_stride, int mlp, double err_scale,
                                                 double *__restrict__ v, double *__restrict__ e,
                                                 uint32_t *__restrict__ f, unsigned long long *__restrict__ heads,
-                                                unsigned long long *__restrict__ cnt, int64_t cap, int levels) {
+                                                unsigned long long *__restrict__ cnt, int64_t cap, int levels, int rounds) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < nb) {
     const int32_t r = redo[t];
@@ -1734,7 +1732,7 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
   }
   if (cnt == nullptr || blockIdx.x != 0 || threadIdx.x >= 2 * kSegs) return;
   const int seg = threadIdx.x & (kSegs - 1), pass = threadIdx.x / kSegs;
-  unsigned long long *c = cnt + pass * kPassWords;
+  unsigned long long *c = cnt + pass * pass_words(rounds);
   unsigned long long x[kPassHead] = {0, 0, 0, 0, seg == 0 ? c[4] : 0, 0, 0, 0};
   if (levels) {
     for (int d = seg; d <= levels; d += kSegs) {
@@ -1756,7 +1754,7 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
     x[2] = tot[4];
     x[5] = tot[3];
     if ((int64_t)tot[3] > cap / kSegs) x[6] = 1;
-    for (int r = 1; r <= kWalkRounds; ++r)
+    for (int r = 1; r <= rounds; ++r)
       if ((int64_t)*seg_round(c, r, seg) > cap / kSegs) x[6] = 1;
   }
 #pragma unroll
@@ -2268,7 +2266,7 @@ int resident_grid(flk_ctx *ctx, const void *kernel) {
 // `cap` items.  A level or leaf list beyond that, or items left after the
 // last launched level, mark the pass as overflowed: its sums are incomplete,
 // and the batch is re-run on the host-driven schedule.
-// Or, with few segments a pair, by kWalkRounds launches of bh_walk, each taking
+// Or, with few segments a pair, by some launches of bh_walk, each taking
 // what the one before left in the queue.  The line lies where the walk's gain
 // in launches is spent: a pair of random walks of 5,000 vertices each takes
 // 0.58 ms walked and 0.68 by levels, 30,000 1.14 and 1.13, 100,000 1.66 and
@@ -2276,11 +2274,24 @@ int resident_grid(flk_ctx *ctx, const void *kernel) {
 // walk's waves one a step).  The learned criterion's network leaves too little
 // LDS for a walk's stacks.
 constexpr int64_t kWalkSegmentsPerPair = 32768;
+// The last round ends with its longest subtree, so a large pair among small ones
+// takes more rounds to share out, two for each doubling.  Beside 380 pairs of
+// rings, a pair of tangled walks of 60,000 takes 3.8 ms in 6 rounds, 2.0 in 12 and
+// 2.1 in 24, one of 300,000 25, 5.9 and 4.2, of 1,000,000 187, 26 and 10.7, of
+// 4,000,000 beside one of 100,000 1,003, 136 and 19.6; by levels 2.0, 3.7, 9.0
+// and 90 (where pairs mix there, every far field is an atomic).  48 rounds gain
+// nothing over 24; a round that finds nothing takes 4 us.
+constexpr int kWalkRounds = 6;
+inline int walk_rounds(int64_t largest_pair) {
+  int rounds = kWalkRounds;
+  for (int64_t n = kWalkSegmentsPerPair; n < largest_pair; n *= 2) rounds += 2;
+  return rounds;
+}
 
 struct PassShape {
   int64_t cap = 0;
   bool walk = false;
-  int D = 0, ipt = 4;
+  int D = 0, rounds = 0, ipt = 4;
   int copies = 1;  // of the per-pair sums: a walk's blocks of different XCDs add to different ones
   unsigned grid_lev = 1, grid_leaf = 1;
 };
@@ -2292,11 +2303,14 @@ constexpr int kHostCounterWords = 4 + 2 * 1024;
 // Sizes the device schedule of a batch of nb pairs on trees of `segments`
 // segments, the deepest with `depth` node levels, and reserves its buffers;
 // false when it cannot hold the batch (the host-driven schedule runs it
-// instead).
-bool plan_device_passes(flk_ctx *ctx, int64_t nb, int64_t segments, int depth, bool use_mlp, PassShape &P) {
+// instead).  largest_pair: the most segments of any pair, each curve counted
+// with those of the shorter (a short curve meets little of a long one).
+bool plan_device_passes(flk_ctx *ctx, int64_t nb, int64_t segments, int64_t largest_pair, int depth, bool use_mlp,
+                        PassShape &P) {
   BhScratch &B = ctx->bh;
   P.walk = !use_mlp && segments <= nb * kWalkSegmentsPerPair;
   P.D = P.walk ? 0 : 2 * depth + 1;
+  P.rounds = P.walk ? walk_rounds(largest_pair) : 0;
   if (P.D > kMaxLevels) return false;
   if (B.dev_cap == 0) {
     // two level buffers and the leaf list (16 B per item), within a tenth of
@@ -2346,12 +2360,12 @@ void enqueue_pass(flk_ctx *ctx, const PassShape &P, const BhItem *items0, const 
   const InferImage *mlp_img = use_mlp ? ctx->mlp.d_image.as<InferImage>() : nullptr;
   const LevelKernel lev = level_kernel(P.ipt, use_mlp);
   auto leafk = P.ipt == 2 ? bh_leaf_pairs<2> : P.ipt == 8 ? bh_leaf_pairs<8> : bh_leaf_pairs<4>;
-  for (int d = 0; d < (P.walk ? kWalkRounds : P.D); ++d) {
+  for (int d = 0; d < (P.walk ? P.rounds : P.D); ++d) {
     const BhItem *in = d == 0 ? items0 : buf[(d - 1) & 1];
     if (P.walk)
       hipLaunchKernelGGL(bh_walk, dim3(P.grid_lev), dim3(kTravBlock), 0, s, in, P.cap, B.geo.as<BhGeo>(),
-                         B.mom.as<BhMom>(), beta2, eps, cnt, d, buf[d & 1], B.leaves.as<BhItem>(), d_sum, d_err,
-                         P.copies, copy_stride);
+                         B.mom.as<BhMom>(), beta2, eps, cnt, d, (int)(d + 1 == P.rounds), buf[d & 1], B.leaves.as<BhItem>(), d_sum,
+                         d_err, P.copies, copy_stride);
     else
       hipLaunchKernelGGL(lev, dim3(P.grid_lev), dim3(kTravBlock), 0, s, reinterpret_cast<const int4 *>(in), P.cap,
                          (const unsigned long long *)(cnt + 4 + 2 * d), (int)(d == 0), B.geo.as<BhGeo>(), B.mom.as<BhMom>(), beta2,
@@ -2548,18 +2562,21 @@ void plan_batch(flk_ctx *ctx, const int32_t *pairs, std::vector<int64_t> idx, co
   bp.ra.resize(nb);
   bp.rb.resize(nb);
   bp.beta2.assign(nb, (float)(prm.beta_init * prm.beta_init));
+  int64_t largest = 0;
   for (int64_t t = 0; t < nb; ++t) {
-    bp.ra[t] = root[pairs[2 * bp.idx[t]]];
-    bp.rb[t] = root[pairs[2 * bp.idx[t] + 1]];
+    const int32_t a = pairs[2 * bp.idx[t]], b = pairs[2 * bp.idx[t] + 1];
+    bp.ra[t] = root[a];
+    bp.rb[t] = root[b];
+    largest = std::max<int64_t>(largest, 2 * (int64_t)std::min(cv.n[a], cv.n[b]));
   }
-  bp.device = plan_device_passes(ctx, nb, bp.forest.S, (int)bp.forest.level_base.size(), use_mlp, bp.shape);
+  bp.device = plan_device_passes(ctx, nb, bp.forest.S, largest, (int)bp.forest.level_base.size(), use_mlp, bp.shape);
   BhScratch &B = ctx->bh;
   B.beta2.reserve(sizeof(float) * 2 * nb);
   B.items0.reserve(sizeof(BhItem) * nb);
   B.redo.reserve(sizeof(int32_t) * nb);
   B.sum.reserve(sizeof(double) * 2 * nb * bp.shape.copies);
   B.err.reserve(sizeof(double) * 2 * nb * bp.shape.copies);
-  B.cnt.reserve(sizeof(unsigned long long) * std::max(2 * kPassWords, kHostCounterWords + 8));
+  B.cnt.reserve(sizeof(unsigned long long) * std::max(2 * pass_words(bp.shape.rounds), kHostCounterWords + 8));
   if (use_mlp) mlp_upload(ctx);
   bp.v.assign(nb, 0.0);
   bp.e.assign(nb, 0.0);
@@ -2580,7 +2597,7 @@ void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, unsigned 
                      (const int32_t *)B.redo.as<int32_t>(), (const double *)B.sum.as<double>(),
                      (const double *)B.err.as<double>(), bp.shape.copies, 2 * nb,
                      prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, v, e, f, heads, cnt, bp.shape.cap,
-                     bp.shape.D);
+                     bp.shape.D, bp.shape.rounds);
   FLK_HIP(hipGetLastError());
 }
 
@@ -2599,9 +2616,10 @@ void enqueue_adapt(flk_ctx *ctx, const BatchPlan &bp, const flk_params &prm, uns
 void enqueue_begin(flk_ctx *ctx, const BatchPlan &bp, hipStream_t s) {
   BhScratch &B = ctx->bh;
   const int64_t nb = (int64_t)bp.idx.size(), nsums = 2 * nb * bp.shape.copies;
-  hipLaunchKernelGGL(bh_begin, dim3((unsigned)((std::max<int64_t>(nsums, 2 * kPassWords) + 255) / 256)), dim3(256), 0,
-                     s, bp.d_ra, bp.d_rb, nb, B.items0.as<BhItem>(), B.cnt.as<unsigned long long>(), nsums, B.sum.as<double>(),
-                     B.err.as<double>());
+  const int words = pass_words(bp.shape.rounds);
+  hipLaunchKernelGGL(bh_begin, dim3((unsigned)((std::max<int64_t>(nsums, 2 * words) + 255) / 256)), dim3(256), 0, s,
+                     bp.d_ra, bp.d_rb, nb, B.items0.as<BhItem>(), B.cnt.as<unsigned long long>(), words, nsums,
+                     B.sum.as<double>(), B.err.as<double>());
   FLK_HIP(hipGetLastError());
 }
 
@@ -2620,7 +2638,7 @@ void enqueue_traversal(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, hipSt
   const float eps = (float)(prm.eps_sq * cv.scale * cv.scale);
   const float log_tol = (float)prm.mlp_log_tol;
   double *sum = B.sum.as<double>(), *err = B.err.as<double>();
-  unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + kPassWords;
+  unsigned long long *c1 = B.cnt.as<unsigned long long>(), *c2 = c1 + pass_words(P.rounds);
   if (first) {
     enqueue_begin(ctx, bp, s);
     enqueue_pass(ctx, P, B.items0.as<BhItem>(), bp.d_beta2, eps, use_mlp, log_tol, c1, sum, err, 2 * nb, s);

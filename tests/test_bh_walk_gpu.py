@@ -83,3 +83,28 @@ def test_deep_stacks_stay_in_the_walk(engine):
         again = engine.linking_numbers(pairs, method="barneshut", fallback_tol=0.0)
         assert again.stats["bh_host_passes"] == 0
         np.testing.assert_allclose(again.lk, first.lk, rtol=0, atol=1e-9)
+
+
+def _rings(n, count, at):
+    t = 2 * np.pi * np.arange(n) / n
+    flat, tilted = (np.stack([np.cos(t), np.sin(t), 0 * t], 1), np.stack([np.cos(t), 0 * t, np.sin(t)], 1))
+    return [(tilted if k % 2 else flat) + np.array([at + 1.4 * k, 0.0, 0.0]) for k in range(count)]
+
+
+@pytest.mark.parametrize("n", [300000, 1500])
+def test_one_large_pair_among_many_small(engine, n):
+    """A dominant tangled pair takes the rounds it needs to spread over the chip:
+    the batch costs little more than the pair and the rings by themselves (in six
+    rounds 13 times as much for 300,000 segments a curve)."""
+    curves = W.random_walk_pair(seed=7, n=n, rg=100.0 * np.sqrt(n / 2e6), workload=3) + _rings(200, 380, 1000.0)
+    engine.set_curves(curves)
+    pairs = engine.potential_links()
+    assert len(pairs) > 300 and list(pairs[0]) == [0, 1]
+    _check(engine, pairs)
+
+    def fastest(p):
+        return min(engine.linking_numbers(p, method="barneshut", fallback_tol=0.0).stats["ms_total"] for _ in range(5))
+
+    parts, whole = fastest(pairs[:1]) + fastest(pairs[1:]), fastest(pairs)
+    print(n, "parts", parts, "whole", whole)
+    assert whole < 5 * parts

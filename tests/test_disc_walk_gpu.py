@@ -1,5 +1,7 @@
 """The discretization's walk for overlapping pieces: what it finds does not
 depend on where the model lies, how large it is, or the curves' order."""
+import time
+
 import numpy as np
 import pytest
 
@@ -36,3 +38,43 @@ def test_models_beyond_fp32(engine, na, nb):
     assert db == du
     for u, b in zip(unit, big):  # a power of two changes no rounding
         np.testing.assert_array_equal(b, 2.0 ** 130 * u)
+
+
+def _rings(n, rows, columns):
+    """Chain mail of rows x columns rings of n points, on a grid of 2^-20."""
+    t = 2 * np.pi * np.arange(n) / n
+    out = []
+    for k in range(rows * columns):
+        i, j = divmod(k, columns)
+        s = 1 if (i + j) % 2 else -1
+        x = np.stack([1.5 * i + np.cos(t), 1.5 * j + 0.7 * np.sin(t), 0.7 * s * np.sin(t) + 0.05 * np.sin(3 * t + k)], 1)
+        out.append(np.round(x * 2.0 ** 20) / 2.0 ** 20)
+    return out
+
+
+def _timed(engine, curves, seg_type=None):
+    """The discretization of curves that are on the device, and the fastest of five."""
+    best = np.inf
+    for _ in range(5):
+        engine.set_curves(curves)
+        pairs = engine.potential_links()
+        start = time.perf_counter()
+        d = engine.discretize_current(flk.SEG_POLYLINE if seg_type is None else seg_type, True, pairs)
+        best = min(best, time.perf_counter() - start)
+    return d, best
+
+
+def test_model_far_from_the_origin(engine):
+    """At 2^23 an FP32 number is 1 from the next, more than a hundred segments'
+    length: the same rounds, and no longer than at the origin (17 times as long
+    with boxes about 0)."""
+    curves = _rings(400, 16, 16)
+    near, t_near = _timed(engine, curves)
+    far, t_far = _timed(engine, [c + 2.0 ** 23 for c in curves])
+    print("near", t_near, "far", t_far)
+    assert far == near
+    assert t_far < 2 * t_near
+    few = [c + 2.0 ** 23 for c in _rings(60, 3, 4)]
+    m = O.Model.from_curves(few)
+    got, _ = engine.discretize(few, flk.SEG_POLYLINE, True, m.pls())
+    assert [len(c) for c in got] == [len(c) for c in m.discretize().curves()]

@@ -303,7 +303,7 @@ struct DiscScratch {
     DevBuf c, s, lo, hi, box;
   } gen[2], ret;
   DevBuf q, land, cs, links, cnt, diag, part;
-  DevBuf heap, curve_end, hit, flag, scan, tmp;
+  DevBuf heap, hit, flag, scan, tmp;
   DevBuf k0, k1, i0, i1, i2, open, out, per_curve;
   HostBuf host;  // pinned: tables on their way to the device, results on their way back
   static constexpr size_t kKept = size_t(1) << 30;  // more is given back after the call
@@ -311,7 +311,7 @@ struct DiscScratch {
     size_t n = 0;
     for (const Gen *g : {&gen[0], &gen[1], &ret})
       for (const DevBuf *b : {&g->c, &g->s, &g->lo, &g->hi, &g->box}) n += b->bytes;
-    for (const DevBuf *b : {&q, &land, &cs, &links, &cnt, &diag, &part, &heap, &curve_end, &hit, &flag, &scan, &tmp, &k0,
+    for (const DevBuf *b : {&q, &land, &cs, &links, &cnt, &diag, &part, &heap, &hit, &flag, &scan, &tmp, &k0,
                             &k1, &i0, &i1, &i2, &open, &out, &per_curve})
       n += b->bytes;
     return n;

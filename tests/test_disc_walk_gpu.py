@@ -1,5 +1,6 @@
 """The discretization's walk for overlapping pieces: what it finds does not
 depend on where the model lies, how large it is, or the curves' order."""
+import re
 import time
 
 import numpy as np
@@ -78,3 +79,49 @@ def test_model_far_from_the_origin(engine):
     m = O.Model.from_curves(few)
     got, _ = engine.discretize(few, flk.SEG_POLYLINE, True, m.pls())
     assert [len(c) for c in got] == [len(c) for c in m.discretize().curves()]
+
+
+@pytest.mark.parametrize("rows,columns,n", [(5, 7, 33), (70, 70, 60)])
+def test_order_of_the_curves(engine, rows, columns, n):
+    """Curves in random order: the same rounds and polylines, and no longer (55
+    times as long when a query walked every piece behind its curve)."""
+    curves = _rings(n, rows, columns)
+    perm = np.random.default_rng(1).permutation(len(curves))
+    ordered, t_ordered = _timed(engine, curves)
+    shuffled, t_shuffled = _timed(engine, [curves[k] for k in perm])
+    print("ordered", t_ordered, "shuffled", t_shuffled, ordered["rounds"])
+    assert shuffled == ordered
+    assert t_shuffled < 3 * t_ordered
+    if rows == 5:
+        pairs = O.Model.from_curves(curves).pls()
+        want, _ = engine.discretize(curves, flk.SEG_BSPLINE, True, pairs)
+        back = np.argsort(perm)
+        got, _ = engine.discretize([curves[k] for k in perm], flk.SEG_BSPLINE, True, back[pairs])
+        assert all(np.array_equal(got[back[k]], w) for k, w in enumerate(want))
+
+
+def _through_one_another(count, n):
+    """Closed curves of two modes a coordinate, all about the origin."""
+    t = 2 * np.pi * np.arange(n) / n
+    out = []
+    for k in range(count):
+        g = np.random.default_rng([7, k])
+        out.append(sum(g.normal(size=3) / m * np.cos(m * t[:, None] + g.uniform(0, 6.28, 3)) for m in (1, 2)))
+    return out
+
+
+# up to 32 partners of a curve are asked one by one, beyond that the pieces are sorted
+@pytest.mark.parametrize("looped", [True, False])
+@pytest.mark.parametrize("count,n", [(12, 100), (33, 40), (34, 40), (70, 25), (80, 23), (80, 150)])
+def test_many_partners(engine, capfd, count, n, looped):
+    curves = _through_one_another(count, n) + [c + [9.0, 0, 0] for c in _through_one_another(2, 9)]
+    m = O.Model.from_curves(curves, looped=looped)
+    pairs = m.pls()
+    capfd.readouterr()
+    ref = m.discretize().curves()
+    overlaps = [int(x) for x in re.findall(r"Iteration \d+, (\d+) overlaps", capfd.readouterr().out)]
+    got, d = engine.discretize(curves, flk.SEG_POLYLINE, looped, pairs)
+    assert d["overlaps"] == overlaps
+    assert [len(c) for c in got] == [len(c) for c in ref]
+    for a, b in zip(got, ref):
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-12)

@@ -47,9 +47,13 @@ constexpr int64_t kBoxChunk = 4096;
 // Coordinates that came as FP32 are read there and written to xyz as FP64 on the
 // way (a pass of its own read and wrote them again: 215 us for 3.1e7 vertices).
 // A block of 1,024 threads with four vertices each in flight: for a few curves of
-// thousands of vertices the pass is as long as one chunk.
-template <bool LANDED>
-__global__ __launch_bounds__(1024) void curve_box_chunks(double *__restrict__ xyz, const float *__restrict__ land,
+// thousands of vertices the pass is as long as one chunk.  Launching such a block
+// takes 14 ns, so for more than kManyChunks chunks it has as many threads as a
+// chunk has fours on average, in quarters: 200,000 curves of 16 vertices 2,887 ->
+// 370 us, 20,000 of 400 302 -> 79, 3,000 of 100 53 -> 11, 1,100 of 900 28 -> 16.
+constexpr int64_t kManyChunks = 1024;
+template <bool LANDED, int THREADS>
+__global__ __launch_bounds__(THREADS) void curve_box_chunks(double *__restrict__ xyz, const float *__restrict__ land,
                                                         const int64_t *__restrict__ chunk_v,
                                                         double *__restrict__ part, double *__restrict__ host,
                                                         int32_t *__restrict__ inexact) {
@@ -57,11 +61,11 @@ __global__ __launch_bounds__(1024) void curve_box_chunks(double *__restrict__ xy
   if (host && c == 0 && threadIdx.x == 0) *inexact = 0;
   const int64_t v0 = chunk_v[2 * c], v1 = chunk_v[2 * c + 1];
   double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  for (int64_t base = v0 + threadIdx.x; base < v1; base += 4 * 1024) {
+  for (int64_t base = v0 + threadIdx.x; base < v1; base += 4 * THREADS) {
     double x[4][3];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int64_t v = min(base + 1024 * k, v1 - 1);  // the last again past the end
+      const int64_t v = min(base + THREADS * k, v1 - 1);  // the last again past the end
 #pragma unroll
       for (int d = 0; d < 3; ++d) x[k][d] = LANDED ? (double)land[3 * v + d] : xyz[3 * v + d];
     }
@@ -69,12 +73,12 @@ __global__ __launch_bounds__(1024) void curve_box_chunks(double *__restrict__ xy
     for (int k = 0; k < 4; ++k)
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        if (LANDED && base + 1024 * k < v1) xyz[3 * (base + 1024 * k) + d] = x[k][d];
+        if (LANDED && base + THREADS * k < v1) xyz[3 * (base + THREADS * k) + d] = x[k][d];
         mn[d] = fmin(mn[d], x[k][d]);
         mx[d] = fmax(mx[d], x[k][d]);
       }
   }
-  __shared__ double smn[3][16], smx[3][16];
+  __shared__ double smn[3][THREADS / 64], smx[3][THREADS / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -91,7 +95,7 @@ __global__ __launch_bounds__(1024) void curve_box_chunks(double *__restrict__ xy
   if (threadIdx.x == 0) {
     for (int d = 0; d < 3; ++d) {
       double lo = smn[d][0], hi = smx[d][0];
-      for (int k = 1; k < (int)(blockDim.x >> 6); ++k) {
+      for (int k = 1; k < THREADS / 64; ++k) {
         lo = fmin(lo, smn[d][k]);
         hi = fmax(hi, smx[d][k]);
       }
@@ -512,10 +516,15 @@ void curve_boxes_run(flk_ctx *ctx, std::vector<double> &boxes, const float *land
   double *d_boxes = ctx->d_boxes.as<double>(), *d_part = d_boxes + 6 * nc;
   const int64_t *d_coff = ctx->d_misc.as<int64_t>() + 2 * (nc + 1), *d_chunk = d_coff + nc + 1;
   int32_t *flag = ctx->d_count.as<int32_t>();
-  if (nchunks > 0)
-    hipLaunchKernelGGL(land ? curve_box_chunks<true> : curve_box_chunks<false>, dim3((unsigned)nchunks), dim3(1024), 0,
-                       s, cv.raw.as<double>(), land, d_chunk,
+  if (nchunks > 0) {
+    const int64_t mean = nchunks > kManyChunks ? cv.in_off[nc] / nchunks : kBoxChunk;
+    const auto pass = mean <= 256    ? (land ? curve_box_chunks<true, 64> : curve_box_chunks<false, 64>)
+                      : mean <= 1024 ? (land ? curve_box_chunks<true, 256> : curve_box_chunks<false, 256>)
+                                     : (land ? curve_box_chunks<true, 1024> : curve_box_chunks<false, 1024>);
+    hipLaunchKernelGGL(pass,
+                       dim3((unsigned)nchunks), dim3(mean <= 256 ? 64 : mean <= 1024 ? 256 : 1024), 0, s, cv.raw.as<double>(), land, d_chunk,
                        single ? d_boxes : d_part, single ? host : (double *)nullptr, flag);
+  }
   if (!single)
     hipLaunchKernelGGL(curve_box_merge, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, d_part, d_coff,
                        cv.ncurves, d_boxes, host, flag);

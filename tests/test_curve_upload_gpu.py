@@ -63,3 +63,26 @@ def test_boxes_around_a_chunk(engine, sizes, dtype):
         if b > a:
             v = packed[a:b].astype(np.float64)
             assert np.array_equal(boxes[k], np.concatenate([v.min(0), v.max(0)])), k
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mean", [3, 256, 257, 1000, 1100])
+@pytest.mark.parametrize("longest", [0, 9000])
+def test_boxes_of_many_curves(engine, mean, longest, dtype):
+    """More than 1,024 curves: blocks of a wave, of four and of sixteen by the
+    mean chunk, each over curves shorter and longer than its rounds (and, with
+    one beyond a chunk, through the merge); empty ones among them."""
+    rng = np.random.default_rng(mean + longest)
+    sizes = rng.integers(0, 2 * mean, size=1300)
+    sizes[:6] = [0, 1, 2 * mean, 255, 4 * 255 + 1, longest]
+    packed = rng.normal(size=(sizes.sum(), 3)).astype(dtype)
+    offsets = np.concatenate([[0], np.cumsum(sizes)])
+    full = sizes > 0
+    packed[offsets[:-1][full]], packed[offsets[1:][full] - 1] = -9, 9
+    engine.set_curves_packed(packed, offsets)
+    boxes = engine.curve_boxes()
+    want = np.array([np.concatenate([v.min(0), v.max(0)]) for v in np.split(packed.astype(np.float64), offsets[1:-1])
+                     if len(v)])
+    assert np.array_equal(boxes[full], want)
+    assert np.array_equal(engine.linking_numbers([[2, 3]], method="directsum", fp64=1).lk,
+                          engine.linking_numbers([[2, 3]], method="directsum", fp64=1, graph=0).lk)

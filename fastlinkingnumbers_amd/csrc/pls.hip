@@ -365,7 +365,9 @@ __global__ __launch_bounds__(256) void pls_all_pairs(const double *__restrict__ 
 // curve, the tree (with its two library sorts, an allocation per array and one
 // atomic per pair) against all pairs: 137 and 25 us for 10 curves, 270 and 44
 // for 400, 393 and 77 for 1,600, 587 and 237 for 10,000, 727 and 250 for
-// 16,384, 1,052 and 636 for 30,000; the sweep grows with the square.
+// 16,384, 1,052 and 636 for 30,000; the sweep grows with the square.  With a pair
+// for every four curves the two meet at 28,000 (537 and 530 us; 32,000: 546 and 658), with
+// two pairs a curve all pairs are ahead at 32,000 still (979 and 665).
 constexpr int32_t kAllPairsCurves = 32768;
 
 // Up to kOneBlockCurves curves in one launch: the boxes in LDS, a row a wave at a

@@ -612,13 +612,15 @@ struct DsPlan {
 // at 256 and 64 columns: ten loops of 200-400 vertices (2e5 pairs) 313 and 240
 // us, a 12 x 12 chain mail (1.5e8 pairs) 635 and 564 us.  Below 64 the FP32
 // sums would change; 32 gave 225 and 590 us.  Larger batches are cut by
-// ds_tasks_per_wave.
-constexpr int64_t kMinCols = 64;
+// ds_tasks_per_wave; where a tuned value of it would make more tasks than a batch
+// without allocation holds, none is below 256, so that both entry points have
+// one plan (the order of their FP64 additions) for every batch.
+constexpr int64_t kMinCols = 64, kMinColsMany = 256;
 
 // share: the fraction of the resident blocks per CU to launch when the grid
 // is sized from residency (a direct sum that runs beside other kernels).
 void ds_plan(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, const flk_tune &t, int64_t stride,
-             DsPlan &P, double share = 1.0, int64_t min_cols = kMinCols) {
+             DsPlan &P, double share = 1.0) {
   Curves &cv = ctx->curves;
   P.fp64 = fp64;
   P.precise = cv.inexact;
@@ -657,11 +659,16 @@ void ds_plan(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, cons
     }
   }
   // Column chunk: aim for ds_tasks_per_wave tasks per wave over the batch,
-  // never below min_cols columns; short chunks are whole runs of the FP32
+  // never below kMinCols columns; short chunks are whole runs of the FP32
   // kernel's 64-column partial sums, which a chunk's length must not change.
   const int64_t tpw = std::max(1, t.ds_tasks_per_wave);
-  int64_t chunk_cols = std::max<int64_t>(min_cols, wave_cost / (nwaves * tpw) / rows_per_wave);
-  if (chunk_cols < 256) chunk_cols = (chunk_cols + 63) / 64 * 64;
+  int64_t chunk_cols = std::max<int64_t>(kMinCols, wave_cost / (nwaves * tpw) / rows_per_wave);
+  if (chunk_cols < kMinColsMany) {
+    chunk_cols = (chunk_cols + 63) / 64 * 64;
+    int64_t ntasks = 0;
+    for (const auto &rb : rowblk) ntasks += (P.dp[rb.first].n_c + chunk_cols - 1) / chunk_cols;
+    if (ntasks > FLK_NOALLOC_MAX_TASKS) chunk_cols = kMinColsMany;
+  }
   P.tasks.clear();
   P.prefix.clear();
   P.task0.assign(npairs + 1, 0);
@@ -960,8 +967,6 @@ void ds_run_noalloc(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp6
   if (!base) throw Error(FLK_ERR_STATE, "no scratch array on this device");
   DsPlan P;
   ds_plan(ctx, pairs, npairs, fp64, ctx->tune, 1, P);
-  if ((int64_t)P.tasks.size() > FLK_NOALLOC_MAX_TASKS)  // the fixed array holds more work in longer tasks
-    ds_plan(ctx, pairs, npairs, fp64, ctx->tune, 1, P, 1.0, 256);
   const int64_t nt = (int64_t)P.tasks.size();
   if (nt > FLK_NOALLOC_MAX_TASKS)
     throw Error(FLK_ERR_ARG, "a batch without allocation holds at most " + std::to_string(FLK_NOALLOC_MAX_TASKS) +

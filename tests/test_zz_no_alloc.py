@@ -64,3 +64,17 @@ def test_noalloc_limits_and_methods(engine):
     # the context and the array stay usable after the refusals
     ref = engine.linking_numbers([[0, 1]], method="directsum", graph=0)
     _same(engine.linking_numbers_noalloc([[0, 1]]), ref)
+
+
+@pytest.mark.parametrize("fp64", [0, 1])
+def test_noalloc_with_many_tuned_tasks(engine, fp64):
+    """1,024 tasks per wave would cut a pair of 100,000 segments into 1.2e6 chunks of
+    64 columns, more than the array holds: both entry points take 256 columns."""
+    t = 2 * np.pi * np.arange(100000) / 100000
+    a = np.stack([np.cos(t), np.sin(t), 0.1 * np.sin(3 * t)], 1)
+    engine.set_curves([a, a[:, [0, 2, 1]] + [1.0, 0.0, 0.0]])
+    engine.set_tune(ds_tasks_per_wave=1024)
+    got = engine.linking_numbers_noalloc([[0, 1]], fp64=fp64)
+    for graph in (0, 1):
+        _same(got, engine.linking_numbers([[0, 1]], method="directsum", graph=graph, fp64=fp64))
+    assert abs(abs(got.lk[0]) - 1) < 1e-5

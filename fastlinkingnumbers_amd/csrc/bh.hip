@@ -28,7 +28,6 @@
 // error estimates are FP64; a block of 1024 items reduces its sums and queue
 // slots in LDS before one global atomic each.
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cfloat>
@@ -811,32 +810,6 @@ __device__ __forceinline__ float leaf_term(F3 r, F3 t1, F3 t2) {
   const float yp = det * s;
   const float sg = det == 0.f ? -copysignf(1.f, div1) : copysignf(1.f, det);
   return kInv2PiF * atan2f(yp, xp) + ((s < 0.f || (s == 0.f && det < 0.f)) ? sg : 0.f);
-}
-
-// Per-wave FP64 accumulation into per-pair sums: one atomic per wave when
-// the wave's active items share a pair, one per item otherwise.
-__device__ __forceinline__ void pair_add(int pair, bool active, double v, double e,
-                                         double *__restrict__ sum, double *__restrict__ err) {
-  const unsigned long long act = __ballot(active);
-  if (act == 0) return;
-  const int lead = __ffsll((long long)act) - 1;
-  const int p0 = __shfl(pair, lead, 64);
-  const bool uniform = __ballot(active && pair != p0) == 0;
-  if (uniform) {
-    double a = active ? v : 0.0, b = active ? e : 0.0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      a += __shfl_xor(a, off, 64);
-      b += __shfl_xor(b, off, 64);
-    }
-    if ((int)(threadIdx.x & 63) == lead) {
-      atomicAdd(sum + p0, a);
-      if (b != 0.0) atomicAdd(err + p0, b);
-    }
-  } else if (active) {
-    atomicAdd(sum + pair, v);
-    if (e != 0.0) atomicAdd(err + pair, e);
-  }
 }
 
 // Wave-aggregated append of `cnt` slots; returns this lane's first slot.

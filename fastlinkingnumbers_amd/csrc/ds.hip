@@ -701,17 +701,18 @@ struct DsBufs {
   int32_t *corr;
 };
 
+// (out null: the sums go straight to pinned memory)
 DsBufs reserve_bufs(DevBuf &pairs, DevBuf &tasks, DevBuf &cost, DevBuf &theta, DevBuf &corr, DevBuf &task0,
-                    DevBuf &out, size_t np, size_t nt) {
+                    DevBuf *out, size_t np, size_t nt) {
   pairs.reserve(sizeof(DsPair) * np);
   tasks.reserve(sizeof(DsTask) * nt);
   cost.reserve(sizeof(int64_t) * (nt + 1));
   theta.reserve(sizeof(double) * nt);
   corr.reserve(sizeof(int32_t) * nt);
   task0.reserve(sizeof(int64_t) * (np + 1));
-  out.reserve(sizeof(double) * np);
+  if (out) out->reserve(sizeof(double) * np);
   return DsBufs{pairs.as<DsPair>(), tasks.as<DsTask>(), cost.as<int64_t>(), task0.as<int64_t>(),
-                theta.as<double>(), out.as<double>(), corr.as<int32_t>()};
+                theta.as<double>(), out ? out->as<double>() : nullptr, corr.as<int32_t>()};
 }
 
 // Uploads of the plan arrays, the tile kernel (between ev_a and ev_b when
@@ -778,7 +779,7 @@ float ds_eager(flk_ctx *ctx, const DsPlan &P, std::vector<double> *lk_out) {
   if (P.tasks.empty()) return 0.f;
   const int64_t np = (int64_t)P.dp.size(), nt = (int64_t)P.tasks.size();
   const DsBufs d = reserve_bufs(ctx->d_pairs, ctx->d_tasks, ctx->d_cost, ctx->d_task_theta, ctx->d_task_corr,
-                                ctx->d_pair_task0, ctx->d_pair_out, np, nt);
+                                ctx->d_pair_task0, &ctx->d_pair_out, np, nt);
   hipStream_t s = ctx->stream;
   ds_enqueue(ctx, P, P.dp.data(), P.tasks.data(), P.prefix.data(), P.task0.data(), np, nt, d, s, ctx->ev0,
              ctx->ev1, lk_out ? lk_out->data() : nullptr);
@@ -807,17 +808,14 @@ float ds_graph_run(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64
       *work = 0;
       return 0.f;
     }
-    // the graph's copy nodes read the host arrays kept in G
     G.dp = std::move(P.dp);
     G.tasks = std::move(P.tasks);
     G.prefix = std::move(P.prefix);
     G.task0 = std::move(P.task0);
-    G.out.assign(npairs, 0.0);
     G.work = P.work;
     G.waves = P.blocks * 4;
     const int64_t nt = (int64_t)G.tasks.size();
-    DsBufs d = reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, G.d_out, npairs, nt);
-    d.out = nullptr;
+    const DsBufs d = reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, nullptr, npairs, nt);
     G.h_out.reserve(sizeof(double) * npairs);
     // the plan goes to the device once; the graph reads it there
     ds_upload(G.dp.data(), G.tasks.data(), G.prefix.data(), G.task0.data(), npairs, nt, d, s);
@@ -862,7 +860,6 @@ void ds_capture_prepare(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool
   G.tasks = std::move(P.tasks);
   G.prefix = std::move(P.prefix);
   G.task0 = std::move(P.task0);
-  G.out.assign(npairs, 0.0);
   G.work = P.work;
   G.waves = P.blocks * 4;
   G.npairs = npairs;
@@ -873,7 +870,7 @@ void ds_capture_prepare(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool
   G.h_out.reserve(sizeof(double) * std::max<int64_t>(npairs, 1));
   std::fill(G.h_out.as<double>(), G.h_out.as<double>() + npairs, 0.0);
   if (!G.tasks.empty()) {
-    const DsBufs d = reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, G.d_out, npairs,
+    const DsBufs d = reserve_bufs(G.d_pairs, G.d_tasks, G.d_cost, G.d_theta, G.d_corr, G.d_task0, nullptr, npairs,
                                   G.tasks.size());
     ds_upload(G.dp.data(), G.tasks.data(), G.prefix.data(), G.task0.data(), npairs, (int64_t)G.tasks.size(), d,
               ctx->stream);
@@ -881,7 +878,7 @@ void ds_capture_prepare(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool
 }
 
 void ds_capture_enqueue(flk_ctx *ctx, DsGraph &G, hipStream_t s) {
-  if (G.tasks.empty()) return;  // G.out stays zero: no segment pairs
+  if (G.tasks.empty()) return;  // G.h_out stays zero: no segment pairs
   DsPlan P;
   P.R = G.R;
   P.blocks = G.blocks;

@@ -10,9 +10,6 @@
 
 #include "flk_internal.h"
 
-namespace flk {
-}
-
 using flk::Error;
 
 static thread_local std::string g_create_err;
@@ -81,7 +78,6 @@ void curves_clear(flk_ctx *ctx) {
 void curves_finish(flk_ctx *ctx, const float *land) {
   Curves &cv = ctx->curves;
   const int32_t ncurves = cv.ncurves;
-  hipStream_t s = ctx->stream;
   curve_boxes_run(ctx, cv.box, land);
   // Origin and power-of-two scale: stored = (x - origin) * scale with the
   // model extent near 1.  The origin stays 0 unless the model is far from it

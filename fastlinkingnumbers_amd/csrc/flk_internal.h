@@ -246,10 +246,10 @@ struct GraphKey {
   bool operator==(const GraphKey &o) const { return rest == o.rest && sizes == o.sizes && pairs == o.pairs; }
 };
 
-// A captured direct-sum batch (tile kernel, per-pair reduction, read-back) for
-// replay when the same pairs of curves of the same sizes come again.  It owns
-// its device buffers and host staging, so reallocations elsewhere cannot leave
-// dangling pointers in the graph.
+// A captured direct-sum batch (tile kernel and per-pair reduction) for replay
+// when the same pairs of curves of the same sizes come again.  It owns its device
+// buffers and its pinned sums, so reallocations elsewhere cannot leave dangling
+// pointers in the graph.
 struct DsGraph {
   GraphKey key;
   hipGraphExec_t exec = nullptr;
@@ -261,17 +261,16 @@ struct DsGraph {
   std::vector<DsPair> dp;
   std::vector<DsTask> tasks;
   std::vector<int64_t> prefix, task0;
-  std::vector<double> out;
-  DevBuf d_pairs, d_tasks, d_cost, d_theta, d_corr, d_task0, d_out;
-  HostBuf h_out;  // pinned end of the read-back (copied into out)
+  DevBuf d_pairs, d_tasks, d_cost, d_theta, d_corr, d_task0;
+  HostBuf h_out;  // pinned: the sums
   void reset() {
     if (exec) (void)hipGraphExecDestroy(exec);
     exec = nullptr;
   }
   void take_buffers(DsGraph &o) {
-    DevBuf *mine[] = {&d_pairs, &d_tasks, &d_cost, &d_theta, &d_corr, &d_task0, &d_out};
-    DevBuf *from[] = {&o.d_pairs, &o.d_tasks, &o.d_cost, &o.d_theta, &o.d_corr, &o.d_task0, &o.d_out};
-    for (int k = 0; k < 7; ++k) std::swap(*mine[k], *from[k]);
+    DevBuf *mine[] = {&d_pairs, &d_tasks, &d_cost, &d_theta, &d_corr, &d_task0};
+    DevBuf *from[] = {&o.d_pairs, &o.d_tasks, &o.d_cost, &o.d_theta, &o.d_corr, &o.d_task0};
+    for (int k = 0; k < 6; ++k) std::swap(*mine[k], *from[k]);
     std::swap(h_out, o.h_out);
   }
   ~DsGraph() { reset(); }
@@ -397,8 +396,7 @@ int64_t ds_work(flk_ctx *ctx, const int32_t *pairs, int64_t npairs);
 // A direct-sum batch recorded inside a larger graph: ds_capture_prepare plans
 // the pairs into G's host arrays, reserves G's buffers and uploads the plan
 // (call it before the capture begins); ds_capture_enqueue enqueues the tile
-// kernel, the per-pair reduction and the read-back into G.h_out, which the
-// caller copies into G.out after the launch.  share: the fraction of the
+// kernel and the per-pair reduction into G.h_out.  share: the fraction of the
 // tile kernel's resident blocks per CU its grid takes (below 1 when it runs
 // beside other kernels; a tuned ds_blocks_per_cu takes precedence).
 void ds_capture_prepare(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, DsGraph &G,

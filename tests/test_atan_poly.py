@@ -57,3 +57,19 @@ def test_fitting_script_reproduces_the_polynomials():
     c = F.remez(16.0 / 63.0, 4, grid=40001)
     assert F.max_rel_error(list(c[::-1]), 16.0 / 63.0)[0] < 3e-10
     assert F.max_rel_error([float(np.float32(v)) for v in c[::-1]], 16.0 / 63.0)[0] < 1.2e-9
+
+
+def test_fp64_series_meets_its_stated_bound():
+    """The FP64 kernel's Q, read from its source: 2.6e-17 as stated there, and the
+    fitting script's interpolation is the same polynomial."""
+    src = open(os.path.join(CSRC, "ds.hip")).read()
+    body = src[src.index("double atan_short_f64("):]
+    body = body[body.index("double p ="): body.index("return fma(t * s, p, t);")]
+    kernel = [float(v) for v in re.findall(r"(-?\d+\.\d+)[;)]", body)]
+    assert len(kernel) == 8
+    a = np.tan(4 * np.arctan(1 / 16))
+    e = F.max_rel_error_f64(kernel[::-1], a)
+    fit, e_fit = F.interpolate_f64(a, 7)
+    print("kernel", e, "fit", e_fit)
+    assert e < 2.65e-17 and e_fit < 2.65e-17
+    np.testing.assert_allclose(fit[::-1], kernel, rtol=1e-7)

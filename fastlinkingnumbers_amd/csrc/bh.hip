@@ -3,13 +3,13 @@
 // Reference: src/compute_link.cpp:294-934 (trees, moments, far field, node-pair
 // traversal) and src/linking_number_certificate.cpp:102-229 (adaptive beta).
 //
-// Trees.  All segments of the curves in Barnes–Hut pairs are sorted once by
-// (curve, 30-bit Morton code of the segment midpoint in the curve's box), a
-// single radix sort.  Each curve's tree is the balanced median split of its
+// Trees.  Each curve's segments are sorted by the 30-bit Morton code of their
+// midpoint in the curve's box: short curves by a block each, the others by one
+// segmented radix sort.  A curve's tree is the balanced median split of its
 // Morton-ordered segments (left half floor(n/2)), down to leaf buckets of at
 // most leaf_size segments; a subtree is a contiguous range of the sorted order
-// (the reference's ModifiedKdBVH.h:128-131 property).  Nodes are created level
-// by level with scan-assigned child slots (deterministic numbering).
+// (the reference's ModifiedKdBVH.h:128-131 property).  Every node's range and
+// children follow from the segment counts alone and come from one launch.
 //
 // Moments (reference compute_link.cpp:333-389) are built bottom-up in FP64
 // about each node's box centre: nodes of at most 8 segments sum their
@@ -17,14 +17,15 @@
 // children's moments in FP64 (Eqs. 21-23), and the records are stored in FP32.  The centre keeps an FP32 hi/lo split so node
 // separations are exact to FP32 precision of the separation itself.
 //
-// Traversal.  Work items (pair, node1, node2) live in level buffers; one
-// kernel per level classifies every item: leaf-bucket pairs go to a leaf list
+// Traversal.  Work items are (pair, node1, node2).  A pass goes level by level, one
+// kernel a level, or, with few segments a pair, depth first in a few rounds of
+// bh_walk; either classifies every item: leaf-bucket pairs go to a leaf list
 // evaluated exactly by a second kernel, pairs with |r|^2 > beta^2 (r1+r2)^2
 // are evaluated with the second-order far field (reference
 // compute_link.cpp:410-524, Supplemental Eqs. 29-30) and the Eq. 14 error
-// estimate, the rest split the larger node (a leaf is never split) into the
-// next level.  Levels are processed in chunks with a LIFO stack, so memory is
-// bounded by depth x chunk whatever the frontier width.  Per-pair sums and
+// estimate, the rest split the larger node (a leaf is never split).  A pass whose
+// buffers overflow is run again from the host, in chunks of a level with a LIFO
+// stack, so memory is bounded by depth x chunk whatever the frontier width.  Per-pair sums and
 // error estimates are FP64; a block of 1024 items reduces its sums and queue
 // slots in LDS before one global atomic each.
 #include <hip/hip_runtime.h>
@@ -2801,10 +2802,9 @@ std::vector<std::vector<int64_t>> form_batches(flk_ctx *ctx, const int32_t *pair
 }  // namespace
 
 // A whole Barnes–Hut certificate as one captured graph: the direct-sum batch
-// of the pairs below the threshold (uploads, persistent tile kernel,
-// reduction, read-back) and, per Barnes–Hut batch, the forest build (sort,
-// levels, moments), both traversal passes with the device re-run decision
-// between them, the merge and the read-back.  The device pointers it holds
+// of the pairs below the threshold (persistent tile kernel, reduction) and, per Barnes–Hut batch, the forest build (sort,
+// topology, moments), both traversal passes with the device re-run decision
+// between them and the merge, results straight to pinned memory: kernels only.  The device pointers it holds
 // belong to the context's scratch: it is replayed only while no DevBuf has
 // been allocated or freed since its capture (g_devbuf_epoch).  Its plans follow
 // from the pairs and the curves' sizes but for the key boxes, so new positions

@@ -8,8 +8,9 @@
 // to FP32 on the way whenever every value converts exactly -- the case for any
 // model whose coordinates came from FP32 data, for which it halves the bytes
 // sent.  One value that does not convert exactly sends the whole array as
-// FP64 instead.  On the device a widening kernel writes the FP64 array the
-// rest of the engine reads, so both routes give identical bits.
+// FP64 instead.  On the device the pass that takes the boxes writes the FP64
+// array that the rest of the engine reads (a widening kernel where there is no such
+// pass), so both routes give identical bits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -46,3 +46,33 @@ def test_guard_names_the_first_smallest_segment(engine, n):
     # one unit above the threshold's order passes
     got, d = engine.discretize([a], flk.SEG_POLYLINE, True, np.zeros((0, 2), np.int32))
     assert d["segments"] == n and np.array_equal(got[0], a)
+
+
+def test_scratch_beyond_the_kept_is_given_back(engine):
+    """Two polylines of 2.5e6 segments take more than 1 GiB, which is given back,
+    also when the input guard throws: the calls behind are a fresh engine's."""
+    n = 2500000
+    t = 2 * np.pi * np.arange(n) / n
+    large = [np.stack([x + np.cos(t), np.sin(t), 0 * t], 1) for x in (0.0, 5.0)]
+    none = np.zeros((0, 2), np.int32)
+    small = _rings(300, 6, 0.01)
+    pairs = [[i, i + 1] for i in range(5)]
+    fresh = flk.Engine(0)
+    want, dw = fresh.discretize(small, flk.SEG_BSPLINE, True, pairs)
+    want_boxes = fresh.curve_boxes()
+    fresh.close()
+    bad = [large[0], large[1].copy()]
+    bad[1][7] = bad[1][6]
+    for attempt in ("whole", "guard"):
+        if attempt == "whole":
+            got, d = engine.discretize(large, flk.SEG_POLYLINE, True, none)
+            assert d["segments"] == d["pieces"] == 2 * n
+            assert all(np.array_equal(g, c) for g, c in zip(got, large))
+        else:
+            with pytest.raises(flk.FlkError, match="Smallest input segment"):
+                engine.discretize(bad, flk.SEG_POLYLINE, True, none)
+        got, d = engine.discretize(small, flk.SEG_BSPLINE, True, pairs)
+        assert d == dw and all(np.array_equal(g, w) for g, w in zip(got, want)), attempt
+        engine.set_curves(small)
+        d = engine.discretize_current(flk.SEG_BSPLINE, True, pairs)
+        assert d["pieces"] == dw["pieces"] and np.array_equal(engine.curve_boxes(), want_boxes), attempt

@@ -31,3 +31,24 @@ def test_captured_certificate_on_new_positions(engine, kw):
             np.testing.assert_allclose(got.lk, want.lk, rtol=0, atol=1e-9, err_msg=str(k))
             np.testing.assert_allclose(got.err, want.err, rtol=1e-9, atol=1e-15, err_msg=str(k))
             assert np.array_equal(got.flags, want.flags), k
+
+
+def test_one_graph_with_and_without_re_runs(engine):
+    """The re-runs' own graph is launched behind the first pass, at once, or not at
+    all, as the positions of one key ask for them."""
+    walks = W.random_walk_pair(seed=3, n=16000, rg=25.0, workload=3)
+    t = 2 * np.pi * np.arange(16000) / 16000
+    rings = [np.stack([np.cos(t), np.sin(t), 0 * t], 1), np.stack([1 + np.cos(t), 0.1 * np.cos(3 * t), np.sin(t)], 1)]
+    rings = [r + 1e-9 * w for r, w in zip(rings, walks)]  # FP32 holds neither
+    retries = []
+    for curves in (rings, rings, walks, walks, rings, walks, rings, rings):
+        engine.set_curves(curves)
+        got = engine.linking_numbers([[0, 1]], method="barneshut", fallback_tol=0.0)
+        want = engine.linking_numbers([[0, 1]], method="barneshut", fallback_tol=0.0, graph=0)
+        retries.append(got.stats["retries"])
+        for key in ("bh_visits", "bh_far", "bh_leaf_pairs", "retries"):
+            assert got.stats[key] == want.stats[key], key
+        np.testing.assert_allclose(got.lk, want.lk, rtol=0, atol=1e-9)
+        np.testing.assert_allclose(got.err, want.err, rtol=1e-9)
+        assert np.array_equal(got.flags, want.flags)
+    assert retries == [0, 0, 1, 1, 0, 1, 0, 0]

@@ -2852,9 +2852,14 @@ template <typename F> hipGraphExec_t captured(hipStream_t s, F &&body) {
   return exec;
 }
 
+// Most batches of one graph (about 7,000 nodes in a chain; a call that would
+// have captured hundreds of thousands, 5e5 pairs in batches of 250 curves, ended in
+// a segmentation fault on the host).  The largest benchmark has two.
+constexpr size_t kGraphBatches = 64;
+
 // Captures (or finds) the certificate graph for these pairs and launches it;
-// false when a batch does not fit the device schedule (the caller then runs
-// the eager path).
+// false when a batch does not fit the device schedule, or there are too many
+// (the caller then runs the eager path).
 bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_params &prm,
                   const std::vector<int64_t> &ds_idx, const std::vector<int32_t> &ds_pairs,
                   const std::vector<int64_t> &bh_idx, std::vector<double> &lk, std::vector<double> &err,
@@ -2869,12 +2874,14 @@ bool bh_run_graph(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, const flk_
   CertGraph *G = ctx->cert_graph.get();
   PlanUpload up;
   if (!(G && G->key == key && G->epoch == g_devbuf_epoch.load())) {
+    auto formed = form_batches(ctx, pairs, bh_idx, prm);
+    if (formed.size() > kGraphBatches) return false;
     auto NG = std::make_shared<CertGraph>();
     if (G) NG->ds.take_buffers(G->ds);
     ctx->cert_graph.reset();
     NG->key = std::move(key);
     NG->ds_idx = ds_idx;
-    for (auto &idx : form_batches(ctx, pairs, bh_idx, prm)) {
+    for (auto &idx : formed) {
       NG->batches.emplace_back();
       BatchPlan &bp = NG->batches.back();
       plan_batch(ctx, pairs, std::move(idx), prm, bp);

@@ -69,7 +69,8 @@ typedef struct flk_params {
                            replayed when the same pairs come again; a
                            certificate with both parts runs its direct sum as
                            a branch of its own, on the context's second stream
-                           (default priority), beside the Barnes–Hut batches;
+                           (default priority), beside the Barnes–Hut batches
+                           (one graph holds up to 64; more run eagerly);
                            0: launched eagerly every time */
   int32_t reserved[5];
 } flk_params;

@@ -223,3 +223,19 @@ def test_hybrid_branches_independent_of_the_direct_sum_grid(engine):
         g = engine.linking_numbers(pairs, **kw)
         assert g.stats["graph_launches"] == 1
         _same(g, shared)
+
+
+def test_more_batches_than_a_graph_holds_run_eagerly(engine):
+    """One graph holds 64 Barnes-Hut batches; the results are the same beyond."""
+    curves = W.chainmail(seed=3, grid=26, nmin=40, nmax=80)
+    engine.set_curves(curves)
+    pairs = engine.potential_links()
+    kw = dict(method="barneshut", fallback_tol=0.0)
+    one = engine.linking_numbers(pairs, **kw)
+    many = engine.linking_numbers(pairs, bh_batch_ksegs=1, **kw)
+    few = engine.linking_numbers(pairs[:40], bh_batch_ksegs=1, **kw)
+    assert one.stats["graph_launches"] == few.stats["graph_launches"] == 1
+    assert many.stats["graph_launches"] == 0 and len(pairs) > 600
+    assert many.stats["bh_visits"] == one.stats["bh_visits"]
+    np.testing.assert_allclose(many.lk, one.lk, rtol=0, atol=1e-9)
+    np.testing.assert_allclose(few.lk, one.lk[:40], rtol=0, atol=1e-9)

@@ -2745,8 +2745,8 @@ void bh_batch(flk_ctx *ctx, const int32_t *pairs, const std::vector<int64_t> &id
 // Device bytes the trees and their build records take per segment: two
 // 192-byte node records (384), 288-byte FP64 records for the nodes above 8
 // segments (about one node in eight: ~72), ranges and children (32), sort keys,
-// ids and order (24), the staged segment endpoints (48), scan flags (8) and
-// sort scratch, with headroom.
+// values, ids and order (20), the staged segment endpoints (48) and sort scratch,
+// with headroom.
 constexpr double kBhBytesPerSegment = 648.0;
 
 // Batches of Barnes–Hut pairs whose curves' trees fit the device: the

@@ -323,8 +323,9 @@ __global__ __launch_bounds__(256) void ds_tile_f32(
 // ---------------------------------------------------------------- FP64 tiles
 // The judge: the FP32 kernel's layout and sharing in FP64 (see there for the
 // algebra), bound by the FP64 vector rate, which equals the unpacked FP32
-// one: what counts is instructions per pair, 62 here (106 for a column step of
-// two pairs, 24 for the arctangent of two steps).  Square roots and the
+// one: what counts is instructions per pair, 64 executed (106 for a column step of
+// two pairs and 24 for the arctangent of two steps are 59, the rest the general
+// path and the loops).  Square roots and the
 // reciprocal start from the hardware's estimates and are refined to FP64 in
 // line; the small angles of two columns' pairs are added as one product of
 // x' + i y'.  Any lane of the wave outside the short path's conditions sends
@@ -790,8 +791,8 @@ float ds_eager(flk_ctx *ctx, const DsPlan &P, std::vector<double> *lk_out) {
 }
 
 // Graph run: the batch is captured once per (pairs, curves' sizes, shape,
-// precision) and replayed after that.  The graph is timed whole (its uploads and
-// the reduction add well under a percent to a batch worth a launch).
+// precision) and replayed after that.  The graph is timed whole (the
+// reduction adds well under a percent to a batch worth a launch).
 float ds_graph_run(flk_ctx *ctx, const int32_t *pairs, int64_t npairs, bool fp64, std::vector<double> &lk_out,
                    int64_t *work) {
   const flk_tune &t = ctx->tune;

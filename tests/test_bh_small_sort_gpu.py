@@ -21,7 +21,7 @@ def _spread(v):
                                    [8191, 8192, 100], [8193, 20000, 8192, 65]], ids=str)
 def test_order_is_the_stable_sort_of_the_keys(engine, sizes, exact):
     """Points on a coarse grid, so that many keys are equal; the last set has
-    curves of both sorts in one tree build each."""
+    curves of both sorts, each in a tree build of its own."""
     rng = np.random.default_rng(len(sizes))
     curves = [np.round(rng.normal(size=(n, 3)) * 6) / 8 + (0 if exact else rng.normal(size=(n, 3)) * 1e-13)
               for n in sizes]

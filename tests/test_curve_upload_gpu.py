@@ -1,5 +1,5 @@
 """An upload's boxes and vertices at the edges of their kernels: curves of one and
-of several box chunks (16,384 vertices), empty and short ones among them, and
+of several box chunks (4,096 vertices), empty and short ones among them, and
 the one-block potential-link search at the ends of its range."""
 import numpy as np
 import pytest

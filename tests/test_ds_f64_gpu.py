@@ -1,5 +1,5 @@
 """The FP64 tile kernel at the sizes where its rows (2 per lane, 128 per wave),
-columns (two per iteration, chunks of a multiple of 32) and general path can go
+columns (two per iteration, chunks of a multiple of 64) and general path can go
 wrong, against the FP64 oracle.
 
 Tolerance 1e-12 per pair: a pair of at most 1,100 x 700 segments sums 8e5

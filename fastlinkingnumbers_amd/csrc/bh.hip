@@ -1182,7 +1182,8 @@ constexpr int kWalkSteps = 8;
 constexpr int kSegs = 64;
 constexpr int kLine = 16;  // words of a counter line (128 bytes)
 
-// Counter words of a pass.  Walked: [4] root items, and lines of
+// Counter words of a pass.  Walked: [4] root items, [6] set when the leaf list
+// could not hold every item, and lines of
 // the segments' totals (visits, splits, -, leaf items, leaf segment pairs) and,
 // for each round, of its items, the chunks taken of it and the waves that have
 // ended.  Level by level: [2] leaf segment pairs, [3] network evaluations, [4 +
@@ -1254,14 +1255,24 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
   psum += (blockIdx.x % (unsigned)copies) * copy_stride;
   perr += (blockIdx.x % (unsigned)copies) * copy_stride;
   auto wrap = [](int k) { return k < kStack ? k : k - kStack; };
-  int nleaf = 0;
+  int nleaf = 0, leaf_seg = seg;
+  // A segment's share of the leaf list that is full sends the rest to the next
+  // one's: shares fill unevenly, by a tenth of the list and more.
   auto flush_leaves = [&]() {
-    unsigned long long at = 0;
-    if (lane == 0) at = atomicAdd(totals + 3, (unsigned long long)nleaf);
-    at = __shfl(at, 0, 64);
     wave_lds_sync();
-    for (int i = lane; i < nleaf; i += 64)
-      if ((int64_t)at + i < seg_cap) leaves[seg * seg_cap + (int64_t)at + i] = BhItem{L.lp[i], L.la[i], L.lb[i], 0};
+    for (int from = 0, full = 0; from < nleaf && full < kSegs;) {
+      unsigned long long at = 0;
+      if (lane == 0) at = atomicAdd(seg_totals(cnt, leaf_seg) + 3, (unsigned long long)(nleaf - from));
+      at = __shfl(at, 0, 64);
+      const int fits = (int)max((int64_t)0, min((int64_t)(nleaf - from), seg_cap - (int64_t)at));
+      for (int i = lane; i < fits; i += 64)
+        leaves[leaf_seg * seg_cap + (int64_t)at + i] = BhItem{L.lp[from + i], L.la[from + i], L.lb[from + i], 0};
+      from += fits;
+      if (from < nleaf) {
+        leaf_seg = (leaf_seg + 1) & (kSegs - 1);
+        if (++full == kSegs && lane == 0) atomicOr(cnt + 6, 1ull);
+      }
+    }
     wave_lds_sync();
     nleaf = 0;
   };
@@ -1425,7 +1436,8 @@ __global__ __launch_bounds__(kTravBlock) void bh_leaf_pairs(
       psum += (blockIdx.x % (unsigned)copies) * copy_stride;
       perr += (blockIdx.x % (unsigned)copies) * copy_stride;
     }
-    n = level_count(count, n);
+    // (a walked share may have been asked for more than it holds)
+    n = walked ? min((int64_t)*count, n) : level_count(count, n);
     if (n == 0) return;
     // a short list spread over the blocks in whole multiples of 256
     csz = min<int64_t>(csz, ((n + stride - 1) / stride + kTravBlock - 1) / kTravBlock * kTravBlock);
@@ -1687,8 +1699,9 @@ __global__ __launch_bounds__(1024) void bh_adapt(int64_t nb, const int32_t *__re
 // second pass's for a re-run pair; sums of the second pass are at + nb.
 // Block 0 makes both device-scheduled passes' kPassHead words of their counters
 // (cnt, null for a host-driven batch; levels: how many a level pass has, 0 when
-// walked in `rounds`), with an overflow noted where a queue or a leaf list is over its
-// capacity (its segment's share of it) or items were left after the last level.
+// walked in `rounds`), with an overflow noted where a queue is over its capacity (its
+// segment's share of it), the leaf list is over its own, or items were left after
+// the last level.
 __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__restrict__ redo,
                                                 const double *__restrict__ sum, const double *__restrict__ err,
                                                 int copies, int64_t copy_stride, int mlp, double err_scale,
@@ -1726,8 +1739,8 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
     x[0] = tot[0];
     x[1] = tot[1];
     x[2] = tot[4];
-    x[5] = tot[3];
-    if ((int64_t)tot[3] > cap / kSegs) x[6] = 1;
+    x[5] = min(tot[3], (unsigned long long)(cap / kSegs));
+    if (c[6]) x[6] = 1;
     for (int r = 1; r <= rounds; ++r)
       if ((int64_t)*seg_round(c, r, seg) > cap / kSegs) x[6] = 1;
   }

@@ -108,3 +108,26 @@ def test_one_large_pair_among_many_small(engine, n):
     parts, whole = fastest(pairs[:1]) + fastest(pairs[1:]), fastest(pairs)
     print(n, "parts", parts, "whole", whole)
     assert whole < 5 * parts
+
+
+def test_the_leaf_list_is_used_up(engine):
+    """A leaf list with room for every item holds them, though the segments' shares
+    of it fill unevenly (some 20% over the mean here); one with too little goes to
+    the host.  One pass: beta_limit leaves nothing to re-run."""
+    curves = []
+    for k in range(20):
+        curves += [c + np.array([100.0 * k, 0, 0]) for c in W.random_walk_pair(seed=k, n=8000, rg=6.3, workload=3)]
+    engine.set_curves(curves)
+    pairs = [[2 * k, 2 * k + 1] for k in range(20)]
+    kw = dict(method="barneshut", fallback_tol=0.0, beta_limit=2.0)
+    base = engine.linking_numbers(pairs, **kw)
+    leaves = base.stats["bh_leaf_pairs"]
+    assert base.stats["retries"] == base.stats["bh_host_passes"] == 0 and leaves > 100000
+    for room, passes in ((1.01, 0), (0.95, 1)):
+        engine.set_tune(bh_level_capacity=int(room * leaves))
+        for _ in range(3):
+            got = engine.linking_numbers(pairs, **kw)
+            assert got.stats["bh_host_passes"] == passes, room
+            for key in COUNTS:
+                assert got.stats[key] == base.stats[key], key
+            np.testing.assert_allclose(got.lk, base.lk, rtol=0, atol=1e-9)

@@ -1697,9 +1697,10 @@ __global__ __launch_bounds__(1024) void bh_adapt(int64_t nb, const int32_t *__re
 // Per-pair results of a batch: the first pass's sum and estimate (scaled by
 // err_scale for beta, the root-sum-square for the learned criterion), or the
 // second pass's for a re-run pair; sums of the second pass are at + nb.
-// Block 0 makes both device-scheduled passes' kPassHead words of their counters
-// (cnt, null for a host-driven batch; levels: how many a level pass has, 0 when
-// walked in `rounds`), with an overflow noted where a queue is over its capacity (its
+// With counters (cnt, null for a host-driven batch) one block more, which makes
+// both device-scheduled passes' kPassHead words of them (behind the results of
+// block 0 they took it 1 us longer).  levels: how many a level pass has, 0 when walked
+// in `rounds`.  An overflow is noted where a queue is over its capacity (its
 // segment's share of it), the leaf list is over its own, or items were left after
 // the last level.
 __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__restrict__ redo,
@@ -1717,7 +1718,7 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
     e[t] = mlp ? sqrt(es) : es * err_scale;
     f[t] = r < 0 ? 0u : FLK_PAIR_RETRY;
   }
-  if (cnt == nullptr || blockIdx.x != 0 || threadIdx.x >= 2 * kSegs) return;
+  if (cnt == nullptr || blockIdx.x + 1 != gridDim.x || threadIdx.x >= 2 * kSegs) return;
   const int seg = threadIdx.x & (kSegs - 1), pass = threadIdx.x / kSegs;
   unsigned long long *c = cnt + pass * pass_words(rounds);
   unsigned long long x[kPassHead] = {0, 0, 0, 0, seg == 0 ? c[4] : 0, 0, 0, 0};
@@ -1741,8 +1742,12 @@ __global__ __launch_bounds__(256) void bh_merge(int64_t nb, const int32_t *__res
     x[2] = tot[4];
     x[5] = min(tot[3], (unsigned long long)(cap / kSegs));
     if (c[6]) x[6] = 1;
-    for (int r = 1; r <= rounds; ++r)
-      if ((int64_t)*seg_round(c, r, seg) > cap / kSegs) x[6] = 1;
+    for (int r = 1; r <= rounds; r += 6) {  // six loads in flight
+      unsigned long long most = 0;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) most = max(most, *seg_round(c, min(r + k, rounds), seg));
+      if ((int64_t)most > cap / kSegs) x[6] = 1;
+    }
   }
 #pragma unroll
   for (int i = 0; i < kPassHead; ++i) {
@@ -2580,7 +2585,7 @@ void enqueue_merge(flk_ctx *ctx, BatchPlan &bp, const flk_params &prm, unsigned 
   double *v = bp.res.as<double>(), *e = v + nb;
   auto *heads = reinterpret_cast<unsigned long long *>(e + nb);
   auto *f = reinterpret_cast<uint32_t *>(heads + bp.counts.size());
-  hipLaunchKernelGGL(bh_merge, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, nb,
+  hipLaunchKernelGGL(bh_merge, dim3((unsigned)((nb + 255) / 256) + (cnt ? 1 : 0)), dim3(256), 0, s, nb,
                      (const int32_t *)B.redo.as<int32_t>(), (const double *)B.sum.as<double>(),
                      (const double *)B.err.as<double>(), bp.shape.copies, 2 * nb,
                      prm.criterion == FLK_CRIT_MLP ? 1 : 0, prm.err_scale, v, e, f, heads, cnt, bp.shape.cap,

@@ -382,9 +382,9 @@ __device__ __forceinline__ double atan_short_f64(double zi, double zr) {
 // curves' first vertices, with their boxes' diagonals.
 __device__ __forceinline__ double short_path_limit(const double4 &p0, const double4 &q0) {
   const double x = q0.x - p0.x, y = q0.y - p0.y, z = q0.z - p0.z;
-  const double longest = sqrt(x * x + y * y + z * z) + p0.w + q0.w;
-  const double r2 = fmin(longest * longest, 1.0);
-  const double limit = longest < 1e11 ? fmax(1e-28 * r2 * r2 * r2, 1e-70) : __builtin_inf();
+  // at least the square of the sum of the three lengths
+  const double most = 3.0 * (x * x + y * y + z * z + p0.w * p0.w + q0.w * q0.w), r2 = fmin(most, 1.0);
+  const double limit = most < 1e22 ? fmax(1e-28 * r2 * r2 * r2, 1e-70) : __builtin_inf();
   return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(limit)),
                           __builtin_amdgcn_readfirstlane(__double2loint(limit)));  // the wave's, in scalar registers
 }
